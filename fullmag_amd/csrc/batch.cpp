@@ -338,7 +338,7 @@ int fullmag_fdm_ext_autotune(fullmag_fdm_backend *handle, int reps, char *chosen
                                {"x_rows", &T::x_rows, {0, 8, 4, 2}, true},
                                {"y_radix", &T::y_radix, {16, 8, 4}, true},
                                {"y_lpw", &T::y_lpw, {0, 1, 2}, true},
-                               {"fixed", &T::fixed, {1, 0}, false},
+                               {"fixed", &T::fixed, {1, 0}, true},
                                {"y_pipe", &T::y_pipe, {1, 0, 2, 4, 8}, false},
                                {"y_pipe_f", &T::y_pipe_f, {1, 2, 4, 8}, false},
                                {"z_quad", &T::z_quad, {0, 1}, false},

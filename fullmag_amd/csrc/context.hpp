@@ -29,13 +29,13 @@ enum Mode { MODE_SINGLE = 1, MODE_DOUBLE = 2, MODE_MIXED = 3 };
 // Launch-schedule knobs of the demag transforms (0 = automatic).  Settable
 // per backend from the FULLMAG_FDM_TUNE environment variable as a comma list
 // of key=value (x_radix, x_lanes, x_rows, y_radix, y_lanes, y_lpw, fixed,
-// z_quad, xcd, y_pipe, y_pipe_f, z_tile, zc, y_split).  x_radix, x_lanes,
-// x_rows, y_radix, y_lanes, y_lpw, z_tile and y_split shape the plan made at
-// set-up; the others are read at every launch.
+// z_quad, xcd, y_pipe, y_pipe_f, z_tile, zc, y_split, pad).  x_radix, x_lanes,
+// x_rows, y_radix, y_lanes, y_lpw, fixed, z_tile, y_split and pad shape the
+// plan made at set-up; the others are read at every launch.
 struct DemagTuning {
     int x_radix = 16, x_lanes = 0, x_rows = 0;
     int y_radix = 16, y_lanes = 0, y_lpw = 0;
-    int fixed = 1;   // 0: runtime-planned line kernels even for fixed schedules
+    int fixed = 1;   // 0: runtime-planned line kernels even for scheduled lengths
     int z_quad = -1;  // 1: four lanes per z column instead of two (even nz); -1: FP64 only
     int xcd = 1;     // 0: no per-XCD renumbering of workgroups
     int y_pipe = 1;    // line groups per workgroup of the y line kernel; > 1 prefetches the next (0: off)
@@ -43,6 +43,7 @@ struct DemagTuning {
     int z_tile = 0;    // > 0: at most this many columns per long-z (LDS line) workgroup
     int zc = 0;        // z planes per workgroup of the cell kernels (0: automatic)
     int y_split = 0;   // 1: thin-film y convolution as separate line and tensor passes
+    int pad = 1;       // 0: transform lengths 2n even where a longer scheduled length is faster
 };
 
 // Applies "key=value,..." (unknown keys ignored) on top of t.
@@ -55,12 +56,12 @@ struct DemagPlan {
     bool projection = false;  // no tensor: k-space projection fallback
     int nx = 0, ny = 0, nz = 0;
     int px = 0, py = 0, pz = 1;
-    int hx = 0;    // nx + 1 columns of the half spectrum
+    int hx = 0;    // px / 2 + 1 columns of the half spectrum
     size_t lds_limit = 65536;  // LDS bytes one workgroup may allocate on this device
     bool y_split = false;      // thin film: y lines, tensor and inverse y lines as three passes
     int rows = 0;  // rows per plane of `spec`
     int kcomp = 0; // 6 (3-D) or 4 (2-D: xz = yz = 0 on the film plane)
-    int kz_n = 1;  // octant planes in kz: nz + 1 (3-D) or 1
+    int kz_n = 1;  // octant planes in kz: pz / 2 + 1 (3-D) or 1
     double inv_npad = 0.0;
     LinePlan lx, ly, lz;
     // launch geometry

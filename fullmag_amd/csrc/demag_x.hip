@@ -1,0 +1,415 @@
+// demag_x.hip -- x passes of the demag convolution: real-to-complex of two
+// packed rows per line and back (see demag.hip for the pipeline).  Compiled
+// once per field precision (FM_REAL).
+#include "demag.hpp"
+
+namespace fm {
+namespace {
+
+// Forward real-to-complex along x for xr rows (y0 .. y0+xr-1) of plane
+// (c = blockIdx.z, z = blockIdx.y).  Rows 2j, 2j+1 are packed as a + i b;
+// with Z = FFT(a + i b):  A_k = (Z_k + conj Z_{N-k}) / 2,
+// B_k = (Z_k - conj Z_{N-k}) / (2i), k = 0..N/2, stored at spec[c][z][k][y].
+template <typename Real, class Src, int N>
+__device__ __forceinline__ void xfwd_body(const XArgs<Real> &a, const Src &src, cplx<Real> *spec, int c) {
+    using L = LineOps<N>;
+    extern __shared__ unsigned char smem_raw[];
+    cplx<Real> *lds = reinterpret_cast<cplx<Real> *>(smem_raw);
+    const int LINES = a.xr >> 1;
+    const int n = L::n(a.lp), ls = a.ls, T = L::threads(a.lp);
+    const int tid = threadIdx.x, nthr = blockDim.x;
+    const int y0 = blockIdx.x * a.xr, z = blockIdx.y;
+    // the T lanes of packed line j (= tid / T, blockDim.x = LINES * T) load it
+    const int jl = tid / T, t = tid - jl * T;
+    cplx<Real> *line = lds + jl * ls;
+    const int lx = L::line_xor(jl);
+    {
+        const int ya = y0 + 2 * jl;
+        if constexpr (N > 0) {
+            // scheduled length: all loads of a lane in flight before the first pass
+            constexpr int E = fx_elems(N), NT = fx_lanes(N);
+            cplx<Real> v[E];
+            if (!Src::kGather && src.uniform() && 2 * a.n_in <= N) {
+                // branch-free: clamped addresses, every load issued before
+                // any is used; elements t + e NT with e >= E / 2 lie in
+                // the zero padding (n_in <= N/2) and are not loaded
+                const bool oka = ya < a.rows, okb = ya + 1 < a.rows;
+                const int yA = oka ? ya : 0, yB = okb ? ya + 1 : 0;
+#pragma unroll
+                for (int e = 0; e < E / 2; ++e) {
+                    const int x = t + e * NT;
+                    const bool okx = x < a.n_in;
+                    const int xs = okx ? x : 0;
+                    const Real va = src.uniform_at(c, z, yA, xs), vb = src.uniform_at(c, z, yB, xs);
+                    v[e] = {(okx && oka) ? va : Real(0), (okx && okb) ? vb : Real(0)};
+                }
+#pragma unroll
+                for (int e = E / 2; e < E; ++e) v[e] = {Real(0), Real(0)};
+            } else if (Src::kGather && 2 * a.n_in <= N) {
+                // the same with the mask, volume fraction and per-cell Ms
+                // read beside each element, all unconditionally
+                const bool oka = ya < a.rows, okb = ya + 1 < a.rows;
+                const int yA = oka ? ya : 0, yB = okb ? ya + 1 : 0;
+#pragma unroll
+                for (int e = 0; e < E / 2; ++e) {
+                    const int x = t + e * NT;
+                    const bool okx = x < a.n_in;
+                    const int xs = okx ? x : 0;
+                    const Real va = src.gather_at(c, z, yA, xs), vb = src.gather_at(c, z, yB, xs);
+                    v[e] = {(okx && oka) ? va : Real(0), (okx && okb) ? vb : Real(0)};
+                }
+#pragma unroll
+                for (int e = E / 2; e < E; ++e) v[e] = {Real(0), Real(0)};
+            } else {
+#pragma unroll
+                for (int e = 0; e < E; ++e) {
+                    const int x = t + e * NT;
+                    v[e] = {Real(0), Real(0)};
+                    if (x < a.n_in) {
+                        if (ya < a.rows) v[e].x = src(c, z, ya, x);
+                        if (ya + 1 < a.rows) v[e].y = src(c, z, ya + 1, x);
+                    }
+                }
+            }
+            // the loaded elements are the first pass's inputs
+            fx_first_pass<Real, N>(line, t, v, a.tw, false, lx);
+            fx_rest<Real, N>(line, t, a.tw, false, lx);
+        } else {
+            for (int x = t; x < n; x += T) {
+                cplx<Real> v = {Real(0), Real(0)};
+                if (x < a.n_in) {
+                    if (ya < a.rows) v.x = src(c, z, ya, x);
+                    if (ya + 1 < a.rows) v.y = src(c, z, ya + 1, x);
+                }
+                line[L::slot(a.lp, x, lx)] = v;
+            }
+            __syncthreads();
+            L::template fft<Real>(line, a.lp, t, a.tw, false, lx);
+        }
+    }
+    __syncthreads();  // the unpack reads every line
+    const int hx = a.g.hx;
+    // lane (j, k) splits line j into rows 2j (A) and 2j + 1 (B) at kx = k;
+    // the two are adjacent in memory (one 16-byte store in FP32 when the
+    // row pitch is even)
+    if constexpr (sizeof(Real) == 8) {
+        // FP64: one 16-byte complex per lane, consecutive lanes on consecutive rows
+        for (int idx = tid; idx < hx * a.xr; idx += nthr) {
+            const int yl = idx & (a.xr - 1), k = idx >> a.xr_log2;
+            const int y = y0 + yl;
+            if (y >= a.rows) continue;
+            const int j = yl >> 1, jx = L::line_xor(j);
+            const cplx<Real> zk = lds[j * ls + L::slot(a.lp, k, jx)];
+            const cplx<Real> zn = lds[j * ls + L::slot(a.lp, k == 0 ? 0 : n - k, jx)];
+            const Real h = Real(0.5);
+            cplx<Real> v;
+            if ((yl & 1) == 0) v = {h * (zk.x + zn.x), h * (zk.y - zn.y)};
+            else v = {h * (zk.y + zn.y), h * (zn.x - zk.x)};
+            spec[a.g.at(c, z, k, y)] = v;
+        }
+        return;
+    }
+    const bool pair16 = (a.g.pitch & 1) == 0;
+    for (int idx = tid; idx < hx * LINES; idx += nthr) {
+        const int j = idx & (LINES - 1), k = idx >> (a.xr_log2 - 1);
+        const int y = y0 + 2 * j;
+        if (y >= a.rows) continue;
+        const int jx = L::line_xor(j);
+        const cplx<Real> zk = lds[j * ls + L::slot(a.lp, k, jx)];
+        const cplx<Real> zn = lds[j * ls + L::slot(a.lp, k == 0 ? 0 : n - k, jx)];
+        const Real h = Real(0.5);
+        const cplx<Real> A = {h * (zk.x + zn.x), h * (zk.y - zn.y)};
+        const cplx<Real> B = {h * (zk.y + zn.y), h * (zn.x - zk.x)};
+        cplx<Real> *dst = spec + a.g.at(c, z, k, y);
+        if (y + 1 < a.rows) {
+            if (pair16) {
+                *reinterpret_cast<float4 *>(dst) = float4{float(A.x), float(A.y), float(B.x), float(B.y)};
+            } else {
+                dst[0] = A;
+                dst[1] = B;
+            }
+        } else {
+            dst[0] = A;
+        }
+    }
+}
+
+// Component c = blockIdx.z.
+template <typename Real, class Src, int N = 0>
+__global__ void __launch_bounds__(kMaxBlock) xfwd_kernel(XArgs<Real> a, Src src, cplx<Real> *spec) {
+    xfwd_body<Real, Src, N>(a, src, spec, (int)blockIdx.z);
+}
+
+// Multi-instance form: instance blockIdx.z / zdiv of the table, component
+// blockIdx.z % zdiv.  Each multi-instance kernel copies its instance's
+// arguments into a local before the body runs, so the body sees invariant
+// values exactly as the plain kernel does (a reference into the table would be
+// re-read after the body's stores, which changes how the compiler contracts
+// the arithmetic, and with it the last bit of FP32 results).
+template <typename Real, class Src>
+struct XFwdPack {
+    XArgs<Real> a;
+    Src src;
+    cplx<Real> *spec;
+};
+template <typename Real, class Src, int N = 0>
+__global__ void __launch_bounds__(kMaxBlock) xfwd_multi(const XFwdPack<Real, Src> *tab, int zdiv) {
+    const XFwdPack<Real, Src> p = tab[blockIdx.z / zdiv];
+    xfwd_body<Real, Src, N>(p.a, p.src, p.spec, (int)(blockIdx.z % zdiv));
+}
+
+// Inverse complex-to-real along x: Z_k = A_k + i B_k for k <= N/2 and the
+// Hermitian continuation A_{N-k} = conj A_k; z = IFFT(Z); rows a = Re z,
+// b = Im z.  Reads spec[c][z][k][y0..y0+xr-1].
+template <typename Real, class Sink, int N>
+__device__ __forceinline__ void xinv_body(const XArgs<Real> &a, const cplx<Real> *spec, const Sink &sink, int c) {
+    using L = LineOps<N>;
+    extern __shared__ unsigned char smem_raw[];
+    cplx<Real> *lds = reinterpret_cast<cplx<Real> *>(smem_raw);
+    const int LINES = a.xr >> 1;
+    const int n = L::n(a.lp), ls = a.ls, T = L::threads(a.lp);
+    const int tid = threadIdx.x, nthr = blockDim.x;
+    const int y0 = blockIdx.x * a.xr, z = blockIdx.y;
+    const int hx = a.g.hx;
+    // consecutive lanes read consecutive rows of one kx column
+    auto put = [&](int idx, cplx<Real> A, cplx<Real> B) {
+        const int j = idx & (LINES - 1), k = idx >> (a.xr_log2 - 1);
+        const int jx = L::line_xor(j);
+        lds[j * ls + L::slot(a.lp, k, jx)] = {A.x - B.y, A.y + B.x};
+        if (k > 0 && k < n - k) lds[j * ls + L::slot(a.lp, n - k, jx)] = {A.x + B.y, B.x - A.y};
+    };
+    if constexpr (N > 0) {
+        // fixed length: every load of the lane (hx / T <= U row pairs) in
+        // flight before the LDS writes; a row pair is one 16-byte load in
+        // FP32 when the row pitch is even
+        constexpr int U = (N / 2 + 1 + fx_lanes(N) - 1) / fx_lanes(N);
+        const bool pair16 = sizeof(Real) == 4 && (a.g.pitch & 1) == 0;
+        cplx<Real> A[U], B[U];
+        // branch-free: clamped addresses, selects after the loads
+        if (pair16) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int idx = tid + u * nthr;
+                const int j = idx & (LINES - 1), k = idx >> (a.xr_log2 - 1);
+                const int ya = y0 + 2 * j;
+                const bool oka = k < hx && ya < a.rows, okb = oka && ya + 1 < a.rows;
+                // an even row pitch and an even ya keep the pair 16-byte aligned
+                const float4 q = *reinterpret_cast<const float4 *>(spec + (oka ? a.g.at(c, z, k, ya) : 0));
+                A[u] = oka ? cplx<Real>{Real(q.x), Real(q.y)} : cplx<Real>{Real(0), Real(0)};
+                B[u] = okb ? cplx<Real>{Real(q.z), Real(q.w)} : cplx<Real>{Real(0), Real(0)};
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int idx = tid + u * nthr;
+                const int j = idx & (LINES - 1), k = idx >> (a.xr_log2 - 1);
+                const int ya = y0 + 2 * j;
+                const bool oka = k < hx && ya < a.rows, okb = oka && ya + 1 < a.rows;
+                const cplx<Real> qa = spec[oka ? a.g.at(c, z, k, ya) : 0];
+                const cplx<Real> qb = spec[okb ? a.g.at(c, z, k, ya + 1) : 0];
+                A[u] = oka ? qa : cplx<Real>{Real(0), Real(0)};
+                B[u] = okb ? qb : cplx<Real>{Real(0), Real(0)};
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int idx = tid + u * nthr;
+            if (idx < hx * LINES) put(idx, A[u], B[u]);
+        }
+    } else {
+        // batches of four loads per lane in flight before their LDS writes
+        constexpr int U = 4;
+        for (int base = tid; base < hx * LINES; base += U * nthr) {
+            cplx<Real> A[U], B[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int idx = base + u * nthr;
+                const int j = idx & (LINES - 1), k = idx >> (a.xr_log2 - 1);
+                const int ya = y0 + 2 * j;
+                A[u] = B[u] = {Real(0), Real(0)};
+                if (idx < hx * LINES) {
+                    if (ya < a.rows) A[u] = spec[a.g.at(c, z, k, ya)];
+                    if (ya + 1 < a.rows) B[u] = spec[a.g.at(c, z, k, ya + 1)];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int idx = base + u * nthr;
+                if (idx >= hx * LINES) break;
+                put(idx, A[u], B[u]);
+            }
+        }
+    }
+    __syncthreads();
+    const int jl = tid / T, t = tid - jl * T;
+    const cplx<Real> *line = lds + jl * ls;
+    const int lx = L::line_xor(jl);
+    L::template fft<Real>(lds + jl * ls, a.lp, t, a.tw, true, lx);
+    // the lanes of line jl store its rows 2 jl (real part) and 2 jl + 1
+    const int ya = y0 + 2 * jl;
+    if constexpr (N > 0 && std::is_same<Sink, FieldSink<float>>::value) {
+        if (2 * a.n_out <= N && sink.masked() && (a.n_out & 3) == 0 && (sink.n & 3) == 0) {
+            // four consecutive outputs of a row per lane: their mask bytes in
+            // one 4-byte load, every mask word read before the first store,
+            // and the values in one 16-byte store (rows start on 16-byte
+            // boundaries: nx = n_out and n are multiples of four)
+            constexpr int TT = fx_lanes(N), Q = (N / 2 + 4 * TT - 1) / (4 * TT);
+            const bool oka = ya < a.rows, okb = ya + 1 < a.rows;
+            const int yA = oka ? ya : 0, yB = okb ? ya + 1 : 0;
+            uint32_t ka[Q], kb[Q];
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                const int x = 4 * (t + q * TT);
+                const int xs = x < a.n_out ? x : 0;
+                ka[q] = *reinterpret_cast<const uint32_t *>(sink.mask + ((int64_t)z * sink.ny + yA) * sink.nx + xs);
+                kb[q] = *reinterpret_cast<const uint32_t *>(sink.mask + ((int64_t)z * sink.ny + yB) * sink.nx + xs);
+            }
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                const int x = 4 * (t + q * TT);
+                if (x < a.n_out) {
+                    cplx<Real> v[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] = line[L::slot(a.lp, x + e, lx)];
+                    auto row = [&](uint32_t k, int part) {
+                        float o[4];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            o[e] = ((k >> (8 * e)) & 0xffu) ? (part ? v[e].y : v[e].x) * a.scale : 0.0f;
+                        return float4{o[0], o[1], o[2], o[3]};
+                    };
+                    const int64_t i = ((int64_t)z * sink.ny + ya) * sink.nx + x;
+                    if (oka) *reinterpret_cast<float4 *>(sink.out + (int64_t)c * sink.n + i) = row(ka[q], 0);
+                    if (okb)
+                        *reinterpret_cast<float4 *>(sink.out + (int64_t)c * sink.n + i + sink.nx) = row(kb[q], 1);
+                }
+            }
+            return;
+        }
+    }
+    if constexpr (N > 0) {
+        if (2 * a.n_out <= N && sink.masked()) {
+            // at most E / 2 outputs per row and lane: every mask byte read
+            // (clamped addresses) before the first store
+            constexpr int H = fx_elems(N) / 2;
+            const bool oka = ya < a.rows, okb = ya + 1 < a.rows;
+            const int yA = oka ? ya : 0, yB = okb ? ya + 1 : 0;
+            uint8_t ka[H], kb[H];
+#pragma unroll
+            for (int e = 0; e < H; ++e) {
+                const int x = t + e * T;
+                const int xs = x < a.n_out ? x : 0;
+                ka[e] = sink.keep(z, yA, xs);
+                kb[e] = sink.keep(z, yB, xs);
+            }
+#pragma unroll
+            for (int e = 0; e < H; ++e) {
+                const int x = t + e * T;
+                if (x < a.n_out) {
+                    const cplx<Real> v = line[L::slot(a.lp, x, lx)];
+                    if (oka) sink.put(c, z, ya, x, v.x * a.scale, ka[e]);
+                    if (okb) sink.put(c, z, ya + 1, x, v.y * a.scale, kb[e]);
+                }
+            }
+            return;
+        }
+    }
+    if constexpr (std::is_same<Sink, FieldSink<float>>::value) {
+        if (!sink.masked() && (a.n_out & 3) == 0 && (sink.n & 3) == 0) {
+            // four consecutive outputs of a row per lane and one 16-byte
+            // store (rows start on 16-byte boundaries: nx = n_out and n are
+            // multiples of four)
+            for (int x = 4 * t; x < a.n_out; x += 4 * T) {
+                cplx<Real> v[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = line[L::slot(a.lp, x + e, lx)];
+                const int64_t i = ((int64_t)z * sink.ny + ya) * sink.nx + x;
+                if (ya < a.rows)
+                    *reinterpret_cast<float4 *>(sink.out + (int64_t)c * sink.n + i) =
+                        float4{v[0].x * a.scale, v[1].x * a.scale, v[2].x * a.scale, v[3].x * a.scale};
+                if (ya + 1 < a.rows)
+                    *reinterpret_cast<float4 *>(sink.out + (int64_t)c * sink.n + i + sink.nx) =
+                        float4{v[0].y * a.scale, v[1].y * a.scale, v[2].y * a.scale, v[3].y * a.scale};
+            }
+            return;
+        }
+    }
+    for (int x = t; x < a.n_out; x += T) {
+        const cplx<Real> v = line[L::slot(a.lp, x, lx)];
+        if (ya < a.rows) sink(c, z, ya, x, v.x * a.scale);
+        if (ya + 1 < a.rows) sink(c, z, ya + 1, x, v.y * a.scale);
+    }
+}
+
+template <typename Real, class Sink, int N = 0>
+__global__ void __launch_bounds__(kMaxBlock) xinv_kernel(XArgs<Real> a, const cplx<Real> *spec, Sink sink) {
+    xinv_body<Real, Sink, N>(a, spec, sink, (int)blockIdx.z);
+}
+
+template <typename Real, class Sink>
+struct XInvPack {
+    XArgs<Real> a;
+    const cplx<Real> *spec;
+    Sink sink;
+};
+template <typename Real, class Sink, int N = 0>
+__global__ void __launch_bounds__(kMaxBlock) xinv_multi(const XInvPack<Real, Sink> *tab, int zdiv) {
+    const XInvPack<Real, Sink> p = tab[blockIdx.z / zdiv];
+    xinv_body<Real, Sink, N>(p.a, p.spec, p.sink, (int)(blockIdx.z % zdiv));
+}
+
+}  // namespace
+
+template <typename Real, class Src>
+void launch_xfwd(Context &c, const XArgs<Real> &xa, const Src &src, cplx<Real> *spec, unsigned row_groups,
+                 unsigned planes, unsigned comps, size_t lds) {
+    const dim3 grid(row_groups, planes, comps), block((unsigned)((xa.xr / 2) * xa.lp.threads));
+    if constexpr (std::is_same<Src, NewellSource>::value) {
+        hipLaunchKernelGGL((xfwd_kernel<Real, Src, 0>), grid, block, lds, c.stream, xa, src, spec);
+    } else {
+        with_line(xa.lp, [&](auto NC) {
+            constexpr int N = decltype(NC)::value;
+            const XFwdPack<Real, Src> pk{xa, src, spec};
+            launch_rec(c, N > 0 ? reinterpret_cast<const void *>(&xfwd_multi<Real, Src, N>) : nullptr, grid, block,
+                       lds, (int)comps, pk, [&] {
+                           hipLaunchKernelGGL((xfwd_kernel<Real, Src, N>), grid, block, lds, c.stream, xa, src, spec);
+                       });
+        });
+    }
+}
+
+template <typename Real>
+void launch_xinv(Context &c, const XArgs<Real> &xa, const cplx<Real> *spec, const FieldSink<Real> &sink,
+                 unsigned row_groups, unsigned planes, size_t lds) {
+    const dim3 grid(row_groups, planes, 3), block((unsigned)((xa.xr / 2) * xa.lp.threads));
+    with_line(xa.lp, [&](auto NC) {
+        constexpr int N = decltype(NC)::value;
+        const XInvPack<Real, FieldSink<Real>> pk{xa, spec, sink};
+        launch_rec(c, N > 0 ? reinterpret_cast<const void *>(&xinv_multi<Real, FieldSink<Real>, N>) : nullptr, grid,
+                   block, lds, 3, pk, [&] {
+                       hipLaunchKernelGGL((xinv_kernel<Real, FieldSink<Real>, N>), grid, block, lds, c.stream, xa,
+                                          spec, sink);
+                   });
+    });
+}
+
+using R = FM_REAL;
+#define FM_XFWD(SRC) \
+    template void launch_xfwd<R, SRC>(Context &, const XArgs<R> &, const SRC &, cplx<R> *, unsigned, unsigned, \
+                                      unsigned, size_t);
+using SrcState = MagSource<R, double>;
+using SrcStateG = MagSource<R, double, true>;
+FM_XFWD(SrcState)
+FM_XFWD(SrcStateG)
+#ifdef FM_REAL_IS_FLOAT
+using SrcStage = MagSource<R, float>;
+using SrcStageG = MagSource<R, float, true>;
+FM_XFWD(SrcStage)
+FM_XFWD(SrcStageG)
+#else
+FM_XFWD(NewellSource)
+#endif
+template void launch_xinv<R>(Context &, const XArgs<R> &, const cplx<R> *, const FieldSink<R> &, unsigned, unsigned,
+                             size_t);
+
+}  // namespace fm

@@ -28,6 +28,7 @@ struct LinePlan {
     int npass = 0;    // number of Stockham passes
     int threads = 0;  // lanes per line (each holds up to 16 complex values)
     int swz = 0;      // 1: LDS slots XOR-swizzled within 16-element blocks
+    int fixed = 0;    // 1: the compile-time schedule of length n (fx_has) runs this line
     int radix[kMaxPass] = {};
 };
 
@@ -41,9 +42,16 @@ __host__ __device__ __forceinline__ int lslot(const LinePlan &lp, int i) { retur
 // factor of n as a direct-sum pass, and the lanes per line: the fewest lanes
 // such that no lane holds more than 16 complex values in any pass, or
 // `min_lanes` if larger (capped at the largest pass's butterfly count);
-// power-of-two radices are capped at max_radix (16, 8 or 4).  Returns false
-// (with `err`) for lengths needing more than kMaxPass passes or 1024 lanes.
-bool plan_line(int n, LinePlan &lp, std::string &err, int min_lanes = 1, int max_radix = 16);
+// power-of-two radices are capped at max_radix (16, 8 or 4).  With `fixed`, a
+// length that has a compile-time schedule gets that schedule's lanes and
+// radices (default knobs only).  Returns false (with `err`) for lengths
+// needing more than kMaxPass passes or 1024 lanes.
+bool plan_line(int n, LinePlan &lp, std::string &err, int min_lanes = 1, int max_radix = 16, bool fixed = false);
+
+// Padded length of a linear convolution of n cells: any length >= 2n - 1
+// gives the same field, so 2n where that has a compile-time schedule, else
+// the next length that has one if it is at most 4/3 of 2n, else 2n.
+int pick_padded(int n);
 
 // w[t] = exp(-2 pi i t / n), t in [0, n), correctly rounded from long double.
 std::vector<cplx<double>> twiddle_table(int n);
@@ -150,6 +158,81 @@ __device__ __forceinline__ void dft_prime(cplx<T> *v, const cplx<T> *tw, int n, 
     for (int q = 0; q < R; ++q) v[q] = out[q];
 }
 
+// Odd prime R = 3, 5, 7 with literal roots: the pair sums s_r = v_r + v_(R-r)
+// carry the cosines and the differences d_r the sines.
+template <typename T, int R>
+__device__ __forceinline__ void dft_odd(cplx<T> *v, bool inv) {
+    static_assert(R == 3 || R == 5 || R == 7, "literal roots");
+    constexpr int H = (R - 1) / 2;
+    constexpr double C3[1] = {-0.5}, S3[1] = {0.86602540378443864676};
+    constexpr double C5[2] = {0.30901699437494742410, -0.80901699437494742410},
+                     S5[2] = {0.95105651629515357212, 0.58778525229247312917};
+    constexpr double C7[3] = {0.62348980185873353053, -0.22252093395631440429, -0.90096886790241912624},
+                     S7[3] = {0.78183148246802980871, 0.97492791218182360702, 0.43388373911755812048};
+    cplx<T> s[H], d[H];
+#pragma unroll
+    for (int r = 1; r <= H; ++r) {
+        s[r - 1] = cadd(v[r], v[R - r]);
+        d[r - 1] = csub(v[r], v[R - r]);
+    }
+    cplx<T> o0 = v[0], out[R];
+#pragma unroll
+    for (int r = 0; r < H; ++r) o0 = cadd(o0, s[r]);
+#pragma unroll
+    for (int q = 1; q <= H; ++q) {
+        cplx<T> a = v[0], b{T(0), T(0)};
+#pragma unroll
+        for (int r = 1; r <= H; ++r) {
+            const int m = (q * r) % R, i = (m <= H ? m : R - m) - 1;
+            const T c = T(R == 3 ? C3[i % 1] : R == 5 ? C5[i % 2] : C7[i]);
+            const T w0 = T(R == 3 ? S3[i % 1] : R == 5 ? S5[i % 2] : S7[i]);
+            const T w = m <= H ? w0 : -w0;
+            a.x += c * s[r - 1].x;
+            a.y += c * s[r - 1].y;
+            b.x += w * d[r - 1].x;
+            b.y += w * d[r - 1].y;
+        }
+        // forward: a - i b at q, a + i b at R - q; the inverse swaps them
+        const cplx<T> lo{a.x + b.y, a.y - b.x}, hi{a.x - b.y, a.y + b.x};
+        out[q] = inv ? hi : lo;
+        out[R - q] = inv ? lo : hi;
+    }
+    v[0] = o0;
+#pragma unroll
+    for (int q = 1; q < R; ++q) v[q] = out[q];
+}
+
+template <typename T, int R>
+__device__ __forceinline__ void dft_any(cplx<T> *v, const cplx<T> *tw, int n, bool inv);
+
+constexpr int inv_mod(int a, int m, int x = 1) { return (a * x) % m == 1 % m ? x : inv_mod(a, m, x + 1); }
+
+// R = A B with coprime A and B (Good and Thomas): inputs (B i + A j) mod R,
+// A-point DFTs over i, B-point DFTs over j, no twiddles; outputs at the index
+// that is p mod A and q mod B.
+template <typename T, int A, int B>
+__device__ __forceinline__ void dft_coprime(cplx<T> *v, const cplx<T> *tw, int n, bool inv) {
+    constexpr int R = A * B;
+    // 1 mod A and 0 mod B; 0 mod A and 1 mod B
+    constexpr int EA = B * inv_mod(B, A), EB = A * inv_mod(A, B);
+    cplx<T> u[B][A];
+#pragma unroll
+    for (int j = 0; j < B; ++j) {
+#pragma unroll
+        for (int i = 0; i < A; ++i) u[j][i] = v[(B * i + A * j) % R];
+        dft_any<T, A>(u[j], tw, n, inv);
+    }
+#pragma unroll
+    for (int p = 0; p < A; ++p) {
+        cplx<T> w[B];
+#pragma unroll
+        for (int j = 0; j < B; ++j) w[j] = u[j][p];
+        dft_any<T, B>(w, tw, n, inv);
+#pragma unroll
+        for (int q = 0; q < B; ++q) v[(p * EA + q * EB) % R] = w[q];
+    }
+}
+
 template <typename T, int R>
 __device__ __forceinline__ void dft_any(cplx<T> *v, const cplx<T> *tw, int n, bool inv) {
     if constexpr (R == 2) {
@@ -160,6 +243,14 @@ __device__ __forceinline__ void dft_any(cplx<T> *v, const cplx<T> *tw, int n, bo
         dft8(v, inv);
     } else if constexpr (R == 16) {
         dft16(v, inv);
+    } else if constexpr (R == 12) {
+        dft_coprime<T, 4, 3>(v, tw, n, inv);
+    } else if constexpr (R == 10) {
+        dft_coprime<T, 2, 5>(v, tw, n, inv);
+    } else if constexpr (R == 14) {
+        dft_coprime<T, 2, 7>(v, tw, n, inv);
+    } else if constexpr (R == 3 || R == 5 || R == 7) {
+        dft_odd<T, R>(v, inv);
     } else {
         dft_prime<T, R>(v, tw, n, inv);
     }
@@ -304,14 +395,37 @@ __device__ __forceinline__ void line_fft(cplx<T> *line, const LinePlan &lp, int 
 }
 
 // ---------------------------------------------------------------------------
-// Compile-time schedules for power-of-two lines, 16 <= n <= 4096
+// Compile-time schedules: 2^a (32..4096) and 5, 3 and 7 times a power of two
+// (10, 12 or 14 times 2 .. 64)
 // ---------------------------------------------------------------------------
-// The same radices plan_line() picks for these lengths with default knobs
-// (radix-16 passes, then an 8/4 tail; 2^(4a+1) uses 16^(a-1) 8 4), so a line
-// transformed by either path carries the same roundings.  With n, the radix
-// and the span known at compile time every index is a shift or mask, the
-// swizzle is fixed and each kernel only holds one pass's registers.
+// With n, the radices and the spans known at compile time every index is a
+// shift, mask or constant product, the swizzle is fixed and each kernel holds
+// one pass's registers.  Powers of two use 16 elements per lane and the
+// radices plan_line() picks with default knobs (radix-16 passes, then an 8/4
+// tail; 2^(4a+1) uses 16^(a-1) 8 4), so a line transformed by either path
+// carries the same roundings.  The other lengths give a lane E = 12, 10 or 14
+// elements, the inputs of one first-pass butterfly of that radix, and keep a
+// power-of-two number of lanes per line, so that lines never straddle a
+// wavefront; the remaining power of two is one or two passes of radix 16, 8,
+// 4 or 2 in which some lanes may have no butterfly.
 constexpr int clog2(int n) { return n <= 1 ? 0 : 1 + clog2(n / 2); }
+constexpr int fx_odd(int n) { return n % 2 == 0 ? fx_odd(n / 2) : n; }
+
+// Elements per lane.
+constexpr int fx_elems(int n) {
+    const int o = fx_odd(n);
+    return o == 1 ? 16 : o == 3 ? 12 : o == 5 ? 10 : 14;
+}
+constexpr int fx_lanes(int n) { return n / fx_elems(n); }
+
+constexpr bool fx_has(int n) {
+    if (n < 20 || n % 2 != 0) return false;
+    const int o = fx_odd(n);
+    if (o == 1) return n >= 32 && n <= 4096;
+    if (o != 3 && o != 5 && o != 7) return false;
+    const int e = fx_elems(n), t = n / e;
+    return t * e == n && t >= 2 && t <= 64;
+}
 
 constexpr int p2_npass(int n) {
     return (clog2(n) % 4 == 0) ? clog2(n) / 4 : (clog2(n) % 4 == 1 && clog2(n) < 4) ? 1 : clog2(n) / 4 + 1;
@@ -325,25 +439,36 @@ constexpr int p2_radix(int n, int p) {
     return p < a ? 16 : 8;
 }
 
-// Host check: `lp` is the default plan of a length with a fixed schedule.
-inline bool p2_matches(const LinePlan &lp, int n) {
-    if (lp.n != n || lp.threads != n / 16 || lp.npass != p2_npass(n) || !lp.swz) return false;
-    for (int p = 0; p < lp.npass; ++p)
-        if (lp.radix[p] != p2_radix(n, p)) return false;
-    return true;
+// Passes and radices of a scheduled length: for the lengths with an odd
+// factor, fx_elems() and then 2, 4, 8, 16, 8 4 or 16 4.
+constexpr int fx_npass(int n) {
+    if (fx_odd(n) == 1) return p2_npass(n);
+    return fx_lanes(n) <= 16 ? 2 : 3;
+}
+constexpr int fx_radix(int n, int p) {
+    if (fx_odd(n) == 1) return p2_radix(n, p);
+    if (p == 0) return fx_elems(n);
+    const int t = fx_lanes(n);
+    if (t <= 16) return t;
+    return p == 1 ? t / 4 : 4;
 }
 
-__host__ __device__ constexpr int p2slot(int i) { return i ^ ((i >> 4) & 15); }
+// LDS slot of element i of a scheduled line (lslot's swizzle where the
+// length is a multiple of 16).
+template <int N>
+__host__ __device__ constexpr int fxslot(int i) {
+    return N % 16 == 0 ? i ^ ((i >> 4) & 15) : i;
+}
 
-// Ordering point between the reads and the writes of a pass.  With N / 16
-// <= 64 lanes per line, every line lies inside one wavefront, whose LDS
-// operations execute in program order, so a wavefront-scope fence (which
-// also keeps the compiler from moving LDS accesses across it) replaces the
-// workgroup barrier and the other lines' waves run on independently.
+// Ordering point between the reads and the writes of a pass.  With at most
+// 64 lanes per line (a power of two), every line lies inside one wavefront,
+// whose LDS operations execute in program order, so a wavefront-scope fence
+// (which also keeps the compiler from moving LDS accesses across it) replaces
+// the workgroup barrier and the other lines' waves run on independently.
 // Callers that read other lines after the transform add their own barrier.
 template <int N>
 __device__ __forceinline__ void pass_sync() {
-    if constexpr (N / 16 <= 64) {
+    if constexpr (fx_lanes(N) <= 64) {
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         __builtin_amdgcn_wave_barrier();
     } else {
@@ -354,18 +479,19 @@ __device__ __forceinline__ void pass_sync() {
 // `lx` XORs every slot of the line (a per-line bank rotation for workgroups
 // that read several lines at one element index; 0 or a multiple of 4 < 32).
 template <typename T, int N, int R, int NS>
-__device__ __forceinline__ void stockham_pass_p2(cplx<T> *line, int t, const cplx<T> *tw, bool inv, int lx) {
-    constexpr int MB = lane_butterflies<R>();
-    constexpr int NT = N / 16, NR = N / R, ST = N / (NS * R);
-    static_assert(MB * NT == NR, "every butterfly has a lane");
+__device__ __forceinline__ void fx_pass(cplx<T> *line, int t, const cplx<T> *tw, bool inv, int lx) {
+    constexpr int NT = fx_lanes(N), NR = N / R, ST = N / (NS * R);
+    constexpr int MB = (NR + NT - 1) / NT;  // butterflies per lane; the last may be beyond NR
+    constexpr bool FULL = MB * NT == NR;
     cplx<T> v[MB][R];
     int base[MB];
 #pragma unroll
     for (int b = 0; b < MB; ++b) {
-        const int j = t + b * NT;
+        const int j0 = t + b * NT;
+        const int j = FULL || j0 < NR ? j0 : 0;  // an idle lane repeats butterfly 0 and drops it
         const int k = j % NS;
 #pragma unroll
-        for (int r = 0; r < R; ++r) v[b][r] = line[p2slot(j + r * NR) ^ lx];
+        for (int r = 0; r < R; ++r) v[b][r] = line[fxslot<N>(j + r * NR) ^ lx];
         // k = 0 multiplies by the table's exact w^0 = 1 (no branch: lanes of
         // one wave differ in k, and a branch would split the table loads)
         if (NS > 1) twiddle<T, R>(v[b], tw, k * ST, inv);
@@ -375,91 +501,70 @@ __device__ __forceinline__ void stockham_pass_p2(cplx<T> *line, int t, const cpl
     pass_sync<N>();
 #pragma unroll
     for (int b = 0; b < MB; ++b)
+        if (FULL || t + b * NT < NR)
 #pragma unroll
-        for (int r = 0; r < R; ++r) line[p2slot(base[b] + r * NS) ^ lx] = v[b][r];
+            for (int r = 0; r < R; ++r) line[fxslot<N>(base[b] + r * NS) ^ lx] = v[b][r];
     pass_sync<N>();
 }
 
 template <typename T, int N, int P, int NS>
-__device__ __forceinline__ void p2_passes(cplx<T> *line, int t, const cplx<T> *tw, bool inv, int lx) {
-    if constexpr (P < p2_npass(N)) {
-        constexpr int R = p2_radix(N, P);
-        stockham_pass_p2<T, N, R, NS>(line, t, tw, inv, lx);
-        p2_passes<T, N, P + 1, NS * R>(line, t, tw, inv, lx);
+__device__ __forceinline__ void fx_passes(cplx<T> *line, int t, const cplx<T> *tw, bool inv, int lx) {
+    if constexpr (P < fx_npass(N)) {
+        constexpr int R = fx_radix(N, P);
+        fx_pass<T, N, R, NS>(line, t, tw, inv, lx);
+        fx_passes<T, N, P + 1, NS * R>(line, t, tw, inv, lx);
     }
 }
 
-// The first pass of a fixed schedule whose first radix is 16, fed from
-// registers: lane t holds elements t + r N/16 (r < 16), exactly the inputs
-// of its butterfly, so the line need not be written to LDS and read back
-// before it.  Continue with p2_passes<T, N, 1, 16>.
-template <int N>
-constexpr bool p2_first_from_regs() {
-    return N >= 256 && p2_radix(N, 0) == 16;
-}
-
+// The first pass fed from registers: lane t holds elements t + e T (e < E),
+// which are exactly the inputs of its E / R butterflies, so the line need not
+// be written to LDS and read back before it.  fx_rest runs the other passes.
 template <typename T, int N>
-__device__ __forceinline__ void p2_first_pass_regs(cplx<T> *line, int t, cplx<T> v[16], const cplx<T> *tw,
-                                                   bool inv, int lx) {
-    static_assert(p2_first_from_regs<N>(), "first radix 16");
-    dft_any<T, 16>(v, tw, N, inv);
+__device__ __forceinline__ void fx_first_pass(cplx<T> *line, int t, const cplx<T> v[], const cplx<T> *tw, bool inv,
+                                              int lx) {
+    constexpr int R = fx_radix(N, 0), E = fx_elems(N), B = E / R, NT = fx_lanes(N);
+    static_assert(B * R == E, "whole butterflies per lane");
 #pragma unroll
-    for (int r = 0; r < 16; ++r) line[p2slot(t * 16 + r) ^ lx] = v[r];
+    for (int b = 0; b < B; ++b) {
+        cplx<T> u[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) u[r] = v[b + r * B];
+        dft_any<T, R>(u, tw, N, inv);
+#pragma unroll
+        for (int r = 0; r < R; ++r) line[fxslot<N>((t + b * NT) * R + r) ^ lx] = u[r];
+    }
     pass_sync<N>();
 }
+template <typename T, int N>
+__device__ __forceinline__ void fx_rest(cplx<T> *line, int t, const cplx<T> *tw, bool inv, int lx) {
+    fx_passes<T, N, 1, fx_radix(N, 0)>(line, t, tw, inv, lx);
+}
 
-// Line access policy: N > 0 a fixed power-of-two schedule (N / 16 lanes per
-// line), N == 0 the runtime plan.
+// Line access policy: N > 0 a compile-time schedule, N == 0 the runtime plan.
 template <int N>
 struct LineOps {
     __device__ __forceinline__ static int n(const LinePlan &lp) { return N ? N : lp.n; }
-    __device__ __forceinline__ static int threads(const LinePlan &lp) { return N ? N / 16 : lp.threads; }
-    __device__ __forceinline__ static int slot(const LinePlan &lp, int i) { return N ? p2slot(i) : lslot(lp, i); }
-    // Bank rotation of line j of a multi-line workgroup: fixed schedules of
-    // n >= 32 XOR the slots with (j mod 8) * 4, so eight lines read at one
-    // element index hit eight different bank groups without padding.
-    __device__ __forceinline__ static int line_xor(int j) { return N >= 32 ? ((j & 7) << 2) : 0; }
+    __device__ __forceinline__ static int threads(const LinePlan &lp) { return N ? fx_lanes(N) : lp.threads; }
+    __device__ __forceinline__ static int slot(const LinePlan &lp, int i) { return N ? fxslot<N>(i) : lslot(lp, i); }
+    // Bank rotation of line j of a multi-line workgroup: scheduled lengths
+    // that are a multiple of 32 XOR the slots with (j mod 8) * 4, so eight
+    // lines read at one element index hit eight different bank groups
+    // without padding.
+    __device__ __forceinline__ static int line_xor(int j) { return N >= 32 && N % 32 == 0 ? ((j & 7) << 2) : 0; }
     __device__ __forceinline__ static int slot(const LinePlan &lp, int i, int lx) {
-        return N ? (p2slot(i) ^ lx) : lslot(lp, i);
+        return N ? (fxslot<N>(i) ^ lx) : lslot(lp, i);
     }
     template <typename T>
     __device__ __forceinline__ static void fft(cplx<T> *line, const LinePlan &lp, int t, const cplx<T> *tw, bool inv,
                                                int lx = 0) {
         if constexpr (N > 0) {
             (void)lp;
-            p2_passes<T, N, 0, 1>(line, t, tw, inv, lx);
+            fx_passes<T, N, 0, 1>(line, t, tw, inv, lx);
         } else {
             (void)lx;
             line_fft(line, lp, t, tw, inv);
         }
     }
 };
-
-// Register-resident DFT of a short line (all n values in one lane), used for
-// the z transforms of thin films.  Direct O(n^2) sum with table roots for n
-// not a power of two <= 16.
-template <typename T, int N>
-__device__ __forceinline__ void reg_dft(cplx<T> *v, const cplx<T> *tw, bool inv) {
-    if constexpr (N == 1) {
-        (void)v; (void)tw; (void)inv;
-    } else if constexpr (N == 2 || N == 4 || N == 8 || N == 16) {
-        dft_any<T, N>(v, tw, N, inv);
-    } else {
-        cplx<T> out[N];
-#pragma unroll
-        for (int q = 0; q < N; ++q) {
-            cplx<T> acc = v[0];
-#pragma unroll
-            for (int r = 1; r < N; ++r) {
-                cplx<T> w = tw[(r * q) % N];
-                if (inv) w.y = -w.y;
-                acc = cadd(acc, cmul(v[r], w));
-            }
-            out[q] = acc;
-        }
-#pragma unroll
-        for (int q = 0; q < N; ++q) v[q] = out[q];
-    }
-}
 
 }  // namespace fm

@@ -48,8 +48,24 @@ void pow2_radices(int k, bool wide, std::vector<int> &out, int max_radix) {
 
 }  // namespace
 
-bool plan_line(int n, LinePlan &lp, std::string &err, int min_lanes, int max_radix) {
+int pick_padded(int n) {
+    const int m = 2 * n;
+    for (int l = m; 3 * (int64_t)l <= 4 * (int64_t)m; ++l)
+        if (fx_has(l)) return l;
+    return m;
+}
+
+bool plan_line(int n, LinePlan &lp, std::string &err, int min_lanes, int max_radix, bool fixed) {
     lp = LinePlan{};
+    if (fixed && min_lanes <= 1 && max_radix == 16 && fx_has(n)) {
+        lp.n = n;
+        lp.npass = fx_npass(n);
+        lp.threads = fx_lanes(n);
+        lp.swz = n % 16 == 0 ? 1 : 0;
+        lp.fixed = 1;
+        for (int p = 0; p < lp.npass; ++p) lp.radix[p] = fx_radix(n, p);
+        return true;
+    }
     if (n < 1) {
         err = "FFT line length must be >= 1";
         return false;
