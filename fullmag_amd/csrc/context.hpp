@@ -49,6 +49,18 @@ struct DemagTuning {
 // Applies "key=value,..." (unknown keys ignored) on top of t.
 void parse_tuning_string(DemagTuning &t, const char *text);
 
+// Octant tensor layout in reals: entry (kx, oy, oz) starts at kx skx + oy soy
+// + (oz >> 1) soz (+ odd for odd oz) and holds its components consecutively.
+// Short z lines (pz <= 16): one block per (kx, oy) column holding the even-oz
+// entries and then the odd-oz ones, each half padded to 16 bytes, so that a
+// lane owning kz of one parity reads its whole half with 16-byte loads (kz
+// and pz - kz share an entry and a parity).  Long z lines: oy is the fastest
+// index of the entries, so that lanes on neighbouring columns read
+// neighbouring entries.
+struct KernLayout {
+    int64_t skx = 0, soy = 0, soz = 0, odd = 0;
+};
+
 struct DemagPlan {
     DemagTuning tune;
     bool enabled = false;
@@ -75,9 +87,7 @@ struct DemagPlan {
     void *kern = nullptr;
     uint64_t spec_elems = 0;  // complex elements
     uint64_t kern_elems = 0;  // real elements
-    // tensor layout: one block of kblock reals per (kx, oy); the even-oz
-    // entries first, the odd-oz ones from kodd (see kern_at)
-    int kblock = 0, kodd = 0;
+    KernLayout kl;            // tensor layout (see kern_at)
 };
 
 // One kernel launch as recorded for a multi-instance batch: the kernel's

@@ -41,7 +41,7 @@ namespace {
 // stored at kern_at.  `total` counts kcomp * kz_n * hx * (ny + 1) entries.
 template <typename Real>
 __global__ void extract_octant_kernel(const cplx<double> *spec, Real *kern, int kz_n, int hx, int ny, int pz,
-                                      int py, int64_t total, int kblock, int kodd, int kcomp) {
+                                      int py, int64_t total, KernLayout kl) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= total) return;
     const int64_t ly = ny + 1;
@@ -51,7 +51,7 @@ __global__ void extract_octant_kernel(const cplx<double> *spec, Real *kern, int 
     const int oz = (int)(r / ((int64_t)hx * ly));
     r -= (int64_t)oz * hx * ly;
     const int kx = (int)(r / ly), oy = (int)(r - (int64_t)kx * ly);
-    kern[kern_at(kblock, kodd, kcomp, ly, c, oz, kx, oy)] = Real(spec[(((int64_t)c * pz + oz) * hx + kx) * py + oy].x);
+    kern[kern_at(kl, c, oz, kx, oy)] = Real(spec[(((int64_t)c * pz + oz) * hx + kx) * py + oy].x);
 }
 
 // ---------------------------------------------------------------------------
@@ -64,6 +64,15 @@ size_t lds_budget() { return 65536; }
 // longer than 64 KB takes one packed line (two rows) per workgroup when it
 // fits in `limit`, the device's LDS per workgroup (160 KB on gfx950).
 bool pick_x(const LinePlan &lp, size_t ce, int &xr, int &ls, int max_rows = 16, size_t limit = 65536) {
+    if (lp.fixed) {
+        // two workgroups of a CU's 160 KB; a line distance of 4 mod 32 slots
+        // puts eight lines read at one element index on different banks
+        ls = fx_size(lp.n);
+        ls += (36 - ls % 32) % 32;
+        for (xr = max_rows; xr > 2; xr >>= 1)
+            if (xr / 2 * lp.threads <= kMaxBlock && (size_t)(xr / 2) * ls * ce <= limit / 2) return true;
+        return lp.threads <= kMaxBlock && (size_t)ls * ce <= limit;
+    }
     for (xr = max_rows; xr >= 2; xr >>= 1) {
         const int lines = xr / 2;
         if (lines * lp.threads > kMaxBlock) continue;
@@ -122,8 +131,7 @@ KernelView<Real> kview(const Context &c) {
     KernelView<Real> K;
     K.k = dp.projection ? nullptr : static_cast<const Real *>(dp.kern);
     K.kcomp = dp.kcomp;
-    K.kb = dp.kblock;
-    K.kodd = dp.kodd;
+    K.l = dp.kl;
     K.kz_n = dp.kz_n;
     K.ny = dp.py / 2;
     K.nz = dp.pz / 2;
@@ -301,6 +309,7 @@ void demag_transform_t(Context &c, const S *src, const XArgs<Real> &xa, unsigned
                 za.py = dp.py;
                 za.pitch = dp.rows;
                 za.K = K;
+                za.xcd = dp.tune.xcd;
                 launch_zlds<Real>(c, za, 1);
             }
         }
@@ -433,7 +442,10 @@ bool plan_lines(DemagPlan &dp, std::string &err) {
     const bool fx = t.fixed != 0;
     if (!plan_line(dp.px, dp.lx, err, std::max(1, t.x_lanes), t.x_radix, fx)) return false;
     if (!plan_line(dp.py, dp.ly, err, std::max(1, t.y_lanes), t.y_radix, fx)) return false;
-    if (dp.three_d && !plan_line(dp.pz, dp.lz, err, 1, 16, fx)) return false;
+    // the scheduled z lines read the tensor entries directly (no projection
+    // fallback) and keep a line in one wavefront
+    const bool fz = fx && !dp.projection && fx_has(dp.pz) && fx_lanes(dp.pz) <= 64 && dp.pz > 16;
+    if (dp.three_d && !plan_line(dp.pz, dp.lz, err, 1, 16, fz)) return false;
     return true;
 }
 
@@ -574,8 +586,7 @@ bool host_octant_from_spectra(const DemagPlan &dp, const fullmag_fdm_plan_desc &
                             plan.demag_kernel_zz_spectrum, plan.demag_kernel_xy_spectrum,
                             plan.demag_kernel_xz_spectrum, plan.demag_kernel_yz_spectrum};
     const int pz = dp.three_d ? dp.pz : 1;
-    const int64_t ly = dp.py / 2 + 1;
-    kern.assign((size_t)dp.hx * ly * dp.kblock, 0.0);
+    kern.assign((size_t)(dp.hx * dp.kl.skx), 0.0);
     // parity of the six components along (x, y, z)
     const int odd[6][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}, {1, 1, 0}, {1, 0, 1}, {0, 1, 1}};
     double kmax = 0.0, bad = 0.0;
@@ -598,7 +609,7 @@ bool host_octant_from_spectra(const DemagPlan &dp, const fullmag_fdm_plan_desc &
                     const int64_t j = ((int64_t)oz * dp.py + oy) * dp.px + ox;
                     bad = std::max(bad, std::fabs(re - sg * s[2 * j]));
                     if (x <= dp.nx && y <= dp.ny && (pz == 1 || z <= dp.nz) && c < dp.kcomp)
-                        kern[kern_at(dp.kblock, dp.kodd, dp.kcomp, ly, c, z, x, y)] = re;
+                        kern[kern_at(dp.kl, c, z, x, y)] = re;
                 }
     }
     if (bad > 1e-8 * std::max(kmax, 1e-300)) {
@@ -640,11 +651,21 @@ template <typename Real>
 bool plan_geometry(DemagPlan &dp, std::string &err, int keep_split = -1) {
     const size_t ce = sizeof(cplx<Real>);
     {
-        // tensor blocks: even-oz half, then odd-oz half, each padded to 16 bytes
-        const int vec = 16 / (int)sizeof(Real);
-        const int nzo = dp.kz_n, ne = (nzo + 1) / 2, no = nzo / 2;  // octant kz entries of either parity
-        dp.kodd = (int)cdiv(ne * dp.kcomp, vec) * vec;
-        dp.kblock = dp.kodd + (int)cdiv(no * dp.kcomp, vec) * vec;
+        const int64_t ly = dp.py / 2 + 1, nzo = dp.kz_n;
+        KernLayout &l = dp.kl;
+        if (dp.three_d && dp.pz > z_reg_max<Real>()) {
+            l.soy = dp.kcomp;
+            l.odd = ly * dp.kcomp;
+            l.soz = 2 * l.odd;
+            l.skx = nzo * l.odd;
+        } else {
+            const int64_t vec = 16 / (int64_t)sizeof(Real);
+            const int64_t ne = (nzo + 1) / 2, no = nzo / 2;  // octant kz entries of either parity
+            l.soz = dp.kcomp;
+            l.odd = (int64_t)cdiv(ne * dp.kcomp, vec) * vec;
+            l.soy = l.odd + (int64_t)cdiv(no * dp.kcomp, vec) * vec;
+            l.skx = ly * l.soy;
+        }
     }
     if (!pick_x(dp.lx, ce, dp.xr, dp.x_ls, dp.tune.x_rows > 0 ? dp.tune.x_rows : 16, dp.lds_limit)) {
         err = "x line FFT does not fit in one workgroup";
@@ -674,7 +695,7 @@ bool plan_geometry(DemagPlan &dp, std::string &err, int keep_split = -1) {
         // a scheduled column is three lines of whole wavefront shares: about
         // one wavefront per workgroup keeps the most workgroups in flight
         dp.yconv_kpw = dp.ly.fixed ? std::max(1, 64 / (3 * dp.ly.threads)) : pick_lpw(dp.ly, ce, 3);
-        const bool split = dp.tune.y_split != 0 || (size_t)3 * dp.yconv_kpw * (dp.ly.n + kPad) * ce > dp.lds_limit ||
+        const bool split = dp.tune.y_split != 0 || (size_t)3 * dp.yconv_kpw * line_slots(dp.ly) * ce > dp.lds_limit ||
                            3 * dp.yconv_kpw * dp.ly.threads > 1024;
         if (keep_split >= 0 && split != (keep_split != 0)) {
             err = "schedule changes the thin-film y convolution form";
@@ -715,7 +736,7 @@ bool setup_t(Context &c, const fullmag_fdm_plan_desc &plan) {
     newell_octant(dp.nx, dp.ny, dp.three_d ? dp.nz : 1, c.dx, c.dy, c.dz, oct);
     cplx<double> *spec = nullptr;
     if (!newell_forward(c, dp, oct, &spec, c.last_error)) return false;
-    dp.kern_elems = (uint64_t)dp.hx * (dp.py / 2 + 1) * dp.kblock;
+    dp.kern_elems = (uint64_t)(dp.hx * dp.kl.skx);
     const int64_t entries = (int64_t)dp.kcomp * dp.kz_n * dp.hx * (dp.py / 2 + 1);
     bool ok = ctx_alloc(c, &dp.kern, dp.kern_elems * sizeof(Real), "demag tensor") &&
               hip_ok(hipMemsetAsync(dp.kern, 0, dp.kern_elems * sizeof(Real), c.stream), "hipMemsetAsync(tensor)",
@@ -724,7 +745,7 @@ bool setup_t(Context &c, const fullmag_fdm_plan_desc &plan) {
         const int pz = dp.three_d ? dp.pz : 1;
         hipLaunchKernelGGL((extract_octant_kernel<Real>), dim3((unsigned)cdiv(entries, 256)), dim3(256), 0,
                            c.stream, spec, static_cast<Real *>(dp.kern), dp.kz_n, dp.hx, dp.py / 2, pz, dp.py, entries,
-                           dp.kblock, dp.kodd, dp.kcomp);
+                           dp.kl);
         ok = hip_ok(hipStreamSynchronize(c.stream), "extract octant", c.last_error);
     }
     (void)hipFree(spec);

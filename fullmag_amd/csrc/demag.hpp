@@ -10,7 +10,9 @@
 
 namespace fm {
 
-constexpr int kPad = 1;         // LDS line padding (complex slots)
+constexpr int kPad = 1;         // LDS line padding (complex slots) of runtime-planned lines
+// LDS slots of one line.
+inline int line_slots(const LinePlan &lp) { return lp.fixed ? fx_size(lp.n) : lp.n + kPad; }
 
 // Stand-ins read in place of an absent optional per-cell array, so that the
 // read itself needs no branch: an active-mask byte of 1 and a value of 1.
@@ -45,19 +47,14 @@ template <typename Real>
 struct KernelView {
     const Real *k = nullptr;  // octant tensor, nullptr for the projection fallback
     int kcomp = 6, kz_n = 1;
-    int kb = 0, kodd = 0;     // block per (kx, oy) and offset of its odd-oz half
+    KernLayout l;
     int ny = 0, nz = 0, py = 0, pz = 1, hx = 0;
     double kxs = 0, kys = 0, kzs = 0;  // 2 pi / (p d) per axis (projection)
 };
 
-// Octant tensor layout: one block of `kblock` reals per (kx, oy) column,
-// holding the entries of even oz (0, 2, ...) and, from `kodd`, those of odd
-// oz, each entry `kcomp` consecutive components, each half padded to 16
-// bytes.  A z-transform lane that owns kz of one parity reads its whole half
-// with 16-byte loads (kz and pz - kz share an entry and a parity).
-__host__ __device__ __forceinline__ int64_t kern_at(int kblock, int kodd, int kcomp, int64_t ly, int c, int oz,
-                                                    int kx, int oy) {
-    return ((int64_t)kx * ly + oy) * kblock + ((oz & 1) ? kodd : 0) + (int64_t)(oz >> 1) * kcomp + c;
+// Entry (kx, oy, oz), component c of the octant tensor (KernLayout).
+__host__ __device__ __forceinline__ int64_t kern_at(const KernLayout &l, int c, int oz, int kx, int oy) {
+    return kx * l.skx + oy * l.soy + ((oz & 1) ? l.odd : 0) + (oz >> 1) * l.soz + c;
 }
 
 // t = (xx, yy, zz, xy, xz, yz) at frequency (kx, ky, kz); kx <= nx.
@@ -74,7 +71,7 @@ __device__ __forceinline__ void tensor_at(const KernelView<Real> &K, int kx, int
             oz = zlo ? kz : K.pz - kz;
             sz = zlo ? Real(1) : Real(-1);
         }
-        const Real *e = K.k + kern_at(K.kb, K.kodd, K.kcomp, K.ny + 1, 0, oz, kx, oy);
+        const Real *e = K.k + kern_at(K.l, 0, oz, kx, oy);
         t[0] = e[0];
         t[1] = e[1];
         t[2] = e[2];
@@ -291,6 +288,7 @@ struct ZLdsArgs {
     int inverse;  // conv = 0: the inverse transform (n_in = pz, n_out <= pz)
     int64_t columns, zstride, comp_stride;
     int py, pitch;
+    int xcd;  // renumber workgroups per XCD
     KernelView<Real> K;
 };
 

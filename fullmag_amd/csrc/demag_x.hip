@@ -10,134 +10,146 @@ namespace {
 // (c = blockIdx.z, z = blockIdx.y).  Rows 2j, 2j+1 are packed as a + i b;
 // with Z = FFT(a + i b):  A_k = (Z_k + conj Z_{N-k}) / 2,
 // B_k = (Z_k - conj Z_{N-k}) / (2i), k = 0..N/2, stored at spec[c][z][k][y].
-template <typename Real, class Src, int N>
-__device__ __forceinline__ void xfwd_body(const XArgs<Real> &a, const Src &src, cplx<Real> *spec, int c) {
-    using L = LineOps<N>;
+template <typename Real>
+__device__ __forceinline__ void xfwd_split(cplx<Real> zk, cplx<Real> zn, cplx<Real> &A, cplx<Real> &B) {
+    const Real h = Real(0.5);
+    A = {h * (zk.x + zn.x), h * (zk.y - zn.y)};
+    B = {h * (zk.y + zn.y), h * (zn.x - zk.x)};
+}
+
+// Runtime-planned lines.
+template <typename Real, class Src>
+__device__ __forceinline__ void xfwd_body_rt(const XArgs<Real> &a, const Src &src, cplx<Real> *spec, int c) {
     extern __shared__ unsigned char smem_raw[];
     cplx<Real> *lds = reinterpret_cast<cplx<Real> *>(smem_raw);
     const int LINES = a.xr >> 1;
-    const int n = L::n(a.lp), ls = a.ls, T = L::threads(a.lp);
+    const int n = a.lp.n, ls = a.ls, T = a.lp.threads;
     const int tid = threadIdx.x, nthr = blockDim.x;
     const int y0 = blockIdx.x * a.xr, z = blockIdx.y;
     // the T lanes of packed line j (= tid / T, blockDim.x = LINES * T) load it
-    const int jl = tid / T, t = tid - jl * T;
+    const int jl = tid / T, t = tid - jl * T, ya = y0 + 2 * jl;
     cplx<Real> *line = lds + jl * ls;
-    const int lx = L::line_xor(jl);
-    {
-        const int ya = y0 + 2 * jl;
-        if constexpr (N > 0) {
-            // scheduled length: all loads of a lane in flight before the first pass
-            constexpr int E = fx_elems(N), NT = fx_lanes(N);
-            cplx<Real> v[E];
-            if (!Src::kGather && src.uniform() && 2 * a.n_in <= N) {
-                // branch-free: clamped addresses, every load issued before
-                // any is used; elements t + e NT with e >= E / 2 lie in
-                // the zero padding (n_in <= N/2) and are not loaded
-                const bool oka = ya < a.rows, okb = ya + 1 < a.rows;
-                const int yA = oka ? ya : 0, yB = okb ? ya + 1 : 0;
-#pragma unroll
-                for (int e = 0; e < E / 2; ++e) {
-                    const int x = t + e * NT;
-                    const bool okx = x < a.n_in;
-                    const int xs = okx ? x : 0;
-                    const Real va = src.uniform_at(c, z, yA, xs), vb = src.uniform_at(c, z, yB, xs);
-                    v[e] = {(okx && oka) ? va : Real(0), (okx && okb) ? vb : Real(0)};
-                }
-#pragma unroll
-                for (int e = E / 2; e < E; ++e) v[e] = {Real(0), Real(0)};
-            } else if (Src::kGather && 2 * a.n_in <= N) {
-                // the same with the mask, volume fraction and per-cell Ms
-                // read beside each element, all unconditionally
-                const bool oka = ya < a.rows, okb = ya + 1 < a.rows;
-                const int yA = oka ? ya : 0, yB = okb ? ya + 1 : 0;
-#pragma unroll
-                for (int e = 0; e < E / 2; ++e) {
-                    const int x = t + e * NT;
-                    const bool okx = x < a.n_in;
-                    const int xs = okx ? x : 0;
-                    const Real va = src.gather_at(c, z, yA, xs), vb = src.gather_at(c, z, yB, xs);
-                    v[e] = {(okx && oka) ? va : Real(0), (okx && okb) ? vb : Real(0)};
-                }
-#pragma unroll
-                for (int e = E / 2; e < E; ++e) v[e] = {Real(0), Real(0)};
-            } else {
-#pragma unroll
-                for (int e = 0; e < E; ++e) {
-                    const int x = t + e * NT;
-                    v[e] = {Real(0), Real(0)};
-                    if (x < a.n_in) {
-                        if (ya < a.rows) v[e].x = src(c, z, ya, x);
-                        if (ya + 1 < a.rows) v[e].y = src(c, z, ya + 1, x);
-                    }
-                }
-            }
-            // the loaded elements are the first pass's inputs
-            fx_first_pass<Real, N>(line, t, v, a.tw, false, lx);
-            fx_rest<Real, N>(line, t, a.tw, false, lx);
-        } else {
-            for (int x = t; x < n; x += T) {
-                cplx<Real> v = {Real(0), Real(0)};
-                if (x < a.n_in) {
-                    if (ya < a.rows) v.x = src(c, z, ya, x);
-                    if (ya + 1 < a.rows) v.y = src(c, z, ya + 1, x);
-                }
-                line[L::slot(a.lp, x, lx)] = v;
-            }
-            __syncthreads();
-            L::template fft<Real>(line, a.lp, t, a.tw, false, lx);
+    for (int x = t; x < n; x += T) {
+        cplx<Real> v = {Real(0), Real(0)};
+        if (x < a.n_in) {
+            if (ya < a.rows) v.x = src(c, z, ya, x);
+            if (ya + 1 < a.rows) v.y = src(c, z, ya + 1, x);
         }
+        line[lslot(a.lp, x)] = v;
+    }
+    __syncthreads();
+    line_fft(line, a.lp, t, a.tw, false);
+    __syncthreads();  // the unpack reads every line
+    // lane (j, k) splits line j into rows 2j (A) and 2j + 1 (B) at kx = k
+    for (int idx = tid; idx < a.g.hx * LINES; idx += nthr) {
+        const int j = idx & (LINES - 1), k = idx >> (a.xr_log2 - 1), y = y0 + 2 * j;
+        if (y >= a.rows) continue;
+        cplx<Real> A, B;
+        xfwd_split(lds[j * ls + lslot(a.lp, k)], lds[j * ls + lslot(a.lp, k == 0 ? 0 : n - k)], A, B);
+        cplx<Real> *dst = spec + a.g.at(c, z, k, y);
+        dst[0] = A;
+        if (y + 1 < a.rows) dst[1] = B;
+    }
+}
+
+// Scheduled lines.  A lane's loads are all in flight before the first pass,
+// which takes them from registers.  In the unpack a lane keeps its line (FP32:
+// pair of rows) and walks kx = k0 + u T, so each step is one pointer
+// increment and one LDS read per side at a fixed distance.
+template <typename Real, class Src, int N>
+__device__ __forceinline__ void xfwd_body(const XArgs<Real> &a, const Src &src, cplx<Real> *spec, int c) {
+    constexpr int E = fx_elems(N), T = fx_lanes(N);
+    extern __shared__ unsigned char smem_raw[];
+    cplx<Real> *lds = reinterpret_cast<cplx<Real> *>(smem_raw);
+    const int LINES = a.xr >> 1, ls = a.ls;
+    const int tid = threadIdx.x;
+    const int y0 = blockIdx.x * a.xr, z = blockIdx.y;
+    {
+        const int jl = tid / T, t = tid % T, ya = y0 + 2 * jl;
+        cplx<Real> *line = lds + jl * ls;
+        cplx<Real> v[E];
+        // branch-free: clamped addresses, every load issued before any is
+        // used; elements t + e T with e >= E / 2 lie in the zero padding
+        // (n_in <= N / 2) and are not loaded
+        const bool oka = ya < a.rows, okb = ya + 1 < a.rows;
+        const int yA = oka ? ya : 0, yB = okb ? ya + 1 : 0;
+#pragma unroll
+        for (int e = 0; e < E / 2; ++e) {
+            const int x = t + e * T;
+            const bool okx = x < a.n_in;
+            const int xs = okx ? x : 0;
+            Real va, vb;
+            if constexpr (Src::kGather) {
+                // the mask, volume fraction and per-cell Ms are read beside
+                // each element, all unconditionally
+                va = src.gather_at(c, z, yA, xs);
+                vb = src.gather_at(c, z, yB, xs);
+            } else {
+                va = src.uniform_at(c, z, yA, xs);
+                vb = src.uniform_at(c, z, yB, xs);
+            }
+            v[e] = {(okx && oka) ? va : Real(0), (okx && okb) ? vb : Real(0)};
+        }
+#pragma unroll
+        for (int e = E / 2; e < E; ++e) v[e] = {Real(0), Real(0)};
+        fx_first_pass<Real, N>(line, t, v, a.tw, false);
+        fx_rest<Real, N>(line, t, a.tw, false);
     }
     __syncthreads();  // the unpack reads every line
-    const int hx = a.g.hx;
-    // lane (j, k) splits line j into rows 2j (A) and 2j + 1 (B) at kx = k;
-    // the two are adjacent in memory (one 16-byte store in FP32 when the
-    // row pitch is even)
     if constexpr (sizeof(Real) == 8) {
         // FP64: one 16-byte complex per lane, consecutive lanes on consecutive rows
-        for (int idx = tid; idx < hx * a.xr; idx += nthr) {
-            const int yl = idx & (a.xr - 1), k = idx >> a.xr_log2;
-            const int y = y0 + yl;
-            if (y >= a.rows) continue;
-            const int j = yl >> 1, jx = L::line_xor(j);
-            const cplx<Real> zk = lds[j * ls + L::slot(a.lp, k, jx)];
-            const cplx<Real> zn = lds[j * ls + L::slot(a.lp, k == 0 ? 0 : n - k, jx)];
-            const Real h = Real(0.5);
-            cplx<Real> v;
-            if ((yl & 1) == 0) v = {h * (zk.x + zn.x), h * (zk.y - zn.y)};
-            else v = {h * (zk.y + zn.y), h * (zn.x - zk.x)};
-            spec[a.g.at(c, z, k, y)] = v;
+        constexpr int KS = T / 2;  // LINES T lanes over 2 LINES rows
+        const int yl = tid & (a.xr - 1), k0 = tid >> a.xr_log2, y = y0 + yl;
+        if (y >= a.rows) return;
+        const cplx<Real> *ln = lds + (yl >> 1) * ls;
+        cplx<Real> *dst = spec + a.g.at(c, z, k0, y);
+        const bool odd = (yl & 1) != 0;
+        auto one = [&](int k, int kn, cplx<Real> *d) {
+            // A or B of xfwd_split, selected by value (a select of the two
+            // structs goes through scratch)
+            const cplx<Real> zk = ln[fxslot<N>(k)], zn = ln[fxslot<N>(kn)];
+            const Real p = odd ? zk.y : zk.x, q = odd ? zn.y : zn.x;
+            const Real r = odd ? zn.x : zk.y, s = odd ? zk.x : zn.y;
+            *d = {Real(0.5) * (p + q), Real(0.5) * (r - s)};
+        };
+#pragma unroll
+        for (int u = 0; u < E; ++u) {
+            const int k = k0 + u * KS;
+            one(k, u == 0 && k0 == 0 ? 0 : N - k, dst + (int64_t)(u * KS) * a.g.pitch);
         }
-        return;
-    }
-    const bool pair16 = (a.g.pitch & 1) == 0;
-    for (int idx = tid; idx < hx * LINES; idx += nthr) {
-        const int j = idx & (LINES - 1), k = idx >> (a.xr_log2 - 1);
-        const int y = y0 + 2 * j;
-        if (y >= a.rows) continue;
-        const int jx = L::line_xor(j);
-        const cplx<Real> zk = lds[j * ls + L::slot(a.lp, k, jx)];
-        const cplx<Real> zn = lds[j * ls + L::slot(a.lp, k == 0 ? 0 : n - k, jx)];
-        const Real h = Real(0.5);
-        const cplx<Real> A = {h * (zk.x + zn.x), h * (zk.y - zn.y)};
-        const cplx<Real> B = {h * (zk.y + zn.y), h * (zn.x - zk.x)};
-        cplx<Real> *dst = spec + a.g.at(c, z, k, y);
-        if (y + 1 < a.rows) {
-            if (pair16) {
-                *reinterpret_cast<float4 *>(dst) = float4{float(A.x), float(A.y), float(B.x), float(B.y)};
+        if (k0 == 0) one(N / 2, N / 2, dst + (int64_t)(N / 2) * a.g.pitch);
+    } else {
+        // lane (j, k) splits line j into rows 2j (A) and 2j + 1 (B); the two
+        // are adjacent in memory (one 16-byte store when the row pitch is even)
+        const int j = tid & (LINES - 1), k0 = tid >> (a.xr_log2 - 1), y = y0 + 2 * j;
+        if (y >= a.rows) return;
+        const bool pair16 = (a.g.pitch & 1) == 0, two = y + 1 < a.rows;
+        const cplx<Real> *ln = lds + j * ls;
+        cplx<Real> *dst = spec + a.g.at(c, z, k0, y);
+        auto one = [&](int k, int kn, cplx<Real> *d) {
+            cplx<Real> A, B;
+            xfwd_split(ln[fxslot<N>(k)], ln[fxslot<N>(kn)], A, B);
+            if (two && pair16) {
+                *reinterpret_cast<float4 *>(d) = float4{float(A.x), float(A.y), float(B.x), float(B.y)};
             } else {
-                dst[0] = A;
-                dst[1] = B;
+                d[0] = A;
+                if (two) d[1] = B;
             }
-        } else {
-            dst[0] = A;
+        };
+#pragma unroll
+        for (int u = 0; u < E / 2; ++u) {
+            const int k = k0 + u * T;
+            one(k, u == 0 && k0 == 0 ? 0 : N - k, dst + (int64_t)(u * T) * a.g.pitch);
         }
+        if (k0 == 0) one(N / 2, N / 2, dst + (int64_t)(N / 2) * a.g.pitch);
     }
 }
 
 // Component c = blockIdx.z.
 template <typename Real, class Src, int N = 0>
 __global__ void __launch_bounds__(kMaxBlock) xfwd_kernel(XArgs<Real> a, Src src, cplx<Real> *spec) {
-    xfwd_body<Real, Src, N>(a, src, spec, (int)blockIdx.z);
+    if constexpr (N > 0) xfwd_body<Real, Src, N>(a, src, spec, (int)blockIdx.z);
+    else xfwd_body_rt<Real, Src>(a, src, spec, (int)blockIdx.z);
 }
 
 // Multi-instance form: instance blockIdx.z / zdiv of the table, component
@@ -152,7 +164,7 @@ struct XFwdPack {
     Src src;
     cplx<Real> *spec;
 };
-template <typename Real, class Src, int N = 0>
+template <typename Real, class Src, int N>
 __global__ void __launch_bounds__(kMaxBlock) xfwd_multi(const XFwdPack<Real, Src> *tab, int zdiv) {
     const XFwdPack<Real, Src> p = tab[blockIdx.z / zdiv];
     xfwd_body<Real, Src, N>(p.a, p.src, p.spec, (int)(blockIdx.z % zdiv));
@@ -161,99 +173,118 @@ __global__ void __launch_bounds__(kMaxBlock) xfwd_multi(const XFwdPack<Real, Src
 // Inverse complex-to-real along x: Z_k = A_k + i B_k for k <= N/2 and the
 // Hermitian continuation A_{N-k} = conj A_k; z = IFFT(Z); rows a = Re z,
 // b = Im z.  Reads spec[c][z][k][y0..y0+xr-1].
-template <typename Real, class Sink, int N>
-__device__ __forceinline__ void xinv_body(const XArgs<Real> &a, const cplx<Real> *spec, const Sink &sink, int c) {
-    using L = LineOps<N>;
+// Runtime-planned lines.
+template <typename Real, class Sink>
+__device__ __forceinline__ void xinv_body_rt(const XArgs<Real> &a, const cplx<Real> *spec, const Sink &sink, int c) {
     extern __shared__ unsigned char smem_raw[];
     cplx<Real> *lds = reinterpret_cast<cplx<Real> *>(smem_raw);
     const int LINES = a.xr >> 1;
-    const int n = L::n(a.lp), ls = a.ls, T = L::threads(a.lp);
+    const int n = a.lp.n, ls = a.ls, T = a.lp.threads;
     const int tid = threadIdx.x, nthr = blockDim.x;
     const int y0 = blockIdx.x * a.xr, z = blockIdx.y;
     const int hx = a.g.hx;
-    // consecutive lanes read consecutive rows of one kx column
-    auto put = [&](int idx, cplx<Real> A, cplx<Real> B) {
-        const int j = idx & (LINES - 1), k = idx >> (a.xr_log2 - 1);
-        const int jx = L::line_xor(j);
-        lds[j * ls + L::slot(a.lp, k, jx)] = {A.x - B.y, A.y + B.x};
-        if (k > 0 && k < n - k) lds[j * ls + L::slot(a.lp, n - k, jx)] = {A.x + B.y, B.x - A.y};
-    };
-    if constexpr (N > 0) {
-        // fixed length: every load of the lane (hx / T <= U row pairs) in
-        // flight before the LDS writes; a row pair is one 16-byte load in
-        // FP32 when the row pitch is even
-        constexpr int U = (N / 2 + 1 + fx_lanes(N) - 1) / fx_lanes(N);
-        const bool pair16 = sizeof(Real) == 4 && (a.g.pitch & 1) == 0;
+    // consecutive lanes read consecutive rows of one kx column, in batches of
+    // four loads per lane in flight before their LDS writes
+    constexpr int U = 4;
+    for (int base = tid; base < hx * LINES; base += U * nthr) {
         cplx<Real> A[U], B[U];
-        // branch-free: clamped addresses, selects after the loads
-        if (pair16) {
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int idx = tid + u * nthr;
-                const int j = idx & (LINES - 1), k = idx >> (a.xr_log2 - 1);
-                const int ya = y0 + 2 * j;
-                const bool oka = k < hx && ya < a.rows, okb = oka && ya + 1 < a.rows;
-                // an even row pitch and an even ya keep the pair 16-byte aligned
-                const float4 q = *reinterpret_cast<const float4 *>(spec + (oka ? a.g.at(c, z, k, ya) : 0));
-                A[u] = oka ? cplx<Real>{Real(q.x), Real(q.y)} : cplx<Real>{Real(0), Real(0)};
-                B[u] = okb ? cplx<Real>{Real(q.z), Real(q.w)} : cplx<Real>{Real(0), Real(0)};
-            }
-        } else {
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int idx = tid + u * nthr;
-                const int j = idx & (LINES - 1), k = idx >> (a.xr_log2 - 1);
-                const int ya = y0 + 2 * j;
-                const bool oka = k < hx && ya < a.rows, okb = oka && ya + 1 < a.rows;
-                const cplx<Real> qa = spec[oka ? a.g.at(c, z, k, ya) : 0];
-                const cplx<Real> qb = spec[okb ? a.g.at(c, z, k, ya + 1) : 0];
-                A[u] = oka ? qa : cplx<Real>{Real(0), Real(0)};
-                B[u] = okb ? qb : cplx<Real>{Real(0), Real(0)};
+        for (int u = 0; u < U; ++u) {
+            const int idx = base + u * nthr;
+            const int j = idx & (LINES - 1), k = idx >> (a.xr_log2 - 1);
+            const int ya = y0 + 2 * j;
+            A[u] = B[u] = {Real(0), Real(0)};
+            if (idx < hx * LINES) {
+                if (ya < a.rows) A[u] = spec[a.g.at(c, z, k, ya)];
+                if (ya + 1 < a.rows) B[u] = spec[a.g.at(c, z, k, ya + 1)];
             }
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int idx = tid + u * nthr;
-            if (idx < hx * LINES) put(idx, A[u], B[u]);
-        }
-    } else {
-        // batches of four loads per lane in flight before their LDS writes
-        constexpr int U = 4;
-        for (int base = tid; base < hx * LINES; base += U * nthr) {
-            cplx<Real> A[U], B[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int idx = base + u * nthr;
-                const int j = idx & (LINES - 1), k = idx >> (a.xr_log2 - 1);
-                const int ya = y0 + 2 * j;
-                A[u] = B[u] = {Real(0), Real(0)};
-                if (idx < hx * LINES) {
-                    if (ya < a.rows) A[u] = spec[a.g.at(c, z, k, ya)];
-                    if (ya + 1 < a.rows) B[u] = spec[a.g.at(c, z, k, ya + 1)];
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int idx = base + u * nthr;
-                if (idx >= hx * LINES) break;
-                put(idx, A[u], B[u]);
-            }
+            const int idx = base + u * nthr;
+            if (idx >= hx * LINES) break;
+            const int j = idx & (LINES - 1), k = idx >> (a.xr_log2 - 1);
+            lds[j * ls + lslot(a.lp, k)] = {A[u].x - B[u].y, A[u].y + B[u].x};
+            if (k > 0 && k < n - k) lds[j * ls + lslot(a.lp, n - k)] = {A[u].x + B[u].y, B[u].x - A[u].y};
         }
     }
     __syncthreads();
     const int jl = tid / T, t = tid - jl * T;
     const cplx<Real> *line = lds + jl * ls;
-    const int lx = L::line_xor(jl);
-    L::template fft<Real>(lds + jl * ls, a.lp, t, a.tw, true, lx);
+    line_fft(lds + jl * ls, a.lp, t, a.tw, true);
     // the lanes of line jl store its rows 2 jl (real part) and 2 jl + 1
     const int ya = y0 + 2 * jl;
-    if constexpr (N > 0 && std::is_same<Sink, FieldSink<float>>::value) {
+    for (int x = t; x < a.n_out; x += T) {
+        const cplx<Real> v = line[lslot(a.lp, x)];
+        if (ya < a.rows) sink(c, z, ya, x, v.x * a.scale);
+        if (ya + 1 < a.rows) sink(c, z, ya + 1, x, v.y * a.scale);
+    }
+}
+
+// Scheduled lines.  Every load of a lane (kx = k0 + u T of one row pair) is in
+// flight before the first LDS write; the addresses and LDS slots advance by
+// fixed steps.
+template <typename Real, class Sink, int N>
+__device__ __forceinline__ void xinv_body(const XArgs<Real> &a, const cplx<Real> *spec, const Sink &sink, int c) {
+    constexpr int E = fx_elems(N), T = fx_lanes(N), H = E / 2;
+    extern __shared__ unsigned char smem_raw[];
+    cplx<Real> *lds = reinterpret_cast<cplx<Real> *>(smem_raw);
+    const int LINES = a.xr >> 1, ls = a.ls;
+    const int tid = threadIdx.x;
+    const int y0 = blockIdx.x * a.xr, z = blockIdx.y;
+    {
+        // lane (j, k0): rows 2j and 2j + 1; consecutive lanes read
+        // consecutive rows of one kx column (a row pair is one 16-byte load
+        // in FP32 when the row pitch is even); u = H is kx = N / 2
+        const int j = tid & (LINES - 1), k0 = tid >> (a.xr_log2 - 1), ya = y0 + 2 * j;
+        const bool oka = ya < a.rows, okb = ya + 1 < a.rows;
+        const cplx<Real> *s = spec + a.g.at(c, z, k0, oka ? ya : 0);
+        cplx<Real> A[H + 1], B[H + 1];
+        auto off = [&](int u) { return (int64_t)(u < H ? u * T : k0 == 0 ? N / 2 : 0) * a.g.pitch; };
+        if (sizeof(Real) == 4 && (a.g.pitch & 1) == 0) {
+#pragma unroll
+            for (int u = 0; u <= H; ++u) {
+                // an even row pitch and an even ya keep the pair 16-byte aligned
+                const float4 q = *reinterpret_cast<const float4 *>(s + off(u));
+                A[u] = {Real(q.x), Real(q.y)};
+                B[u] = {Real(q.z), Real(q.w)};
+            }
+        } else {
+            const int nb = okb ? 1 : 0;
+#pragma unroll
+            for (int u = 0; u <= H; ++u) {
+                A[u] = s[off(u)];
+                B[u] = s[off(u) + nb];
+            }
+        }
+        cplx<Real> *ln = lds + j * ls;
+#pragma unroll
+        for (int u = 0; u <= H; ++u) {
+            const int k = u < H ? k0 + u * T : N / 2;
+            if (!oka) A[u] = {Real(0), Real(0)};
+            if (!okb) B[u] = {Real(0), Real(0)};
+            if (u < H || k0 == 0) ln[fxslot<N>(k)] = {A[u].x - B[u].y, A[u].y + B[u].x};
+            if (u < H && (u > 0 || k0 > 0)) ln[fxslot<N>(N - k)] = {A[u].x + B[u].y, B[u].x - A[u].y};
+        }
+    }
+    __syncthreads();
+    const int jl = tid / T, t = tid % T;
+    cplx<Real> *line = lds + jl * ls;
+    {
+        cplx<Real> v[E];
+        fx_load<Real, N>(line, t, v);
+        fx_first_pass<Real, N>(line, t, v, a.tw, true);
+        fx_rest<Real, N>(line, t, a.tw, true);
+    }
+    // the lanes of line jl store its rows 2 jl (real part) and 2 jl + 1
+    const int ya = y0 + 2 * jl;
+    if constexpr (std::is_same<Sink, FieldSink<float>>::value) {
         if (2 * a.n_out <= N && sink.masked() && (a.n_out & 3) == 0 && (sink.n & 3) == 0) {
             // four consecutive outputs of a row per lane: their mask bytes in
             // one 4-byte load, every mask word read before the first store,
             // and the values in one 16-byte store (rows start on 16-byte
             // boundaries: nx = n_out and n are multiples of four)
-            constexpr int TT = fx_lanes(N), Q = (N / 2 + 4 * TT - 1) / (4 * TT);
+            constexpr int TT = T, Q = (N / 2 + 4 * TT - 1) / (4 * TT);
             const bool oka = ya < a.rows, okb = ya + 1 < a.rows;
             const int yA = oka ? ya : 0, yB = okb ? ya + 1 : 0;
             uint32_t ka[Q], kb[Q];
@@ -270,7 +301,7 @@ __device__ __forceinline__ void xinv_body(const XArgs<Real> &a, const cplx<Real>
                 if (x < a.n_out) {
                     cplx<Real> v[4];
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] = line[L::slot(a.lp, x + e, lx)];
+                    for (int e = 0; e < 4; ++e) v[e] = line[fxslot<N>(x + e)];
                     auto row = [&](uint32_t k, int part) {
                         float o[4];
 #pragma unroll
@@ -287,11 +318,10 @@ __device__ __forceinline__ void xinv_body(const XArgs<Real> &a, const cplx<Real>
             return;
         }
     }
-    if constexpr (N > 0) {
+    {
         if (2 * a.n_out <= N && sink.masked()) {
             // at most E / 2 outputs per row and lane: every mask byte read
             // (clamped addresses) before the first store
-            constexpr int H = fx_elems(N) / 2;
             const bool oka = ya < a.rows, okb = ya + 1 < a.rows;
             const int yA = oka ? ya : 0, yB = okb ? ya + 1 : 0;
             uint8_t ka[H], kb[H];
@@ -306,7 +336,7 @@ __device__ __forceinline__ void xinv_body(const XArgs<Real> &a, const cplx<Real>
             for (int e = 0; e < H; ++e) {
                 const int x = t + e * T;
                 if (x < a.n_out) {
-                    const cplx<Real> v = line[L::slot(a.lp, x, lx)];
+                    const cplx<Real> v = line[fxslot<N>(x)];
                     if (oka) sink.put(c, z, ya, x, v.x * a.scale, ka[e]);
                     if (okb) sink.put(c, z, ya + 1, x, v.y * a.scale, kb[e]);
                 }
@@ -322,7 +352,7 @@ __device__ __forceinline__ void xinv_body(const XArgs<Real> &a, const cplx<Real>
             for (int x = 4 * t; x < a.n_out; x += 4 * T) {
                 cplx<Real> v[4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = line[L::slot(a.lp, x + e, lx)];
+                for (int e = 0; e < 4; ++e) v[e] = line[fxslot<N>(x + e)];
                 const int64_t i = ((int64_t)z * sink.ny + ya) * sink.nx + x;
                 if (ya < a.rows)
                     *reinterpret_cast<float4 *>(sink.out + (int64_t)c * sink.n + i) =
@@ -335,7 +365,7 @@ __device__ __forceinline__ void xinv_body(const XArgs<Real> &a, const cplx<Real>
         }
     }
     for (int x = t; x < a.n_out; x += T) {
-        const cplx<Real> v = line[L::slot(a.lp, x, lx)];
+        const cplx<Real> v = line[fxslot<N>(x)];
         if (ya < a.rows) sink(c, z, ya, x, v.x * a.scale);
         if (ya + 1 < a.rows) sink(c, z, ya + 1, x, v.y * a.scale);
     }
@@ -343,7 +373,8 @@ __device__ __forceinline__ void xinv_body(const XArgs<Real> &a, const cplx<Real>
 
 template <typename Real, class Sink, int N = 0>
 __global__ void __launch_bounds__(kMaxBlock) xinv_kernel(XArgs<Real> a, const cplx<Real> *spec, Sink sink) {
-    xinv_body<Real, Sink, N>(a, spec, sink, (int)blockIdx.z);
+    if constexpr (N > 0) xinv_body<Real, Sink, N>(a, spec, sink, (int)blockIdx.z);
+    else xinv_body_rt<Real, Sink>(a, spec, sink, (int)blockIdx.z);
 }
 
 template <typename Real, class Sink>
@@ -352,7 +383,7 @@ struct XInvPack {
     const cplx<Real> *spec;
     Sink sink;
 };
-template <typename Real, class Sink, int N = 0>
+template <typename Real, class Sink, int N>
 __global__ void __launch_bounds__(kMaxBlock) xinv_multi(const XInvPack<Real, Sink> *tab, int zdiv) {
     const XInvPack<Real, Sink> p = tab[blockIdx.z / zdiv];
     xinv_body<Real, Sink, N>(p.a, p.spec, p.sink, (int)(blockIdx.z % zdiv));
@@ -370,8 +401,9 @@ void launch_xfwd(Context &c, const XArgs<Real> &xa, const Src &src, cplx<Real> *
         with_line(xa.lp, [&](auto NC) {
             constexpr int N = decltype(NC)::value;
             const XFwdPack<Real, Src> pk{xa, src, spec};
-            launch_rec(c, N > 0 ? reinterpret_cast<const void *>(&xfwd_multi<Real, Src, N>) : nullptr, grid, block,
-                       lds, (int)comps, pk, [&] {
+            const void *multi = nullptr;
+            if constexpr (N > 0) multi = reinterpret_cast<const void *>(&xfwd_multi<Real, Src, N>);
+            launch_rec(c, multi, grid, block, lds, (int)comps, pk, [&] {
                            hipLaunchKernelGGL((xfwd_kernel<Real, Src, N>), grid, block, lds, c.stream, xa, src, spec);
                        });
         });
@@ -385,8 +417,9 @@ void launch_xinv(Context &c, const XArgs<Real> &xa, const cplx<Real> *spec, cons
     with_line(xa.lp, [&](auto NC) {
         constexpr int N = decltype(NC)::value;
         const XInvPack<Real, FieldSink<Real>> pk{xa, spec, sink};
-        launch_rec(c, N > 0 ? reinterpret_cast<const void *>(&xinv_multi<Real, FieldSink<Real>, N>) : nullptr, grid,
-                   block, lds, 3, pk, [&] {
+        const void *multi = nullptr;
+        if constexpr (N > 0) multi = reinterpret_cast<const void *>(&xinv_multi<Real, FieldSink<Real>, N>);
+        launch_rec(c, multi, grid, block, lds, 3, pk, [&] {
                        hipLaunchKernelGGL((xinv_kernel<Real, FieldSink<Real>, N>), grid, block, lds, c.stream, xa,
                                           spec, sink);
                    });

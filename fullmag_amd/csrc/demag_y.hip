@@ -35,18 +35,18 @@ __global__ void __launch_bounds__(kMaxBlock) line_kernel(LineArgs<Real> a) {
 // issued into registers before the current group's LDS transform, so memory
 // traffic overlaps the FFT; without it (one group per workgroup) the kernel
 // holds no prefetch registers and more waves share each SIMD instead.
-// Inputs: N / IN_DIV per line (RAGGED: a.n_in, fewer; the rest zero);
-// outputs: a.n_out per line.
-template <typename Real, int N, int IN_DIV, bool PIPE, bool RAGGED>
+// Forward: N / 2 inputs per line (RAGGED: a.n_in, fewer), the rest zero, and N
+// outputs; inverse: N inputs, a.n_out <= N / 2 outputs.
+template <typename Real, int N, bool INV, bool PIPE, bool RAGGED>
 __device__ __forceinline__ void line_pipe_body(const LineArgs<Real> &a) {
     constexpr int T = fx_lanes(N), E = fx_elems(N);
     constexpr int G = T >= 64 ? 1 : 64 / T;
-    constexpr int NI = E / IN_DIV;
-    static_assert(NI * IN_DIV == E, "whole loads per lane");
+    constexpr int NI = INV ? E : E / 2;
+    static_assert(E % 2 == 0, "whole loads per lane");
     extern __shared__ unsigned char smem_raw[];
     cplx<Real> *lds = reinterpret_cast<cplx<Real> *>(smem_raw);
     const int j = (int)threadIdx.x / T, t = (int)threadIdx.x - j * T;
-    cplx<Real> *line = lds + j * (N + kPad);
+    cplx<Real> *line = lds + j * fx_size(N);
     const int64_t first = (int64_t)blockIdx.x * (PIPE ? a.iters : 1) * G + j;
     cplx<Real> buf[NI];
     auto fetch = [&](int64_t l) {
@@ -78,33 +78,27 @@ __device__ __forceinline__ void line_pipe_body(const LineArgs<Real> &a) {
 #pragma unroll
         for (int e = 0; e < E; ++e) v[e] = e < NI ? buf[e] : cplx<Real>{Real(0), Real(0)};
         if (PIPE && it + 1 < iters) fetch(l + G);
-        fx_first_pass<Real, N>(line, t, v, a.tw, a.inverse != 0, 0);
-        fx_rest<Real, N>(line, t, a.tw, a.inverse != 0, 0);
-        if (l < a.lines) {
-            cplx<Real> *g = a.data + l * a.line_pitch;
-            if (sizeof(Real) == 4 && ((a.n_out | a.line_pitch) & 1) == 0) {
-                // two consecutive outputs per lane in one 16-byte store (an
-                // even line pitch keeps every line 16-byte aligned)
-                for (int e = 2 * t; e < a.n_out; e += 2 * T) {
-                    const cplx<Real> u = line[fxslot<N>(e)], v = line[fxslot<N>(e + 1)];
-                    *reinterpret_cast<float4 *>(g + e) = float4{float(u.x), float(u.y), float(v.x), float(v.y)};
-                }
-            } else {
-                for (int e = t; e < a.n_out; e += T) g[e] = line[fxslot<N>(e)];
-            }
-        }
+        fx_first_pass<Real, N>(line, t, v, a.tw, INV);
+        // the last pass stores from registers: consecutive lanes hold
+        // consecutive elements, and the inverse produces only the half of
+        // them that is kept
+        const bool live = l < a.lines;
+        cplx<Real> *g = a.data + (live ? l : 0) * a.line_pitch;
+        fx_rest_put<Real, N, INV ? 2 : 1>(line, t, a.tw, INV, [&](int i, const cplx<Real> &q) {
+            if (live && (!INV || i < a.n_out)) g[i] = q;
+        });
         if (PIPE) __syncthreads();
     }
 }
 
-template <typename Real, int N, int IN_DIV, bool PIPE, bool RAGGED = false>
+template <typename Real, int N, bool INV, bool PIPE, bool RAGGED>
 __global__ void __launch_bounds__(256) line_pipe_kernel(LineArgs<Real> a) {
-    line_pipe_body<Real, N, IN_DIV, PIPE, RAGGED>(a);
+    line_pipe_body<Real, N, INV, PIPE, RAGGED>(a);
 }
-template <typename Real, int N, int IN_DIV, bool PIPE, bool RAGGED = false>
+template <typename Real, int N, bool INV, bool PIPE, bool RAGGED>
 __global__ void __launch_bounds__(256) line_pipe_multi(const LineArgs<Real> *tab, int zdiv) {
     const LineArgs<Real> a = tab[blockIdx.z / zdiv];
-    line_pipe_body<Real, N, IN_DIV, PIPE, RAGGED>(a);
+    line_pipe_body<Real, N, INV, PIPE, RAGGED>(a);
 }
 
 // MAXB: kMaxBlock, or 1024 for lines too long for three of them in
@@ -164,7 +158,7 @@ __global__ void __launch_bounds__(MAXB) yconv_multi(const YConvArgs<Real> *tab, 
 template <typename Real, int N>
 __device__ __forceinline__ void yconv_fx_body(const YConvArgs<Real> &a) {
     using C = cplx<Real>;
-    constexpr int T = fx_lanes(N), E = fx_elems(N), NT = (E + 2) / 3, ls = N + kPad;
+    constexpr int T = fx_lanes(N), E = fx_elems(N), NT = (E + 2) / 3, ls = fx_size(N);
     extern __shared__ unsigned char smem_raw[];
     C *lds = reinterpret_cast<C *>(smem_raw);
     const int tid = threadIdx.x, nthr = blockDim.x;
@@ -183,7 +177,7 @@ __device__ __forceinline__ void yconv_fx_body(const YConvArgs<Real> &a) {
         }
 #pragma unroll
         for (int e = E / 2; e < E; ++e) v[e] = C{Real(0), Real(0)};
-        fx_first_pass<Real, N>(line, t, v, a.tw, false, 0);
+        fx_first_pass<Real, N>(line, t, v, a.tw, false);
     }
     // entry u: column j, ky = e of the workgroup's kpw N (kpw N / nthr = E / 3)
     Real k4[NT][4];
@@ -191,11 +185,11 @@ __device__ __forceinline__ void yconv_fx_body(const YConvArgs<Real> &a) {
     for (int u = 0; u < NT; ++u) {
         const int idx = tid + u * nthr, j = idx / N, e = idx % N, kx = kx0 + j;
         const bool ok = j < a.kpw && kx < a.hx;
-        const Real *K = a.K.k + ((int64_t)(ok ? kx : 0) * (N / 2 + 1) + (e <= N / 2 ? e : N - e)) * a.K.kb;
+        const Real *K = a.K.k + kern_at(a.K.l, 0, 0, ok ? kx : 0, e <= N / 2 ? e : N - e);
 #pragma unroll
         for (int q = 0; q < 4; ++q) k4[u][q] = K[q];
     }
-    fx_rest<Real, N>(line, t, a.tw, false, 0);
+    fx_rest<Real, N>(line, t, a.tw, false);
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < NT; ++u) {
@@ -208,9 +202,12 @@ __device__ __forceinline__ void yconv_fx_body(const YConvArgs<Real> &a) {
         }
     }
     __syncthreads();
-    fx_passes<Real, N, 0, 1>(line, t, a.tw, true, 0);
-    if (live)
-        for (int e = t; e < a.ny; e += T) g[e] = line[fxslot<N>(e)];
+    C v[E];
+    fx_load<Real, N>(line, t, v);
+    fx_first_pass<Real, N>(line, t, v, a.tw, true);
+    fx_rest_put<Real, N, 2>(line, t, a.tw, true, [&](int i, const C &q) {
+        if (live && i < a.ny) g[i] = q;
+    });
 }
 
 template <typename Real, int N>
@@ -253,33 +250,32 @@ void launch_lines(Context &c, const LinePlan &lp, LineArgs<Real> la) {
             // of the power-of-two lengths
             constexpr bool P2 = fx_odd(N) == 1;
             if (!P2 || dp.tune.y_pipe > 0) {
-                const bool half = la.n_in < N;  // a padded line: n_in <= N / 2
+                const bool inv = la.inverse != 0;
                 constexpr int T = fx_lanes(N), G = T >= 64 ? 1 : 64 / T;
-                la.iters = !P2 ? 1 : half && dp.tune.y_pipe_f > 0 ? dp.tune.y_pipe_f : dp.tune.y_pipe;
+                la.iters = !P2 ? 1 : !inv && dp.tune.y_pipe_f > 0 ? dp.tune.y_pipe_f : dp.tune.y_pipe;
                 const dim3 grid((unsigned)cdiv(la.lines, (int64_t)G * la.iters)), block((unsigned)(G * T));
-                const size_t lds = (size_t)G * (N + kPad) * ce;
-                auto launch = [&](auto divc, auto pipe, auto ragged) {
-                    constexpr int D = decltype(divc)::value;
-                    constexpr bool P = decltype(pipe)::value, G1 = decltype(ragged)::value;
-                    launch_rec(c, P ? nullptr : reinterpret_cast<const void *>(&line_pipe_multi<Real, N, D, false, G1>),
+                const size_t lds = (size_t)G * fx_size(N) * ce;
+                auto launch = [&](auto invc, auto pipe, auto ragged) {
+                    constexpr bool I = decltype(invc)::value, P = decltype(pipe)::value, G1 = decltype(ragged)::value;
+                    launch_rec(c, P ? nullptr : reinterpret_cast<const void *>(&line_pipe_multi<Real, N, I, false, G1>),
                                grid, block, lds, 1, la, [&] {
-                                   hipLaunchKernelGGL((line_pipe_kernel<Real, N, D, P, G1>), grid, block, lds,
+                                   hipLaunchKernelGGL((line_pipe_kernel<Real, N, I, P, G1>), grid, block, lds,
                                                       c.stream, la);
                                });
                 };
-                using One = std::integral_constant<int, 1>;
-                using Two = std::integral_constant<int, 2>;
+                const std::true_type yes;
+                const std::false_type no;
                 if constexpr (P2) {
                     if (la.iters > 1) {
-                        if (half && 2 * la.n_in == N) launch(Two{}, std::true_type{}, std::false_type{});
-                        else if (half) launch(Two{}, std::true_type{}, std::true_type{});
-                        else launch(One{}, std::true_type{}, std::false_type{});
+                        if (inv) launch(yes, yes, no);
+                        else if (2 * la.n_in == N) launch(no, yes, no);
+                        else launch(no, yes, yes);
                         return;
                     }
                 }
-                if (half && 2 * la.n_in == N) launch(Two{}, std::false_type{}, std::false_type{});
-                else if (half) launch(Two{}, std::false_type{}, std::true_type{});
-                else launch(One{}, std::false_type{}, std::false_type{});
+                if (inv) launch(yes, no, no);
+                else if (2 * la.n_in == N) launch(no, no, no);
+                else launch(no, no, yes);
                 return;
             }
         }
@@ -293,7 +289,7 @@ void launch_lines(Context &c, const LinePlan &lp, LineArgs<Real> la) {
 template <typename Real>
 void launch_yconv(Context &c, const YConvArgs<Real> &ya) {
     const dim3 grid((unsigned)cdiv(ya.hx, ya.kpw)), block((unsigned)(3 * ya.kpw * ya.lp.threads));
-    const size_t lds = (size_t)3 * ya.kpw * (ya.lp.n + kPad) * sizeof(cplx<Real>);
+    const size_t lds = (size_t)3 * ya.kpw * line_slots(ya.lp) * sizeof(cplx<Real>);
     with_line(ya.lp, [&](auto NC) {
         constexpr int N = decltype(NC)::value;
         if constexpr (N > 0) {

@@ -236,7 +236,7 @@ struct ZTensorRegs {
     __device__ __forceinline__ void load(const ZArgs<Real> &a, bool col_valid, int kx, int ky, int p) {
         valid = col_valid && a.K.k;
         const int oy = ky <= a.K.ny ? ky : a.py - ky;
-        blk = valid ? a.K.k + ((int64_t)kx * (a.K.ny + 1) + oy) * a.K.kb + (p ? a.K.kodd : 0) : a.K.k;
+        blk = valid ? a.K.k + kern_at(a.K.l, 0, p, kx, oy) : a.K.k;
         if constexpr (REGS) {
 #pragma unroll
             for (int e = 0; e < NV * 4; ++e) k[e] = Real(0);
@@ -428,12 +428,11 @@ __global__ void __launch_bounds__(256) zconv_quad_multi(const ZArgs<Real> *tab, 
 }
 
 
-template <typename Real, int N = 0>
+template <typename Real>
 __global__ void __launch_bounds__(kMaxBlock) zlds_kernel(ZLdsArgs<Real> a) {
-    using L = LineOps<N>;
     extern __shared__ unsigned char smem_raw[];
     cplx<Real> *lds = reinterpret_cast<cplx<Real> *>(smem_raw);
-    const int n = L::n(a.lp), ls = n + kPad, T = L::threads(a.lp);
+    const int n = a.lp.n, ls = n + kPad, T = a.lp.threads;
     const int tid = threadIdx.x, nthr = blockDim.x;
     const int ncomp = a.conv ? 3 : 1;
     const int cbase = a.conv ? 0 : blockIdx.y;
@@ -458,12 +457,12 @@ __global__ void __launch_bounds__(kMaxBlock) zlds_kernel(ZLdsArgs<Real> a) {
             const int idx = base + u * nthr;
             if (idx < nslots * n) {
                 const int s = idx % nslots, e = idx / nslots;
-                lds[s * ls + L::slot(a.lp, e)] = v[u];
+                lds[s * ls + lslot(a.lp, e)] = v[u];
             }
         }
     }
     __syncthreads();
-    L::template fft<Real>(lds + (tid / T) * ls, a.lp, tid % T, a.tw, !a.conv && a.inverse);
+    line_fft(lds + (tid / T) * ls, a.lp, tid % T, a.tw, !a.conv && a.inverse);
     __syncthreads();  // the tensor product and the stores cross lines
     if (a.conv) {
         // one pass per octant entry oz <= nz, applied at kz = oz and at its
@@ -481,7 +480,7 @@ __global__ void __launch_bounds__(kMaxBlock) zlds_kernel(ZLdsArgs<Real> a) {
                 if (ky >= a.py) continue;
                 Real t[6];
                 tensor_at(a.K, kx, ky, e, t);
-                const int se = L::slot(a.lp, e);
+                const int se = lslot(a.lp, e);
                 apply_tensor(t, lds[j * ls + se], lds[(a.tile + j) * ls + se], lds[(2 * a.tile + j) * ls + se]);
             }
         }
@@ -494,28 +493,251 @@ __global__ void __launch_bounds__(kMaxBlock) zlds_kernel(ZLdsArgs<Real> a) {
             const bool ylo = ky <= a.K.ny;
             const int oy = ylo ? ky : a.py - ky;
             const Real sy = ylo ? Real(1) : Real(-1);
-            const V2 *e = reinterpret_cast<const V2 *>(a.K.k +
-                                                       kern_at(a.K.kb, a.K.kodd, a.K.kcomp, a.K.ny + 1, 0, oz, kx, oy));
+            const V2 *e = reinterpret_cast<const V2 *>(a.K.k + kern_at(a.K.l, 0, oz, kx, oy));
             const V2 t01 = e[0], t23 = e[1], t45 = e[2];
             Real t[6] = {t01.x, t01.y, t23.x, sy * t23.y, t45.x, sy * t45.y};
-            int se = L::slot(a.lp, oz);
+            int se = lslot(a.lp, oz);
             apply_tensor(t, lds[j * ls + se], lds[(a.tile + j) * ls + se], lds[(2 * a.tile + j) * ls + se]);
             if (oz > 0 && oz < a.K.pz - oz) {
                 t[4] = -t[4];
                 t[5] = -t[5];
-                se = L::slot(a.lp, a.K.pz - oz);
+                se = lslot(a.lp, a.K.pz - oz);
                 apply_tensor(t, lds[j * ls + se], lds[(a.tile + j) * ls + se], lds[(2 * a.tile + j) * ls + se]);
             }
         }
         __syncthreads();
-        L::template fft<Real>(lds + (tid / T) * ls, a.lp, tid % T, a.tw, true);
+        line_fft(lds + (tid / T) * ls, a.lp, tid % T, a.tw, true);
         __syncthreads();
     }
     for (int idx = tid; idx < nslots * a.n_out; idx += nthr) {
         const int s = idx % nslots, e = idx / nslots;
         const int c = s / a.tile;
         const int64_t col = col0 + (s - c * a.tile);
-        if (col < a.columns) a.data[(cbase + c) * a.comp_stride + e * a.zstride + col] = lds[s * ls + L::slot(a.lp, e)];
+        if (col < a.columns) a.data[(cbase + c) * a.comp_stride + e * a.zstride + col] = lds[s * ls + lslot(a.lp, e)];
+    }
+}
+
+// Long z lines of a scheduled length N with at most 64 lanes, C = 64 / T
+// groups of V columns per wavefront.  Lane (t, g) = (lane / C, lane % C) holds
+// elements t + e T of the V columns of group g, so a load instruction covers
+// runs of C V consecutive columns (128 bytes for up to 128 z planes), and
+// what it loads are the first pass's inputs: no index is divided and nothing
+// is staged before the transform.  One wavefront per component, lines
+// interleaved in LDS as [slot][group] with the V columns in one 16-byte
+// access, so a pass needs no workgroup barrier and the twiddles serve V
+// columns.  CONV: each tensor entry oz is loaded (beside the columns, before
+// the transform) once per column and applied at kz = oz and pz - oz between
+// two barriers; the inverse transform's last pass stores straight to memory.
+// Bound by VALU work (about half of it butterflies) and by memory latency at
+// nine wavefronts per CU.  256x256x64 mixed (257x512 columns of 128, 507 MB):
+// 213 us with the staged lines of zlds_kernel, 131 us here, 147 us with one
+// column per lane (twice the wavefronts, but each pays its own twiddles and
+// 64-byte runs).  100^3 FP64: 214 -> 109 us.
+template <typename Real, int V>
+struct alignas(sizeof(cplx<Real>) * V) cvec {
+    cplx<Real> c[V];
+};
+
+// v[s][r] *= w^(r st) for the V columns s (see twiddle()).
+template <typename T, int R, int V>
+__device__ __forceinline__ void twiddle_cols(cplx<T> v[V][R], const cplx<T> *tw, int st, bool inv) {
+    constexpr int LB = R == 2 ? 1 : R == 4 ? 2 : R == 8 ? 3 : 4;
+    static_assert((1 << LB) == R, "power-of-two radix");
+    const T sg = inv ? T(-1) : T(1);
+    cplx<T> pw[LB], w[R];
+#pragma unroll
+    for (int b = 0; b < LB; ++b) {
+        pw[b] = tw[st << b];
+        pw[b].y *= sg;
+    }
+#pragma unroll
+    for (int r = 1; r < R; ++r) {
+        const int low = r & -r;
+        const int lb = low == 1 ? 0 : low == 2 ? 1 : low == 4 ? 2 : 3;
+        w[r] = r == low ? pw[lb] : cmul(w[r - low], pw[lb]);
+#pragma unroll
+        for (int s = 0; s < V; ++s) v[s][r] = cmul(v[s][r], w[r]);
+    }
+}
+
+// One pass (see fx_pass) over the lane's V columns; `put(i, q)` takes output
+// element i instead of LDS when LAST.
+template <typename T, int N, int R, int NS, int V, int C, bool LAST, class Put>
+__device__ __forceinline__ void col_pass(cvec<T, V> *l, int t, const cplx<T> *tw, bool inv, Put &&put) {
+    constexpr int G = fx_pad(N), NT = fx_lanes(N), NR = N / R, ST = N / (NS * R);
+    constexpr int MB = (NR + NT - 1) / NT;
+    constexpr bool FULL = MB * NT == NR;
+    cplx<T> v[MB][V][R];
+    int base[MB];
+#pragma unroll
+    for (int b = 0; b < MB; ++b) {
+        const int j0 = t + b * NT, j = FULL || j0 < NR ? j0 : 0, k = j % NS;
+        const cvec<T, V> *p = l + fxslot<N>(j) * C;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const cvec<T, V> q = p[r * (NR + NR / G) * C];
+#pragma unroll
+            for (int s = 0; s < V; ++s) v[b][s][r] = q.c[s];
+        }
+        twiddle_cols<T, R, V>(v[b], tw, k * ST, inv);
+#pragma unroll
+        for (int s = 0; s < V; ++s) dft_any<T, R>(v[b][s], tw, N, inv);
+        base[b] = (j / NS) * NS * R + k;
+    }
+    if constexpr (!LAST) pass_sync<N>();
+#pragma unroll
+    for (int b = 0; b < MB; ++b)
+        if (FULL || t + b * NT < NR)
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                cvec<T, V> q;
+#pragma unroll
+                for (int s = 0; s < V; ++s) q.c[s] = v[b][s][r];
+                if constexpr (LAST) put(base[b] + r * NS, q);
+                else l[(fxslot<N>(base[b]) + r * (NS + NS / G)) * C] = q;
+            }
+    if constexpr (!LAST) pass_sync<N>();
+}
+
+// The first pass, from registers (see fx_first_pass).
+template <typename T, int N, int V, int C>
+__device__ __forceinline__ void col_first(cvec<T, V> *l, int t, const cplx<T> (*v)[fx_elems(N)], const cplx<T> *tw,
+                                          bool inv) {
+    constexpr int R = fx_radix(N, 0), B = fx_elems(N) / R, NT = fx_lanes(N);
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+        cplx<T> u[V][R];
+#pragma unroll
+        for (int s = 0; s < V; ++s) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) u[s][r] = v[s][b + r * B];
+            dft_any<T, R>(u[s], tw, N, inv);
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            cvec<T, V> q;
+#pragma unroll
+            for (int s = 0; s < V; ++s) q.c[s] = u[s][r];
+            l[((t + b * NT) * (R + 1) + r) * C] = q;
+        }
+    }
+    pass_sync<N>();
+}
+
+// Passes P.. of the schedule, the last through `put` when STORE.
+template <typename T, int N, int P, int NS, int V, int C, bool STORE, class Put>
+__device__ __forceinline__ void col_passes(cvec<T, V> *l, int t, const cplx<T> *tw, bool inv, Put &&put) {
+    if constexpr (P < fx_npass(N)) {
+        constexpr int R = fx_radix(N, P);
+        col_pass<T, N, R, NS, V, C, STORE && P + 1 == fx_npass(N)>(l, t, tw, inv, put);
+        col_passes<T, N, P + 1, NS * R, V, C, STORE>(l, t, tw, inv, put);
+    }
+}
+
+template <int N>
+constexpr bool zcol_has() {
+    return N > 16 && fx_lanes(N) <= 64 && fx_npass(N) > 1;
+}
+// columns per lane: as many as fill a 16-byte access
+template <typename Real>
+constexpr int zcol_v() {
+    return sizeof(Real) == 4 ? 2 : 1;
+}
+
+template <typename Real, int N, int V, bool CONV>
+__global__ void __launch_bounds__(CONV ? 192 : 64) zcol_kernel(ZLdsArgs<Real> a) {
+    using Cx = cplx<Real>;
+    using Cv = cvec<Real, V>;
+    constexpr int T = fx_lanes(N), E = fx_elems(N), C = 64 / T, NZO = N / 2 + 1;
+    __shared__ Cv lds[CONV ? 3 : 1][fx_size(N) * C];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int g = lane % C, t = lane / C;
+    const int comp = CONV ? w : (int)blockIdx.y;
+    const uint32_t blk = a.xcd ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
+    const int64_t col = ((int64_t)blk * C + g) * V;  // columns is even: a group is all in or all out
+    const bool live = col < a.columns;
+    Cx *data = a.data + comp * a.comp_stride + (live ? col : 0);
+    Cv *l = lds[CONV ? w : 0] + g;
+    const auto none = [](int, const Cv &) {};
+    const auto store = [&](int i, const Cv &q) {
+        if (live && i < a.n_out) *reinterpret_cast<Cv *>(data + i * a.zstride) = q;
+    };
+    {
+        Cx v[V][E];
+        const bool half = 2 * a.n_in <= N;
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const int i = t + e * T;
+            Cv q{};
+            if (e < E / 2 || !half) {
+                q = *reinterpret_cast<const Cv *>(data + (i < a.n_in ? i : 0) * a.zstride);
+                if (i >= a.n_in) q = Cv{};
+            }
+#pragma unroll
+            for (int s = 0; s < V; ++s) v[s][e] = q.c[s];
+        }
+        col_first<Real, N, V, C>(l, t, v, a.tw, !CONV && a.inverse);
+    }
+    if constexpr (!CONV) {
+        col_passes<Real, N, 1, fx_radix(N, 0), V, C, true>(l, t, a.tw, a.inverse != 0, store);
+    } else {
+        // item tid + 192 u: entry oz = item / C of column group item % C
+        constexpr int NU = (C * NZO + 191) / 192;
+        constexpr int H = 3;  // 2-vectors per entry
+        using V2 = typename std::conditional<sizeof(Real) == 4, float2, double2>::type;
+        V2 k[NU][V][H];
+#pragma unroll
+        for (int u = 0; u < NU; ++u) {
+            const int item = tid + 192 * u, oz = item < C * NZO ? item / C : 0;
+            const int64_t cc = ((int64_t)blk * C + item % C) * V;
+            const int64_t c0 = cc < a.columns ? cc : 0;
+            const int kx = (int)((uint32_t)c0 / (uint32_t)a.pitch), ky = (int)((uint32_t)c0 % (uint32_t)a.pitch);
+#pragma unroll
+            for (int s = 0; s < V; ++s) {
+                const int oy = ky + s <= a.K.ny ? ky + s : a.py - ky - s;
+                const V2 *p = reinterpret_cast<const V2 *>(a.K.k + kern_at(a.K.l, 0, oz, kx, oy));
+#pragma unroll
+                for (int q = 0; q < H; ++q) k[u][s][q] = p[q];
+            }
+        }
+        col_passes<Real, N, 1, fx_radix(N, 0), V, C, false>(l, t, a.tw, false, none);
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < NU; ++u) {
+            const int item = tid + 192 * u;
+            if (item < C * NZO) {
+                const int oz = item / C, gi = item % C;
+                const int64_t cc = ((int64_t)blk * C + gi) * V;
+                const int ky = (int)((uint32_t)cc % (uint32_t)a.pitch);
+                auto apply = [&](int kz, Real sz) {
+                    const int at = fxslot<N>(kz) * C + gi;
+                    Cv x = lds[0][at], y = lds[1][at], z = lds[2][at];
+#pragma unroll
+                    for (int s = 0; s < V; ++s) {
+                        const Real sy = ky + s <= a.K.ny ? Real(1) : Real(-1);
+                        const Real tt[6] = {k[u][s][0].x,      k[u][s][0].y,      k[u][s][1].x,
+                                            sy * k[u][s][1].y, sz * k[u][s][2].x, sy * sz * k[u][s][2].y};
+                        apply_tensor(tt, x.c[s], y.c[s], z.c[s]);
+                    }
+                    lds[0][at] = x;
+                    lds[1][at] = y;
+                    lds[2][at] = z;
+                };
+                apply(oz, Real(1));
+                if (oz > 0 && oz < N - oz) apply(N - oz, Real(-1));
+            }
+        }
+        __syncthreads();
+        Cx v[V][E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const Cv q = l[fxslot<N>(t + e * T) * C];
+#pragma unroll
+            for (int s = 0; s < V; ++s) v[s][e] = q.c[s];
+        }
+        pass_sync<N>();
+        col_first<Real, N, V, C>(l, t, v, a.tw, true);
+        col_passes<Real, N, 1, fx_radix(N, 0), V, C, true>(l, t, a.tw, true, store);
     }
 }
 
@@ -571,13 +793,23 @@ void launch_zreg(Context &c, const ZArgs<Real> &za) {
 
 template <typename Real>
 void launch_zlds(Context &c, const ZLdsArgs<Real> &za, unsigned comps) {
-    const int slots = (za.conv ? 3 : 1) * za.tile;
-    const dim3 grid((unsigned)cdiv(za.columns, za.tile), comps), block((unsigned)(slots * za.lp.threads));
-    const size_t lds = (size_t)slots * (za.lp.n + kPad) * sizeof(cplx<Real>);
     with_line(za.lp, [&](auto NC) {
-        launch_rec(c, nullptr, grid, block, lds, 1, za, [&] {
-            hipLaunchKernelGGL((zlds_kernel<Real, decltype(NC)::value>), grid, block, lds, c.stream, za);
-        });
+        constexpr int N = decltype(NC)::value;
+        if constexpr (zcol_has<N>()) {
+            constexpr int V = zcol_v<Real>(), C = 64 / fx_lanes(N);
+            const dim3 g((unsigned)cdiv(za.columns, C * V), comps);
+            launch_rec(c, nullptr, g, dim3(za.conv ? 192 : 64), 0, 1, za, [&] {
+                if (za.conv) hipLaunchKernelGGL((zcol_kernel<Real, N, V, true>), g, dim3(192), 0, c.stream, za);
+                else hipLaunchKernelGGL((zcol_kernel<Real, N, V, false>), g, dim3(64), 0, c.stream, za);
+            });
+        } else {
+            const int slots = (za.conv ? 3 : 1) * za.tile;
+            const dim3 grid((unsigned)cdiv(za.columns, za.tile), comps), block((unsigned)(slots * za.lp.threads));
+            const size_t lds = (size_t)slots * (za.lp.n + kPad) * sizeof(cplx<Real>);
+            launch_rec(c, nullptr, grid, block, lds, 1, za, [&] {
+                hipLaunchKernelGGL((zlds_kernel<Real>), grid, block, lds, c.stream, za);
+            });
+        }
     });
 }
 
