@@ -193,6 +193,7 @@ struct Context {
     double *h_result = nullptr;  // pinned: the merged stats of the last stats pass
     double *h_partials = nullptr;  // pinned, coherent: workgroup partials of the stats / error passes
     unsigned stats_blocks = 0;     // workgroups of the last stats pass
+    unsigned stats_stride = 0;     // doubles each of them left
 
     // adjoint work buffers (allocated by the first adjoint call)
     bool adj_ready = false;

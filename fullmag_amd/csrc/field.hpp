@@ -15,6 +15,7 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr int kNStat = 9;  // s_ex, c_ex, s_d, c_d, s_ext, c_ext, max|Heff|^2, max|Hd|^2, max|k|^2
+constexpr int kNErr = kNStat + 1;  // the same and the largest squared error (error passes)
 // Read in place of an absent per-cell Ms, so that the read needs no branch.
 __device__ const double kUnitStandIn = 1.0;
 
@@ -308,6 +309,11 @@ __device__ __forceinline__ void neu_add(double &s, double &c, double v) {
     s = t;
 }
 
+// STAGE_STATS accumulates the step diagnostics; STAGE_ERROR, which evaluates
+// the last slope at the candidate state, the adaptive error norm and the same
+// diagnostics, which are the step's if it is accepted (a stats pass of its own
+// would read the state and the demag field again: 50 us of a 2.5 ms DP45 step
+// at 256x256x64).
 enum { STAGE_PLAIN = 0, STAGE_STATS = 1, STAGE_ERROR = 2 };
 
 // Combines two compensated partial sums (s, c) += (s2, c2).
@@ -320,20 +326,16 @@ __device__ __forceinline__ void neu_merge(double &s, double &c, double s2, doubl
 // wavefront partials through LDS; lane 0 writes the result to `out`.
 template <int MODE>
 __device__ __forceinline__ void block_reduce(double *acc, double *out) {
-    constexpr int NQ = MODE == STAGE_STATS ? kNStat : 1;
+    constexpr int NQ = MODE == STAGE_STATS ? kNStat : kNErr;
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
-        if (MODE == STAGE_STATS) {
 #pragma unroll
-            for (int e = 0; e < 3; ++e) {
-                const double s2 = __shfl_down(acc[2 * e], off), c2 = __shfl_down(acc[2 * e + 1], off);
-                neu_merge(acc[2 * e], acc[2 * e + 1], s2, c2);
-            }
-#pragma unroll
-            for (int q = 6; q < 9; ++q) acc[q] = fmax(acc[q], __shfl_down(acc[q], off));
-        } else {
-            acc[0] = fmax(acc[0], __shfl_down(acc[0], off));
+        for (int e = 0; e < 3; ++e) {
+            const double s2 = __shfl_down(acc[2 * e], off), c2 = __shfl_down(acc[2 * e + 1], off);
+            neu_merge(acc[2 * e], acc[2 * e + 1], s2, c2);
         }
+#pragma unroll
+        for (int q = 6; q < NQ; ++q) acc[q] = fmax(acc[q], __shfl_down(acc[q], off));
     }
     __shared__ double red[kBlock / 64][NQ];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -342,12 +344,8 @@ __device__ __forceinline__ void block_reduce(double *acc, double *out) {
     __syncthreads();
     if (threadIdx.x == 0) {
         for (int w = 1; w < (int)(blockDim.x >> 6); ++w) {
-            if (MODE == STAGE_STATS) {
-                for (int e = 0; e < 3; ++e) neu_merge(red[0][2 * e], red[0][2 * e + 1], red[w][2 * e], red[w][2 * e + 1]);
-                for (int q = 6; q < 9; ++q) red[0][q] = fmax(red[0][q], red[w][q]);
-            } else {
-                red[0][0] = fmax(red[0][0], red[w][0]);
-            }
+            for (int e = 0; e < 3; ++e) neu_merge(red[0][2 * e], red[0][2 * e + 1], red[w][2 * e], red[w][2 * e + 1]);
+            for (int q = 6; q < NQ; ++q) red[0][q] = fmax(red[0][q], red[w][q]);
         }
         for (int q = 0; q < NQ; ++q) out[q] = red[0][q];
     }
@@ -423,7 +421,7 @@ __device__ __forceinline__ void stage_cell(const StageArgs<State, Real, Src, Out
 #pragma unroll
         for (int c = 0; c < 3; ++c) a.out[c * n + i] = Out(v[c] * inv);
     }
-    if (MODE == STAGE_STATS && act) {
+    if (MODE != STAGE_PLAIN && act) {
         // m . H per term in FP64 with the state's own m
         double md[3];
 #pragma unroll
@@ -485,7 +483,7 @@ __device__ __forceinline__ void stage_cell(const StageArgs<State, Real, Src, Out
             for (int j = 0; j < a.nprev; ++j) s += a.ap[j] * double(a.kp[j][c * n + i]);
             e[c] = s * a.dt;
         }
-        acc[0] = fmax(acc[0], e[0] * e[0] + e[1] * e[1] + e[2] * e[2]);
+        acc[kNStat] = fmax(acc[kNStat], e[0] * e[0] + e[1] * e[1] + e[2] * e[2]);
     }
 }
 
@@ -498,9 +496,9 @@ template <typename State, typename Real, typename Src, typename Out, int MODE, b
 __global__ void __launch_bounds__(kBlock) stage_kernel(StageArgs<State, Real, Src, Out> a) {
     const FieldArgs &f = a.f;
     const int64_t n = f.n;
-    double acc[kNStat];
+    double acc[kNErr];
 #pragma unroll
-    for (int q = 0; q < kNStat; ++q) acc[q] = 0.0;
+    for (int q = 0; q < kNErr; ++q) acc[q] = 0.0;
     const uint32_t tile = f.xcd ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
     const int chunk = (int)(tile % (uint32_t)f.nchunks);
     const uint32_t t2 = tile / (uint32_t)f.nchunks;
@@ -529,18 +527,19 @@ __global__ void __launch_bounds__(kBlock) stage_kernel(StageArgs<State, Real, Sr
         }
     }
     if (MODE == STAGE_PLAIN) return;
-    block_reduce<MODE>(acc, a.partials + (int64_t)blockIdx.x * (MODE == STAGE_STATS ? kNStat : 1));
+    block_reduce<MODE>(acc, a.partials + (int64_t)blockIdx.x * (MODE == STAGE_STATS ? kNStat : kNErr));
 }
 
 // Uniform-material form of stage_kernel: no region table, no per-cell Ms,
-// no boundary tier, demag and exchange on, at most one earlier slope (the
-// Heun stages and the stats pass; RK4 / RK23 / DP45 / ABM3 stages with more
-// slopes use stage_kernel).  The per-cell arithmetic is stage_cell's, in the
+// demag and exchange on, at most five earlier slopes (every stage of the
+// integrators and the error pass; with a boundary tier at most one, the Heun
+// stages).  The per-cell arithmetic is stage_cell's, in the
 // same order, so results are bit-identical; what changes is that every load
 // of a plane (the z neighbour ahead, the four x/y neighbours, H_d, the base
 // point, the earlier slope, and with MASK their mask bytes) is issued in one
 // branch-free batch before any arithmetic, where stage_kernel's
-// optional-input branches split a plane's loads into several serial waits.
+// optional-input branches split a plane's loads into several serial waits
+// (256x256x64 mixed DP45, three slopes, 450 MB: 151 us as stage_kernel, 112 us here; five slopes 174 -> 120 us).
 // M0_IS_SRC: the base point is src itself (predictor stages and the stats
 // pass), so it is not loaded again.  MASK: an active mask is present; an
 // inactive neighbour enters as the centre value (exchange_col) and an
@@ -553,13 +552,14 @@ __global__ void __launch_bounds__(kBlock) stage_kernel(StageArgs<State, Real, Sr
 template <typename State, typename Real, typename Src, typename Out, int MODE, int NPREV, bool M0_IS_SRC,
           bool HAS_OUT, bool MASK = false, bool TIER = false>
 __device__ __forceinline__ void stage_uniform_body(const StageArgs<State, Real, Src, Out> &a) {
-    static_assert(MODE != STAGE_ERROR && NPREV <= 1, "plain and stats stages with at most one earlier slope");
+    static_assert(NPREV <= 5 && (!TIER || (NPREV <= 1 && MODE != STAGE_ERROR)), "slopes of the launched forms");
+    static_assert(MODE != STAGE_ERROR || !HAS_OUT, "the error pass stores no stage point");
     static_assert(!M0_IS_SRC || sizeof(Src) == sizeof(State), "a base point read from src is a state");
     const FieldArgs &f = a.f;
     const int64_t n = f.n;
-    double acc[kNStat];
+    double acc[kNErr];
 #pragma unroll
-    for (int q = 0; q < kNStat; ++q) acc[q] = 0.0;
+    for (int q = 0; q < kNErr; ++q) acc[q] = 0.0;
     const uint32_t tile = f.xcd ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
     const int chunk = (int)(tile % (uint32_t)f.nchunks);
     const uint32_t t2 = tile / (uint32_t)f.nchunks;
@@ -576,7 +576,10 @@ __device__ __forceinline__ void stage_uniform_body(const StageArgs<State, Real, 
         const Src *__restrict__ src = a.src;
         const Real *__restrict__ hd = a.hd;
         const State *__restrict__ m0p = a.m0;
-        const Real *__restrict__ kp = a.kp[0];
+        constexpr int NK = NPREV > 0 ? NPREV : 1;
+        const Real *__restrict__ kp[NK];
+#pragma unroll
+        for (int j = 0; j < NK; ++j) kp[j] = a.kp[j];
         int64_t i = ((int64_t)z0 * f.ny + y) * f.nx + x;
         Src prev[3], cur[3];
         const int64_t ib = z0 > 0 ? i - nxy : i;
@@ -598,7 +601,7 @@ __device__ __forceinline__ void stage_uniform_body(const StageArgs<State, Real, 
         for (int z = z0; z < z1; ++z, i += nxy) {
             const int64_t ia = z + 1 < f.nz ? i + nxy : i;
             Src nxt[3], xm[3], xp[3], ym[3], yp[3];
-            Real hdv[3], kpv[3];
+            Real hdv[3], kpv[NK][3];
             State m0v[3];
             uint8_t knxt = 1, kxm = 1, kxp = 1, kym = 1, kyp = 1;
             if constexpr (MASK) {
@@ -618,7 +621,8 @@ __device__ __forceinline__ void stage_uniform_body(const StageArgs<State, Real, 
                 yp[c] = sc[i + oyp];
                 hdv[c] = hd[c * n + i];
                 if (HAS_OUT && !M0_IS_SRC) m0v[c] = m0p[c * n + i];
-                if (HAS_OUT && NPREV == 1) kpv[c] = kp[c * n + i];
+#pragma unroll
+                for (int j = 0; j < NPREV; ++j) kpv[j][c] = kp[j][c * n + i];
             }
             double wt[6], phi0 = 0.0, msc = 1.0;
             if constexpr (TIER) {
@@ -678,7 +682,8 @@ __device__ __forceinline__ void stage_uniform_body(const StageArgs<State, Real, 
 #pragma unroll
                 for (int c = 0; c < 3; ++c) {
                     State s = State(a.anew) * State(k[c]);
-                    if constexpr (NPREV == 1) s += State(a.ap[0]) * State(kpv[c]);
+#pragma unroll
+                    for (int j = 0; j < NPREV; ++j) s += State(a.ap[j]) * State(kpv[j][c]);
                     const State base = M0_IS_SRC ? State(cur[c]) : m0v[c];
                     v[c] = base + State(a.dt) * s;
                 }
@@ -687,7 +692,7 @@ __device__ __forceinline__ void stage_uniform_body(const StageArgs<State, Real, 
 #pragma unroll
                 for (int c = 0; c < 3; ++c) a.out[c * n + i] = Out(v[c] * inv);
             }
-            if (MODE == STAGE_STATS && act) {
+            if (MODE != STAGE_PLAIN && act) {
                 double md[3];
 #pragma unroll
                 for (int c = 0; c < 3; ++c) md[c] = double(cur[c]);
@@ -722,6 +727,18 @@ __device__ __forceinline__ void stage_uniform_body(const StageArgs<State, Real, 
                 acc[7] = fmax(acc[7], d2);
                 acc[8] = fmax(acc[8], k2);
             }
+            if constexpr (MODE == STAGE_ERROR) {
+                // lib.rs:1653-1674: |dt sum_j E_j k_j| in FP64
+                double e[3];
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    double s = a.anew * double(k[c]);
+#pragma unroll
+                    for (int j = 0; j < NPREV; ++j) s += a.ap[j] * double(kpv[j][c]);
+                    e[c] = s * a.dt;
+                }
+                acc[kNStat] = fmax(acc[kNStat], e[0] * e[0] + e[1] * e[1] + e[2] * e[2]);
+            }
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
                 prev[c] = cur[c];
@@ -732,7 +749,7 @@ __device__ __forceinline__ void stage_uniform_body(const StageArgs<State, Real, 
         }
     }
     if constexpr (MODE == STAGE_PLAIN) return;
-    block_reduce<MODE>(acc, a.partials + (int64_t)blockIdx.x * kNStat);
+    block_reduce<MODE>(acc, a.partials + (int64_t)blockIdx.x * (MODE == STAGE_STATS ? kNStat : kNErr));
 }
 
 template <typename State, typename Real, typename Src, typename Out, int MODE, int NPREV, bool M0_IS_SRC,
@@ -752,7 +769,7 @@ __global__ void __launch_bounds__(kBlock) stage_uniform_multi(const StageArgs<St
 // (with MASK = f.mask != nullptr and TIER = f.tier_ex != 0; per-cell Ms only
 // with a tier).
 inline bool stage_uniform_ok(const FieldArgs &f, const void *hd, int nprev) {
-    return !f.region && (f.tier_ex || !f.ms_cell) && hd && f.exchange && nprev <= 1;
+    return !f.region && (f.tier_ex || !f.ms_cell) && hd && f.exchange && nprev <= (f.tier_ex ? 1 : 5);
 }
 
 // Column tiling of the stage kernels: tile width TX = 64 (or the smallest

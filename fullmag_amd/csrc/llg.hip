@@ -163,6 +163,19 @@ struct Driver {
         return a;
     }
 
+    // f(std::integral_constant<int, nprev>), nprev <= 5
+    template <class F>
+    static void by_slopes(int nprev, F &&f) {
+        switch (nprev) {
+            case 0: f(std::integral_constant<int, 0>{}); break;
+            case 1: f(std::integral_constant<int, 1>{}); break;
+            case 2: f(std::integral_constant<int, 2>{}); break;
+            case 3: f(std::integral_constant<int, 3>{}); break;
+            case 4: f(std::integral_constant<int, 4>{}); break;
+            default: f(std::integral_constant<int, 5>{}); break;
+        }
+    }
+
     template <typename Src, typename Out>
     void stage(const Src *src, Real *kout, Out *out, std::initializer_list<std::pair<int, double>> prev, double anew,
                double dt) {
@@ -178,33 +191,42 @@ struct Driver {
         a.dt = dt;
         Timed t(c, "llg_stage");
         const dim3 g(grid_stage()), b(kBlock);
-        // the uniform kernel (or its multi-instance twin while a batch records)
+        // the uniform kernel (or its multi-instance twin while a batch, which
+        // steps Heun, records)
         auto uniform_m = [&](auto np, auto m0src, auto masked, auto tier) {
             constexpr int NP = decltype(np)::value;
             constexpr bool MS = decltype(m0src)::value, MK = decltype(masked)::value, TR = decltype(tier)::value;
-            launch_rec(c,
-                       reinterpret_cast<const void *>(
-                           &stage_uniform_multi<State, Real, Src, Out, STAGE_PLAIN, NP, MS, true, MK, TR>),
-                       g, b, 0, 1, a, [&] {
-                           hipLaunchKernelGGL((stage_uniform_kernel<State, Real, Src, Out, STAGE_PLAIN, NP, MS, true, MK, TR>),
-                                              g, b, 0, c.stream, a);
-                       });
+            const void *multi = nullptr;
+            if constexpr (NP <= 1)
+                multi = reinterpret_cast<const void *>(
+                    &stage_uniform_multi<State, Real, Src, Out, STAGE_PLAIN, NP, MS, true, MK, TR>);
+            launch_rec(c, multi, g, b, 0, 1, a, [&] {
+                hipLaunchKernelGGL((stage_uniform_kernel<State, Real, Src, Out, STAGE_PLAIN, NP, MS, true, MK, TR>), g,
+                                   b, 0, c.stream, a);
+            });
         };
         auto uniform = [&](auto np, auto m0src) {
-            if (a.f.tier_ex) {
-                if (a.f.mask) uniform_m(np, m0src, std::true_type{}, std::true_type{});
-                else uniform_m(np, m0src, std::false_type{}, std::true_type{});
-            } else {
-                if (a.f.mask) uniform_m(np, m0src, std::true_type{}, std::false_type{});
-                else uniform_m(np, m0src, std::false_type{}, std::false_type{});
+            if constexpr (decltype(np)::value <= 1) {
+                if (a.f.tier_ex) {
+                    if (a.f.mask) uniform_m(np, m0src, std::true_type{}, std::true_type{});
+                    else uniform_m(np, m0src, std::false_type{}, std::true_type{});
+                    return;
+                }
             }
+            if (a.f.mask) uniform_m(np, m0src, std::true_type{}, std::false_type{});
+            else uniform_m(np, m0src, std::false_type{}, std::false_type{});
         };
         if (out && stage_uniform_ok(a.f, a.hd, a.nprev)) {
             constexpr bool src_is_state = sizeof(Src) == sizeof(State);
             const bool m0_is_src = src_is_state && static_cast<const void *>(src) == static_cast<const void *>(a.m0);
-            if (a.nprev == 1) uniform(std::integral_constant<int, 1>{}, std::false_type{});
-            else if (m0_is_src) uniform(std::integral_constant<int, 0>{}, std::integral_constant<bool, src_is_state>{});
-            else uniform(std::integral_constant<int, 0>{}, std::false_type{});
+            by_slopes(a.nprev, [&](auto np) {
+                if constexpr (decltype(np)::value == 0) {
+                    if (m0_is_src) uniform(np, std::integral_constant<bool, src_is_state>{});
+                    else uniform(np, std::false_type{});
+                } else {
+                    uniform(np, std::false_type{});
+                }
+            });
             return;
         }
         launch_rec(c, nullptr, g, b, 0, 1, a, [&] {
@@ -245,7 +267,21 @@ struct Driver {
         const unsigned g = grid_reduce();
         {
             Timed t(c, "llg_error");
-            if (a.f.tier_ex)
+            if (stage_uniform_ok(a.f, a.hd, a.nprev) && !a.f.tier_ex)
+                by_slopes(a.nprev, [&](auto np) {
+                    constexpr int NP = decltype(np)::value;
+                    if constexpr (NP >= 3) {  // RK23 and DP45
+                        if (a.f.mask)
+                            hipLaunchKernelGGL((stage_uniform_kernel<State, Real, State, Real, STAGE_ERROR, NP, false,
+                                                                     false, true>),
+                                               dim3(g), dim3(kBlock), 0, c.stream, a);
+                        else
+                            hipLaunchKernelGGL((stage_uniform_kernel<State, Real, State, Real, STAGE_ERROR, NP, false,
+                                                                     false, false>),
+                                               dim3(g), dim3(kBlock), 0, c.stream, a);
+                    }
+                });
+            else if (a.f.tier_ex)
                 hipLaunchKernelGGL((stage_kernel<State, Real, State, Real, STAGE_ERROR, true>), dim3(g), dim3(kBlock),
                                    0, c.stream, a);
             else
@@ -255,7 +291,9 @@ struct Driver {
         hipStreamSynchronize(c.stream);
         timing_resolve(c);
         double e = 0.0;
-        for (unsigned b = 0; b < g; ++b) e = std::fmax(e, c.h_partials[b]);
+        for (unsigned b = 0; b < g; ++b) e = std::fmax(e, c.h_partials[(size_t)b * kNErr + kNStat]);
+        c.stats_blocks = g;  // the diagnostics at src
+        c.stats_stride = kNErr;
         return std::sqrt(e);
     }
 
@@ -311,6 +349,7 @@ struct Driver {
             }
         }
         c.stats_blocks = g;
+        c.stats_stride = kNStat;
     }
 
     // The stats pass's workgroups store their partials (compensated energy
@@ -322,7 +361,7 @@ struct Driver {
         double acc[kNStat];
         for (int q = 0; q < kNStat; ++q) acc[q] = 0.0;
         const double *p = c.h_partials;
-        for (unsigned b = 0; b < c.stats_blocks; ++b, p += kNStat) {
+        for (unsigned b = 0; b < c.stats_blocks; ++b, p += c.stats_stride) {
             for (int e = 0; e < 3; ++e) {
                 double &sum = acc[2 * e], &comp = acc[2 * e + 1];
                 const double v = p[2 * e], t = sum + v;
@@ -354,8 +393,10 @@ struct Driver {
     }
 
     // Stats at the new state.  For Heun the same pass stores the next step's
-    // first slope and predictor for a step of the same dt.
+    // first slope and predictor for a step of the same dt; the adaptive
+    // methods' error pass of the accepted step has left them.
     void heun_aware_stats(double dt) {
+        if (c.integrator == FULLMAG_FDM_INTEGRATOR_RK23 || c.integrator == FULLMAG_FDM_INTEGRATOR_DP45) return;
         if (c.integrator == FULLMAG_FDM_INTEGRATOR_HEUN) {
             stats(k(0), mt(0), dt);
             c.pre_valid = true;
@@ -633,7 +674,7 @@ bool alloc_integrator_buffers(Context &c) {
         return false;
     if (!ctx_alloc(c, (void **)&c.d_result, 16 * sizeof(double), "result")) return false;
     // coherent: the stats and error passes store their workgroup partials here
-    if (!hip_ok(hipHostMalloc((void **)&c.h_partials, (size_t)c.max_partial_blocks * kNStat * sizeof(double),
+    if (!hip_ok(hipHostMalloc((void **)&c.h_partials, (size_t)c.max_partial_blocks * kNErr * sizeof(double),
                               hipHostMallocCoherent),
                 "hipHostMalloc(partials)", c.last_error))
         return false;
