@@ -341,7 +341,6 @@ int fullmag_fdm_ext_autotune(fullmag_fdm_backend *handle, int reps, char *chosen
                                {"fixed", &T::fixed, {1, 0}, true},
                                {"y_pipe", &T::y_pipe, {1, 0, 2, 4, 8}, false},
                                {"y_pipe_f", &T::y_pipe_f, {1, 2, 4, 8}, false},
-                               {"z_quad", &T::z_quad, {0, 1}, false},
                                {"xcd", &T::xcd, {1, 0}, false},
                                {"zc", &T::zc, {0, 1, 2, 4}, false}};
     if (c.demag && c.dp.three_d && c.dp.pz > 16) knobs.push_back({"z_tile", &T::z_tile, {0, 16, 8, 4, 2}, true});

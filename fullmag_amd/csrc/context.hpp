@@ -29,14 +29,13 @@ enum Mode { MODE_SINGLE = 1, MODE_DOUBLE = 2, MODE_MIXED = 3 };
 // Launch-schedule knobs of the demag transforms (0 = automatic).  Settable
 // per backend from the FULLMAG_FDM_TUNE environment variable as a comma list
 // of key=value (x_radix, x_lanes, x_rows, y_radix, y_lanes, y_lpw, fixed,
-// z_quad, xcd, y_pipe, y_pipe_f, z_tile, zc, y_split, pad).  x_radix, x_lanes,
+// xcd, y_pipe, y_pipe_f, z_tile, zc, y_split, pad).  x_radix, x_lanes,
 // x_rows, y_radix, y_lanes, y_lpw, fixed, z_tile, y_split and pad shape the
 // plan made at set-up; the others are read at every launch.
 struct DemagTuning {
     int x_radix = 16, x_lanes = 0, x_rows = 0;
     int y_radix = 16, y_lanes = 0, y_lpw = 0;
     int fixed = 1;   // 0: runtime-planned line kernels even for scheduled lengths
-    int z_quad = -1;  // 1: four lanes per z column instead of two (even nz); -1: FP64 only
     int xcd = 1;     // 0: no per-XCD renumbering of workgroups
     int y_pipe = 1;    // line groups per workgroup of the y line kernel; > 1 prefetches the next (0: off)
     int y_pipe_f = 1;  // > 0: the same for the forward y pass (half-zero input)
@@ -49,16 +48,15 @@ struct DemagTuning {
 // Applies "key=value,..." (unknown keys ignored) on top of t.
 void parse_tuning_string(DemagTuning &t, const char *text);
 
-// Octant tensor layout in reals: entry (kx, oy, oz) starts at kx skx + oy soy
-// + (oz >> 1) soz (+ odd for odd oz) and holds its components consecutively.
-// Short z lines (pz <= 16): one block per (kx, oy) column holding the even-oz
-// entries and then the odd-oz ones, each half padded to 16 bytes, so that a
-// lane owning kz of one parity reads its whole half with 16-byte loads (kz
-// and pz - kz share an entry and a parity).  Long z lines: oy is the fastest
-// index of the entries, so that lanes on neighbouring columns read
-// neighbouring entries.
+// Octant tensor layout in reals: component c of entry (kx, oy, oz) at
+// kx skx + oy soy + (oz >> 1) soz (+ odd for odd oz) + c sc.  oy is the fastest
+// index of a 3-D tensor, so that lanes on neighbouring columns read
+// neighbouring entries: component planes (sc = py / 2 + 1) for the register z
+// lines (pz <= 16), whose lanes read one column each, and consecutive
+// components (sc = 1) for the longer ones, whose lanes spread over oz too.
+// Films: the four components of an entry together.
 struct KernLayout {
-    int64_t skx = 0, soy = 0, soz = 0, odd = 0;
+    int64_t skx = 0, soy = 0, soz = 0, odd = 0, sc = 1;
 };
 
 struct DemagPlan {

@@ -470,7 +470,6 @@ void parse_tuning_string(DemagTuning &t, const char *text) {
             else if (k == "y_lanes") t.y_lanes = v;
             else if (k == "y_lpw") t.y_lpw = v;
             else if (k == "fixed") t.fixed = v;
-            else if (k == "z_quad") t.z_quad = v;
             else if (k == "xcd") t.xcd = v;
             else if (k == "y_pipe") t.y_pipe = v;
             else if (k == "y_pipe_f") t.y_pipe_f = v;
@@ -653,19 +652,12 @@ bool plan_geometry(DemagPlan &dp, std::string &err, int keep_split = -1) {
     {
         const int64_t ly = dp.py / 2 + 1, nzo = dp.kz_n;
         KernLayout &l = dp.kl;
-        if (dp.three_d && dp.pz > z_reg_max<Real>()) {
-            l.soy = dp.kcomp;
-            l.odd = ly * dp.kcomp;
-            l.soz = 2 * l.odd;
-            l.skx = nzo * l.odd;
-        } else {
-            const int64_t vec = 16 / (int64_t)sizeof(Real);
-            const int64_t ne = (nzo + 1) / 2, no = nzo / 2;  // octant kz entries of either parity
-            l.soz = dp.kcomp;
-            l.odd = (int64_t)cdiv(ne * dp.kcomp, vec) * vec;
-            l.soy = l.odd + (int64_t)cdiv(no * dp.kcomp, vec) * vec;
-            l.skx = ly * l.soy;
-        }
+        const bool planes = dp.three_d && dp.pz <= z_reg_max<Real>();
+        l.sc = planes ? ly : 1;
+        l.soy = planes ? 1 : dp.kcomp;
+        l.odd = ly * dp.kcomp;
+        l.soz = 2 * l.odd;
+        l.skx = nzo * l.odd;
     }
     if (!pick_x(dp.lx, ce, dp.xr, dp.x_ls, dp.tune.x_rows > 0 ? dp.tune.x_rows : 16, dp.lds_limit)) {
         err = "x line FFT does not fit in one workgroup";
@@ -775,9 +767,6 @@ bool demag_setup(Context &c, const fullmag_fdm_plan_desc &plan, bool newell_on_d
     dp.kz_n = dp.three_d ? dp.pz / 2 + 1 : 1;
     dp.inv_npad = 1.0 / ((double)dp.px * dp.py * dp.pz);
     dp.lds_limit = device_lds_limit(c.device);
-    // measured at 512x512x8: four lanes per column are faster in FP64 (half
-    // the registers per lane), the LDS-staged two-lane tile in FP32
-    if (dp.tune.z_quad < 0) dp.tune.z_quad = c.mode == MODE_DOUBLE ? 1 : 0;
     if (!plan_lines(dp, c.last_error)) return false;
     if (c.mode == MODE_DOUBLE) return setup_t<double>(c, plan);
     return setup_t<float>(c, plan);
@@ -790,7 +779,6 @@ bool demag_replan(Context &c, const DemagTuning &t, std::string &err) {
     }
     DemagPlan dp = c.dp;
     dp.tune = t;
-    if (dp.tune.z_quad < 0) dp.tune.z_quad = c.mode == MODE_DOUBLE ? 1 : 0;
     if (!plan_lines(dp, err)) return false;
     const bool ok = c.mode == MODE_DOUBLE ? plan_geometry<double>(dp, err, c.dp.y_split ? 1 : 0)
                                           : plan_geometry<float>(dp, err, c.dp.y_split ? 1 : 0);

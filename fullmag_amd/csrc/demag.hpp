@@ -54,7 +54,7 @@ struct KernelView {
 
 // Entry (kx, oy, oz), component c of the octant tensor (KernLayout).
 __host__ __device__ __forceinline__ int64_t kern_at(const KernLayout &l, int c, int oz, int kx, int oy) {
-    return kx * l.skx + oy * l.soy + ((oz & 1) ? l.odd : 0) + (oz >> 1) * l.soz + c;
+    return kx * l.skx + oy * l.soy + ((oz & 1) ? l.odd : 0) + (oz >> 1) * l.soz + c * l.sc;
 }
 
 // t = (xx, yy, zz, xy, xz, yz) at frequency (kx, ky, kz); kx <= nx.
@@ -72,13 +72,14 @@ __device__ __forceinline__ void tensor_at(const KernelView<Real> &K, int kx, int
             sz = zlo ? Real(1) : Real(-1);
         }
         const Real *e = K.k + kern_at(K.l, 0, oz, kx, oy);
+        const int64_t sc = K.l.sc;
         t[0] = e[0];
-        t[1] = e[1];
-        t[2] = e[2];
-        t[3] = sy * e[3];
+        t[1] = e[sc];
+        t[2] = e[2 * sc];
+        t[3] = sy * e[3 * sc];
         if (K.kcomp == 6) {
-            t[4] = sz * e[4];
-            t[5] = sy * sz * e[5];
+            t[4] = sz * e[4 * sc];
+            t[5] = sy * sz * e[5 * sc];
         } else {
             t[4] = Real(0);
             t[5] = Real(0);
@@ -345,7 +346,7 @@ template <typename Real>
 void launch_yconv(Context &c, const YConvArgs<Real> &ya);
 template <typename Real>
 void launch_film_tensor(Context &c, cplx<Real> *spec, const KernelView<Real> &K, int hx, int py, int64_t rows);
-// demag_z.hip: the register z convolution (pz <= 16) and the LDS z lines
+// demag_z.hip: the register z convolution (pz <= 16) and the longer z lines
 // (convolution, or plain transforms of `comps` components).
 template <typename Real>
 void launch_zreg(Context &c, const ZArgs<Real> &za);

@@ -6,427 +6,212 @@
 namespace fm {
 namespace {
 
-// DFT of length N on registers with roots w_N^t = w_P^(S t) taken from the
-// length-P = S N table (power-of-two N uses exact constants).
-template <typename Real, int N, int S>
-__device__ __forceinline__ void strided_dft(cplx<Real> *v, const cplx<Real> *tw_p, bool inv) {
-    if constexpr (N == 1) {
-        (void)v; (void)tw_p; (void)inv;
-    } else if constexpr (N == 2 || N == 4 || N == 8 || N == 16) {
-        dft_any<Real, N>(v, tw_p, N, inv);
-    } else {
-        cplx<Real> out[N];
-#pragma unroll
-        for (int q = 0; q < N; ++q) {
-            cplx<Real> acc = v[0];
-#pragma unroll
-            for (int r = 1; r < N; ++r) {
-                cplx<Real> w = tw_p[S * ((r * q) % N)];
-                if (inv) w.y = -w.y;
-                acc = cadd(acc, cmul(v[r], w));
-            }
-            out[q] = acc;
-        }
-#pragma unroll
-        for (int q = 0; q < N; ++q) v[q] = out[q];
-    }
+// Element `i` of an array whose base is uniform over the wavefront: the lane
+// carries a 32-bit byte offset and the base stays in scalar registers.
+template <typename T>
+__device__ __forceinline__ T *lane_at(T *base, uint32_t i) {
+    using B = typename std::conditional<std::is_const<T>::value, const char, char>::type;
+    return reinterpret_cast<T *>(reinterpret_cast<B *>(base) + (uint32_t)(i * (uint32_t)sizeof(T)));
 }
 
-template <typename Real, int N>
-__device__ __forceinline__ void half_dft(cplx<Real> *v, const cplx<Real> *tw_p, bool inv) {
-    if constexpr (N == 1) {
-        (void)v; (void)tw_p; (void)inv;
-    } else if constexpr (N == 2 || N == 4 || N == 8 || N == 16) {
-        dft_any<Real, N>(v, tw_p, N, inv);
-    } else {
-        cplx<Real> out[N];
-#pragma unroll
-        for (int q = 0; q < N; ++q) {
-            cplx<Real> acc = v[0];
-#pragma unroll
-            for (int r = 1; r < N; ++r) {
-                cplx<Real> w = tw_p[2 * ((r * q) % N)];
-                if (inv) w.y = -w.y;
-                acc = cadd(acc, cmul(v[r], w));
-            }
-            out[q] = acc;
-        }
-#pragma unroll
-        for (int q = 0; q < N; ++q) v[q] = out[q];
-    }
-}
+// V neighbouring columns, one 16-byte access.
+template <typename Real, int V>
+struct alignas(sizeof(cplx<Real>) * V) cvec {
+    cplx<Real> c[V];
+};
 
-// z convolution with two lanes per (kx, ky) column (pz = 2 NZ): lane parity p
-// owns kz = 2k + p.  Forward: X[2k+p] = DFT_NZ(x_z w_pz^(p z))[k] (only the
-// NZ non-zero inputs exist); tensor at its own kz; inverse:
-// y_z = IDFT_NZ(Y_even)[z] + w_pz^(-z) IDFT_NZ(Y_odd)[z], z < NZ, summed
-// across the lane pair with a shuffle.  All three components in registers.
-// Consecutive lane pairs take consecutive columns.  Used where the staged
-// tile does not apply (the k-space projection fallback).
-template <typename Real, int NZ>
-__global__ void __launch_bounds__(256) zconv_pair_kernel(ZArgs<Real> a) {
-    const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int p = (int)(gid & 1);
-    // both lanes of a pair stay for the shuffle
-    const int64_t col = gid >> 1;
-    bool valid = col < a.columns;
-    const int kx = valid ? (int)(col / a.pitch) : 0;
-    const int ky = valid ? (int)(col - (int64_t)kx * a.pitch) : 0;
-    valid = valid && ky < a.py;
-    cplx<Real> v[3][NZ];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-#pragma unroll
-        for (int z = 0; z < NZ; ++z) {
-            cplx<Real> x = {Real(0), Real(0)};
-            if (valid) x = a.data[c * a.comp_stride + z * a.zstride + col];
-            if (p && z) x = cmul(x, a.tw[z]);
-            v[c][z] = x;
-        }
-        half_dft<Real, NZ>(v[c], a.tw, false);
-    }
-#pragma unroll
-    for (int k = 0; k < NZ; ++k) {
-        Real t[6];
-        tensor_at(a.K, kx, ky, 2 * k + p, t);
-        apply_tensor(t, v[0][k], v[1][k], v[2][k]);
-    }
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        half_dft<Real, NZ>(v[c], a.tw, true);
-#pragma unroll
-        for (int z = 0; z < NZ; ++z) {
-            cplx<Real> y = v[c][z];
-            if (p && z) y = cmul(y, cconj(a.tw[z]));
-            const cplx<Real> o = {__shfl_xor(y.x, 1), __shfl_xor(y.y, 1)};
-            v[c][z] = cadd(y, o);
-        }
-    }
-    if (!valid) return;
+// Short z lines (pz = 2 NZ <= 16): one lane per (kx, ky) column, all three
+// components in registers, no LDS and no barrier.  The NZ non-zero inputs of
+// the padded line give the even kz = 2k as DFT_NZ(x)[k] and the odd
+// kz = 2k + 1 as DFT_NZ(x_z w_pz^z)[k]; each half gets its tensor entries and
+// is transformed back (the odd half times w_pz^-z), so only one half of the
+// padded spectrum exists at a time and the input registers carry the odd
+// half.  Consecutive lanes take consecutive columns, so every load and store
+// is one contiguous run per wavefront, the tensor entries (oy fastest)
+// included.  kz and pz - kz share an entry and, for kz > NZ, xz and yz change
+// sign.  PROJ: the tensor is the k-space projection's, computed per kz.
+// FP32 512x512x8: 52 us for 259 MB (5.0 TB/s), as much as the LDS-staged tile
+// with two lanes per column took, a copy of the inputs straight to LDS (54 us)
+// and one wavefront per component (57 us); 256x256x4 9.5 -> 7.9 us and
+// 250x150x6 14.9 -> 10.9 us against that tile.
+template <typename Real, int NZ, bool PROJ>
+__device__ __forceinline__ void zreg_body(const ZArgs<Real> &a) {
+    using C = cplx<Real>;
+    constexpr int NE = NZ / 2 + 1, NO = (NZ + 1) / 2;  // octant entries of even and odd kz
+    const uint32_t blk = a.xcd ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
+    const uint32_t cl = blk * 256u + threadIdx.x;
+    // a lane past the end repeats the last column: the kx of a wavefront's
+    // lanes never falls below its first lane's (see kx0)
+    const bool live = cl < a.columns;
+    const uint32_t col = live ? cl : (uint32_t)a.columns - 1u;
+    const int kx = (int)(col / (uint32_t)a.pitch), ky = (int)(col - (uint32_t)kx * (uint32_t)a.pitch);
+    C x[3][NZ];
 #pragma unroll
     for (int c = 0; c < 3; ++c)
 #pragma unroll
-        for (int z = 0; z < NZ; ++z)
-            if ((z & 1) == p) a.data[c * a.comp_stride + z * a.zstride + col] = v[c][z];
-}
-
-// The two-lane z convolution staged through LDS: a workgroup of 256 lanes
-// owns 128 consecutive columns.  It loads the tile's 3 NZ rows of 128
-// complex values (one row = one (component, z) plane segment) with 16-byte
-// loads, all issued before any arithmetic; lane pair j computes column j
-// from LDS exactly as zconv_pair_kernel does; the results go back through
-// LDS and out with 16-byte stores.  The tile's whole input is in flight at
-// once and no lane keeps loaded data in registers across the transform.
-constexpr int kZTile = 128;
-
-// Tile of kZTile consecutive columns starting at col0: 3 NZ rows, each row
-// one contiguous run of the spectrum.  Lane t moves 16-byte units t + 256 i.
-template <typename Real, int NZ, int TW = kZTile>
-struct ZTile {
-    using C = cplx<Real>;
-    static constexpr int ROWS = 3 * NZ;
-    static constexpr int V = sizeof(Real) == 4 ? 2 : 1;  // complex values per 16-byte access
-    static constexpr int UNITS = TW / V;                 // accesses per row
-    static constexpr int PER = (ROWS * UNITS + 255) / 256;
-    C v[PER][V];
-
-    __device__ __forceinline__ void fetch(const ZArgs<Real> &a, int64_t col0, int t) {
-        if (col0 + TW <= a.columns) {
-            // the whole tile lies inside the spectrum (every tile but possibly
-            // the last): unconditional 16-byte loads, all issued before any
-            // wait; a lane's unit past the tile re-reads the tile's last unit
-            // and put() drops it
+        for (int z = 0; z < NZ; ++z) x[c][z] = *lane_at(a.data + c * a.comp_stride + z * a.zstride, col);
+    const bool ylo = ky <= a.K.ny;
+    const Real sy = ylo ? Real(1) : Real(-1);
+    const int kx0 = __builtin_amdgcn_readfirstlane(kx);
+    const Real *kb = a.K.k + kx0 * a.K.l.skx;
+    const uint32_t ko = (uint32_t)((kx - kx0) * (int)a.K.l.skx + (ylo ? ky : a.py - ky));
+    auto load = [&](Real (*t)[6], int n, int64_t off) {
 #pragma unroll
-            for (int i = 0; i < PER; ++i) {
-                const int idx = min(t + 256 * i, ROWS * UNITS - 1);
-                const int r = idx / UNITS, u = idx - r * UNITS;
-                const int c = r / NZ, z = r - c * NZ;
-                const C *src = a.data + c * a.comp_stride + z * a.zstride + col0 + (int64_t)u * V;
-                if constexpr (V == 2) {
-                    const float4 q = *reinterpret_cast<const float4 *>(src);
-                    v[i][0] = C{Real(q.x), Real(q.y)};
-                    v[i][1] = C{Real(q.z), Real(q.w)};
-                } else {
-                    v[i][0] = *src;
-                }
-            }
-            return;
-        }
+        for (int i = 0; i < n; ++i)
 #pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            const int idx = t + 256 * i;
+            for (int q = 0; q < 6; ++q) t[i][q] = *lane_at(kb + off + i * a.K.l.soz + q * a.K.l.sc, ko);
+    };
+    // v = the kz = 2k + odd half; tensor, back to z
+    auto half = [&](C (*v)[NZ], const Real (*t)[6], int odd) {
 #pragma unroll
-            for (int e = 0; e < V; ++e) v[i][e] = C{Real(0), Real(0)};
-            if (idx < ROWS * UNITS) {
-                const int r = idx / UNITS, u = idx - r * UNITS;
-                const int c = r / NZ, z = r - c * NZ;
-                const int64_t col = col0 + (int64_t)u * V;
-                const C *src = a.data + c * a.comp_stride + z * a.zstride + col;
-                if (col + V <= a.columns) {
-                    if constexpr (V == 2) {
-                        const float4 q = *reinterpret_cast<const float4 *>(src);
-                        v[i][0] = C{Real(q.x), Real(q.y)};
-                        v[i][1] = C{Real(q.z), Real(q.w)};
-                    } else {
-                        v[i][0] = *src;
-                    }
-                } else {
-                    for (int e = 0; e < V; ++e)
-                        if (col + e < a.columns) v[i][e] = src[e];
-                }
-            }
-        }
-    }
-    __device__ __forceinline__ void put(C (*tile)[TW + V], int t) const {
+        for (int c = 0; c < 3; ++c) dft_any<Real, NZ>(v[c], a.tw, NZ, false);
 #pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            const int idx = t + 256 * i;
-            if (idx < ROWS * UNITS) {
-                const int r = idx / UNITS, u = idx - r * UNITS;
-#pragma unroll
-                for (int e = 0; e < V; ++e) tile[r][u * V + e] = v[i][e];
-            }
-        }
-    }
-};
-
-template <typename Real, int NZ, int TW = kZTile>
-__device__ __forceinline__ void ztile_store(const ZArgs<Real> &a, cplx<Real> (*tile)[TW + ZTile<Real, NZ, TW>::V],
-                                            int64_t col0, int t) {
-    using C = cplx<Real>;
-    using TL = ZTile<Real, NZ, TW>;
-    constexpr int V = TL::V, UNITS = TL::UNITS;
-#pragma unroll
-    for (int i = 0; i < TL::PER; ++i) {
-        const int idx = t + 256 * i;
-        if (idx < TL::ROWS * UNITS) {
-            const int r = idx / UNITS, u = idx - r * UNITS;
-            const int c = r / NZ, z = r - c * NZ;
-            const int64_t cl = col0 + (int64_t)u * V;
-            C *dst = a.data + c * a.comp_stride + z * a.zstride + cl;
-            if (cl + V <= a.columns) {
-                if constexpr (V == 2) {
-                    const C e0 = tile[r][u * 2], e1 = tile[r][u * 2 + 1];
-                    *reinterpret_cast<float4 *>(dst) = float4{float(e0.x), float(e0.y), float(e1.x), float(e1.y)};
-                } else {
-                    *dst = tile[r][u];
-                }
+        for (int k = 0; k < NZ; ++k) {
+            const int kz = 2 * k + odd, i = (kz <= NZ ? kz : 2 * NZ - kz) >> 1;
+            const Real sz = kz <= NZ ? Real(1) : Real(-1);
+            Real tt[6];
+            if constexpr (PROJ) {
+                tensor_at(a.K, kx, ky, kz, tt);
             } else {
-                for (int e = 0; e < V; ++e)
-                    if (cl + e < a.columns) dst[e] = tile[r][u * V + e];
+                tt[0] = t[i][0];
+                tt[1] = t[i][1];
+                tt[2] = t[i][2];
+                tt[3] = sy * t[i][3];
+                tt[4] = sz * t[i][4];
+                tt[5] = sz * (sy * t[i][5]);
             }
+            apply_tensor(tt, v[0][k], v[1][k], v[2][k]);
         }
-    }
-}
-
-// The lane's half of its column's octant tensor block (the entries of its
-// kz parity, six components each), in registers.  Issued at the start of the
-// tile kernel together with the tile's loads, so one memory wait covers both.
-// Pad columns and the projection fallback keep zeros.
-// FP64 keeps only the block's address (30 doubles would double the
-// registers) and reads each entry where it is applied.
-template <typename Real, int NZ>
-struct ZTensorRegs {
-    static constexpr int NE = NZ / 2 + 1, NO = (NZ + 1) / 2;
-    static constexpr bool REGS = sizeof(Real) == 4;
-    static constexpr int NV = (6 * NE + 3) / 4;  // 16-byte loads of the longer (even) half
-    Real k[REGS ? NV * 4 : 1];
-    const Real *blk = nullptr;
-    bool valid = false;
-    __device__ __forceinline__ void load(const ZArgs<Real> &a, bool col_valid, int kx, int ky, int p) {
-        valid = col_valid && a.K.k;
-        const int oy = ky <= a.K.ny ? ky : a.py - ky;
-        blk = valid ? a.K.k + kern_at(a.K.l, 0, p, kx, oy) : a.K.k;
-        if constexpr (REGS) {
 #pragma unroll
-            for (int e = 0; e < NV * 4; ++e) k[e] = Real(0);
-            if (!valid) return;
-            const float4 *src = reinterpret_cast<const float4 *>(blk);
-            const int nv = p ? (6 * NO + 3) / 4 : NV;
-#pragma unroll
-            for (int e = 0; e < NV; ++e) {
-                if (e < nv) {
-                    const float4 q = src[e];
-                    k[4 * e] = q.x;
-                    k[4 * e + 1] = q.y;
-                    k[4 * e + 2] = q.z;
-                    k[4 * e + 3] = q.w;
-                }
-            }
-        }
-    }
-};
-
-// The register convolution of one column of the tile (two lanes per column,
-// as zconv_pair_kernel), in place in LDS: lane pair t/2 takes column t/2.  A
-// column is read and written only by its own lane pair, which sits in one
-// wave, so no barrier separates the reads from the writes.
-template <typename Real, int NZ, int TW = kZTile>
-__device__ __forceinline__ void ztile_convolve(const ZArgs<Real> &a, cplx<Real> (*tile)[TW + ZTile<Real, NZ, TW>::V],
-                                               int j, int p, int ky, const ZTensorRegs<Real, NZ> &kr) {
-    using C = cplx<Real>;
-    C v[3][NZ];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-#pragma unroll
-        for (int z = 0; z < NZ; ++z) {
-            C x = tile[c * NZ + z][j];
-            if (p && z) x = cmul(x, a.tw[z]);
-            v[c][z] = x;
-        }
-        half_dft<Real, NZ>(v[c], a.tw, false);
-    }
-    const Real sy = ky <= a.K.ny ? Real(1) : Real(-1);
-#pragma unroll
-    for (int k = 0; k < NZ; ++k) {
-        // lane parity p owns kz = 2k + p; its octant entry is (kz or pz - kz) / 2
-        const int kz0 = 2 * k, kz1 = 2 * k + 1;
-        const int i0 = (kz0 <= NZ ? kz0 : 2 * NZ - kz0) >> 1, i1 = (kz1 <= NZ ? kz1 : 2 * NZ - kz1) >> 1;
-        const Real s0 = kz0 <= NZ ? Real(1) : Real(-1), s1 = kz1 <= NZ ? Real(1) : Real(-1);
-        const Real sz = p ? s1 : s0;
-        Real tt[6];
-        if constexpr (sizeof(Real) == 4) {
-            // select between two fixed registers with a bit mask (an index
-            // chosen at run time would move the array to scratch)
-            const uint32_t msk = 0u - (uint32_t)p;
-#pragma unroll
-            for (int q = 0; q < 6; ++q) {
-                const uint32_t b0 = __float_as_uint(kr.k[6 * i0 + q]), b1 = __float_as_uint(kr.k[6 * i1 + q]);
-                tt[q] = __uint_as_float((b0 & ~msk) | (b1 & msk));
-            }
-        } else {
-            const Real *e = kr.blk + 6 * (p ? i1 : i0);
-#pragma unroll
-            for (int q = 0; q < 6; ++q) tt[q] = kr.valid ? e[q] : Real(0);
-        }
-        tt[3] = sy * tt[3];
-        tt[4] = sz * tt[4];
-        tt[5] = sy * sz * tt[5];
-        apply_tensor(tt, v[0][k], v[1][k], v[2][k]);
-    }
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        half_dft<Real, NZ>(v[c], a.tw, true);
-#pragma unroll
-        for (int z = 0; z < NZ; ++z) {
-            C y = v[c][z];
-            if (p && z) y = cmul(y, cconj(a.tw[z]));
-            const C o = {__shfl_xor(y.x, 1), __shfl_xor(y.y, 1)};
-            if ((z & 1) == p) tile[c * NZ + z][j] = cadd(y, o);
-        }
-    }
-}
-
-template <typename Real, int NZ, int TW>
-__device__ __forceinline__ void zconv_tile_body(const ZArgs<Real> &a) {
-    static_assert(TW == 128, "one column per lane pair of a 256-lane workgroup");
-    using TL = ZTile<Real, NZ, TW>;
-    __shared__ cplx<Real> tile[TL::ROWS][TW + TL::V];
-    const uint32_t blk = a.xcd ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
-    const int64_t col0 = (int64_t)blk * TW;
-    const int t = (int)threadIdx.x;
-    const int j = t >> 1, p = t & 1;
-    const int64_t col = col0 + j;
-    bool valid = col < a.columns;
-    const int kx = valid ? (int)(col / a.pitch) : 0;
-    const int ky = valid ? (int)(col - (int64_t)kx * a.pitch) : 0;
-    valid = valid && ky < a.py;  // pad columns: transformed with a zero tensor, never read
-    ZTensorRegs<Real, NZ> kr;
-    kr.load(a, valid, kx, ky, p);
+        for (int c = 0; c < 3; ++c) dft_any<Real, NZ>(v[c], a.tw, NZ, true);
+    };
+    C y[3][NZ];
     {
-        TL in;
-        in.fetch(a, col0, t);
-        in.put(tile, t);
+        Real t[NE][6];
+        if constexpr (!PROJ) load(t, NE, 0);
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int z = 0; z < NZ; ++z) y[c][z] = x[c][z];
+        half(y, t, 0);
     }
-    __syncthreads();
-    ztile_convolve<Real, NZ, TW>(a, tile, j, p, ky, kr);
-    __syncthreads();
-    ztile_store<Real, NZ, TW>(a, tile, col0, t);
+    {
+        Real t[NO][6];
+        if constexpr (!PROJ) load(t, NO, a.K.l.odd);
+#pragma unroll
+        for (int z = 1; z < NZ; ++z) {
+            const C w = a.tw[z];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) x[c][z] = cmul(x[c][z], w);
+        }
+        half(x, t, 1);
+    }
+#pragma unroll
+    for (int z = 0; z < NZ; ++z) {
+        const C w = cconj(a.tw[z]);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const C o = cadd(y[c][z], z > 0 ? cmul(x[c][z], w) : x[c][z]);
+            if (live) *lane_at(a.data + c * a.comp_stride + z * a.zstride, col) = o;
+        }
+    }
 }
 
-template <typename Real, int NZ, int TW = kZTile>
-__global__ void __launch_bounds__(256) zconv_tile_kernel(ZArgs<Real> a) {
-    zconv_tile_body<Real, NZ, TW>(a);
-}
-template <typename Real, int NZ, int TW = kZTile>
-__global__ void __launch_bounds__(256) zconv_tile_multi(const ZArgs<Real> *tab, int zdiv) {
-    const ZArgs<Real> a = tab[blockIdx.z / zdiv];
-    zconv_tile_body<Real, NZ, TW>(a);
-}
-
-// z convolution with four lanes per (kx, ky) column (pz = 2 NZ = 4 M, NZ
-// even): lane q owns kz = 4k + q.  Forward: X[4k+q] = DFT_M(u)[k] with the
-// folded input u_z = x_z w^(q z) + x_(z+M) w^(q (z+M)), z < M; tensor at its
-// own kz; inverse: y_z = sum_q w^(-q z) IDFT_M(Y_q)[z mod M], summed over the
-// quad with two shuffles; lane q stores the z = q (mod 4).  Workgroups are
-// renumbered per XCD so the columns ky and py - ky of one kx row, which read
-// the same tensor octant entries, share an L2.
+// The same in FP64 for NZ >= 3, where one column's three components take more
+// registers than a lane has: one wavefront per component, so that two to four
+// wavefronts share a SIMD.  The spectra of a half meet in LDS
+// ([component][k][lane]): a wavefront reads the other two components and forms
+// its own row of the tensor product.  The mirrored entries' signs go on the y
+// and z vectors: xy and yz change with ky's mirror, xz and yz with kz's, which
+// is the same as flipping y (z) before and after the product.
+// 512x512x8: 157 us with four lanes per column and two shuffles per output,
+// 177 us as zreg_body (one wavefront per SIMD), 109 us here (4.7 TB/s).
 template <typename Real, int NZ>
-__device__ __forceinline__ void zconv_quad_body(const ZArgs<Real> &a) {
-    static_assert(NZ % 2 == 0, "four lanes per column need an even nz");
-    constexpr int M = NZ / 2, PZ = 2 * NZ;
+__device__ __forceinline__ void zreg3_body(const ZArgs<Real> &a) {
+    using C = cplx<Real>;
+    constexpr int NE = NZ / 2 + 1;
+    __shared__ C ex[3][NZ][64];
     const uint32_t blk = a.xcd ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
-    const int64_t gid = (int64_t)blk * blockDim.x + threadIdx.x;
-    const int64_t col = gid >> 2;
-    const int q = (int)(gid & 3);
-    bool valid = col < a.columns;  // all four lanes of a quad stay for the shuffles
-    const int kx = valid ? (int)(col / a.pitch) : 0;
-    const int ky = valid ? (int)(col - (int64_t)kx * a.pitch) : 0;
-    valid = valid && ky < a.py;
-    // w^(q z), z < NZ: one gather per z, reused by all components and the inverse
-    cplx<Real> wq[NZ];
+    const int lane = threadIdx.x & 63;
+    const int c = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const uint32_t cl = blk * 64u + (uint32_t)lane;
+    // a lane past the end repeats the last column: the kx of a wavefront's
+    // lanes never falls below its first lane's (see kx0)
+    const bool live = cl < a.columns;
+    const uint32_t col = live ? cl : (uint32_t)a.columns - 1u;
+    const int kx = (int)(col / (uint32_t)a.pitch), ky = (int)(col - (uint32_t)kx * (uint32_t)a.pitch);
+    C *data = a.data + c * a.comp_stride;
+    C x[NZ];
 #pragma unroll
-    for (int z = 0; z < NZ; ++z) wq[z] = a.tw[(q * z) % PZ];
-    cplx<Real> v[3][M];
+    for (int z = 0; z < NZ; ++z) x[z] = *lane_at(data + z * a.zstride, col);
+    // this component's row of the tensor: its own entry, the next one's and
+    // the one after
+    const int e0 = c, e1 = c == 0 ? 3 : c == 1 ? 5 : 4, e2 = c == 0 ? 4 : c == 1 ? 3 : 5;
+    const int c1 = c == 2 ? 0 : c + 1, c2 = c == 0 ? 2 : c - 1;
+    const bool ylo = ky <= a.K.ny;
+    const int kx0 = __builtin_amdgcn_readfirstlane(kx);
+    const Real *kb = a.K.k + kx0 * a.K.l.skx;
+    const uint32_t ko = (uint32_t)((kx - kx0) * (int)a.K.l.skx + (ylo ? ky : a.py - ky));
+    const Real sy = ylo || c != 1 ? Real(1) : Real(-1), sz = c == 2 ? Real(-1) : Real(1);
+    auto half = [&](C *v, int odd, int n, int64_t off) {
+        Real t[NE][3];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-#pragma unroll
-        for (int z = 0; z < M; ++z) {
-            cplx<Real> lo = {Real(0), Real(0)}, hi = {Real(0), Real(0)};
-            if (valid) {
-                lo = a.data[c * a.comp_stride + z * a.zstride + col];
-                hi = a.data[c * a.comp_stride + (z + M) * a.zstride + col];
-            }
-            v[c][z] = cadd(cmul(lo, wq[z]), cmul(hi, wq[z + M]));
+        for (int i = 0; i < n; ++i) {
+            const Real *p = kb + off + i * a.K.l.soz;
+            t[i][0] = *lane_at(p + e0 * a.K.l.sc, ko);
+            t[i][1] = *lane_at(p + e1 * a.K.l.sc, ko);
+            t[i][2] = *lane_at(p + e2 * a.K.l.sc, ko);
         }
-        strided_dft<Real, M, 4>(v[c], a.tw, false);
-    }
+        dft_any<Real, NZ>(v, a.tw, NZ, false);
 #pragma unroll
-    for (int k = 0; k < M; ++k) {
-        Real t[6];
-        tensor_at(a.K, kx, ky, 4 * k + q, t);
-        apply_tensor(t, v[0][k], v[1][k], v[2][k]);
-    }
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        strided_dft<Real, M, 4>(v[c], a.tw, true);
-        cplx<Real> y[NZ];
-#pragma unroll
-        for (int z = 0; z < NZ; ++z) {
-            cplx<Real> s = cmul(v[c][z % M], cconj(wq[z]));
-            s.x += __shfl_xor(s.x, 1);
-            s.y += __shfl_xor(s.y, 1);
-            s.x += __shfl_xor(s.x, 2);
-            s.y += __shfl_xor(s.y, 2);
-            y[z] = s;
+        for (int k = 0; k < NZ; ++k) {
+            const Real g = 2 * k + odd <= NZ ? Real(1) : sz;
+            ex[c][k][lane] = v[k] = {g * v[k].x, g * v[k].y};
         }
-        if (valid)
+        __syncthreads();
 #pragma unroll
-            for (int z = 0; z < NZ; ++z)
-                if ((z & 3) == q) a.data[c * a.comp_stride + z * a.zstride + col] = y[z];
+        for (int k = 0; k < NZ; ++k) {
+            const int kz = 2 * k + odd, i = (kz <= NZ ? kz : 2 * NZ - kz) >> 1;
+            const Real g = kz <= NZ ? Real(-1) : -sz;
+            const C p = ex[c1][k][lane], q = ex[c2][k][lane];
+            v[k] = {g * (t[i][0] * v[k].x + t[i][1] * p.x + t[i][2] * q.x),
+                    g * (t[i][0] * v[k].y + t[i][1] * p.y + t[i][2] * q.y)};
+        }
+        dft_any<Real, NZ>(v, a.tw, NZ, true);
+    };
+    C y[NZ];
+#pragma unroll
+    for (int z = 0; z < NZ; ++z) y[z] = x[z] = {sy * x[z].x, sy * x[z].y};
+    half(y, 0, NE, 0);
+#pragma unroll
+    for (int z = 1; z < NZ; ++z) x[z] = cmul(x[z], a.tw[z]);
+    __syncthreads();  // the even half's spectra have been read
+    half(x, 1, (NZ + 1) / 2, a.K.l.odd);
+#pragma unroll
+    for (int z = 0; z < NZ; ++z) {
+        const C o = cadd(y[z], z > 0 ? cmul(x[z], cconj(a.tw[z])) : x[z]);
+        if (live) *lane_at(data + z * a.zstride, col) = {sy * o.x, sy * o.y};
     }
 }
-
 template <typename Real, int NZ>
-__global__ void __launch_bounds__(256) zconv_quad_kernel(ZArgs<Real> a) {
-    zconv_quad_body<Real, NZ>(a);
+__global__ void __launch_bounds__(192) zreg3_kernel(ZArgs<Real> a) {
+    zreg3_body<Real, NZ>(a);
 }
 template <typename Real, int NZ>
-__global__ void __launch_bounds__(256) zconv_quad_multi(const ZArgs<Real> *tab, int zdiv) {
+__global__ void __launch_bounds__(192) zreg3_multi(const ZArgs<Real> *tab, int zdiv) {
     const ZArgs<Real> a = tab[blockIdx.z / zdiv];
-    zconv_quad_body<Real, NZ>(a);
+    zreg3_body<Real, NZ>(a);
 }
 
+template <typename Real, int NZ, bool PROJ>
+__global__ void __launch_bounds__(256) zreg_kernel(ZArgs<Real> a) {
+    zreg_body<Real, NZ, PROJ>(a);
+}
+template <typename Real, int NZ>
+__global__ void __launch_bounds__(256) zreg_multi(const ZArgs<Real> *tab, int zdiv) {
+    const ZArgs<Real> a = tab[blockIdx.z / zdiv];
+    zreg_body<Real, NZ, false>(a);
+}
 
 template <typename Real>
 __global__ void __launch_bounds__(kMaxBlock) zlds_kernel(ZLdsArgs<Real> a) {
@@ -533,10 +318,6 @@ __global__ void __launch_bounds__(kMaxBlock) zlds_kernel(ZLdsArgs<Real> a) {
 // 213 us with the staged lines of zlds_kernel, 131 us here, 147 us with one
 // column per lane (twice the wavefronts, but each pays its own twiddles and
 // 64-byte runs).  100^3 FP64: 214 -> 109 us.
-template <typename Real, int V>
-struct alignas(sizeof(cplx<Real>) * V) cvec {
-    cplx<Real> c[V];
-};
 
 // v[s][r] *= w^(r st) for the V columns s (see twiddle()).
 template <typename T, int R, int V>
@@ -745,49 +526,33 @@ __global__ void __launch_bounds__(CONV ? 192 : 64) zcol_kernel(ZLdsArgs<Real> a)
 
 template <typename Real>
 void launch_zreg(Context &c, const ZArgs<Real> &za) {
-    const DemagPlan &dp = c.dp;
-    const dim3 zb(256);
-    const bool quad = dp.tune.z_quad && (dp.nz == 4 || dp.nz == 6 || dp.nz == 8);
-    // the staged tiles read the tensor blocks directly (no projection fallback)
-    const bool staged = !quad && !dp.projection;
-    auto by_nz = [&](auto launch) {
-        switch (dp.nz) {
-            case 1: launch(std::integral_constant<int, 1>{}); break;
-            case 2: launch(std::integral_constant<int, 2>{}); break;
-            case 3: launch(std::integral_constant<int, 3>{}); break;
-            case 4: launch(std::integral_constant<int, 4>{}); break;
-            case 5: launch(std::integral_constant<int, 5>{}); break;
-            case 6: launch(std::integral_constant<int, 6>{}); break;
-            case 7: launch(std::integral_constant<int, 7>{}); break;
-            default: launch(std::integral_constant<int, 8>{}); break;
+    const dim3 grid((unsigned)cdiv(za.columns, 256)), block(256);
+    auto launch = [&](auto NZC) {
+        constexpr int NZ = decltype(NZC)::value;
+        const bool proj = !za.K.k;
+        if constexpr (sizeof(Real) == 8 && NZ >= 3) {
+            if (!proj) {
+                const dim3 g3((unsigned)cdiv(za.columns, 64));
+                launch_rec(c, reinterpret_cast<const void *>(&zreg3_multi<Real, NZ>), g3, dim3(192), 0, 1, za, [&] {
+                    hipLaunchKernelGGL((zreg3_kernel<Real, NZ>), g3, dim3(192), 0, c.stream, za);
+                });
+                return;
+            }
         }
+        launch_rec(c, proj ? nullptr : reinterpret_cast<const void *>(&zreg_multi<Real, NZ>), grid, block, 0, 1, za, [&] {
+            if (proj) hipLaunchKernelGGL((zreg_kernel<Real, NZ, true>), grid, block, 0, c.stream, za);
+            else hipLaunchKernelGGL((zreg_kernel<Real, NZ, false>), grid, block, 0, c.stream, za);
+        });
     };
-    if (staged) {
-        const dim3 zt((unsigned)cdiv(za.columns, kZTile));
-        by_nz([&](auto NZC) {
-            constexpr int NZ = decltype(NZC)::value;
-            launch_rec(c, reinterpret_cast<const void *>(&zconv_tile_multi<Real, NZ>), zt, zb, 0, 1, za,
-                       [&] { hipLaunchKernelGGL((zconv_tile_kernel<Real, NZ>), zt, zb, 0, c.stream, za); });
-        });
-    } else if (quad) {
-        const dim3 zq((unsigned)cdiv(4 * za.columns, 256));
-        auto quad_launch = [&](auto NZC) {
-            constexpr int NZ = decltype(NZC)::value;
-            launch_rec(c, reinterpret_cast<const void *>(&zconv_quad_multi<Real, NZ>), zq, zb, 0, 1, za,
-                       [&] { hipLaunchKernelGGL((zconv_quad_kernel<Real, NZ>), zq, zb, 0, c.stream, za); });
-        };
-        switch (dp.nz) {
-            case 4: quad_launch(std::integral_constant<int, 4>{}); break;
-            case 6: quad_launch(std::integral_constant<int, 6>{}); break;
-            default: quad_launch(std::integral_constant<int, 8>{}); break;
-        }
-    } else {
-        const dim3 zg((unsigned)cdiv(2 * za.columns, 256));
-        by_nz([&](auto NZC) {
-            launch_rec(c, nullptr, zg, zb, 0, 1, za, [&] {
-                hipLaunchKernelGGL((zconv_pair_kernel<Real, decltype(NZC)::value>), zg, zb, 0, c.stream, za);
-            });
-        });
+    switch (za.nz) {
+        case 1: launch(std::integral_constant<int, 1>{}); break;
+        case 2: launch(std::integral_constant<int, 2>{}); break;
+        case 3: launch(std::integral_constant<int, 3>{}); break;
+        case 4: launch(std::integral_constant<int, 4>{}); break;
+        case 5: launch(std::integral_constant<int, 5>{}); break;
+        case 6: launch(std::integral_constant<int, 6>{}); break;
+        case 7: launch(std::integral_constant<int, 7>{}); break;
+        default: launch(std::integral_constant<int, 8>{}); break;
     }
 }
 

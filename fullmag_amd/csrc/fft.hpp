@@ -235,7 +235,9 @@ __device__ __forceinline__ void dft_coprime(cplx<T> *v, const cplx<T> *tw, int n
 
 template <typename T, int R>
 __device__ __forceinline__ void dft_any(cplx<T> *v, const cplx<T> *tw, int n, bool inv) {
-    if constexpr (R == 2) {
+    if constexpr (R == 1) {
+        (void)v;
+    } else if constexpr (R == 2) {
         dft2(v[0], v[1]);
     } else if constexpr (R == 4) {
         dft4(v[0], v[1], v[2], v[3], inv);
@@ -245,6 +247,8 @@ __device__ __forceinline__ void dft_any(cplx<T> *v, const cplx<T> *tw, int n, bo
         dft16(v, inv);
     } else if constexpr (R == 12) {
         dft_coprime<T, 4, 3>(v, tw, n, inv);
+    } else if constexpr (R == 6) {
+        dft_coprime<T, 2, 3>(v, tw, n, inv);
     } else if constexpr (R == 10) {
         dft_coprime<T, 2, 5>(v, tw, n, inv);
     } else if constexpr (R == 14) {
