@@ -354,6 +354,7 @@ Context *create_impl(const fullmag_fdm_plan_desc *plan, const fullmag_fdm_ext_op
 // SoA device field of `elem` bytes per scalar -> AoS host array of T.
 template <typename T>
 bool download_soa(Context &c, const void *dev, size_t elem, T *out) {
+    if (const int done = field_to_host(c, dev, elem == 8, out, sizeof(T) == 8)) return done > 0;
     const uint64_t n = c.n;
     if (elem == 8) {
         std::vector<double> h(3 * n);

@@ -54,6 +54,7 @@ void ctx_free_all(Context &c) {
 // AoS host array -> SoA device state in the storage precision; inactive
 // cells forced to zero (native/backends/fdm/src/context.cu:733-782).
 bool ctx_upload_m(Context &c, const void *host, bool host_is_f64) {
+    if (const int done = state_from_host(c, host, host_is_f64)) return done > 0;
     const uint64_t n = c.n;
     auto get = [&](uint64_t i) -> double {
         return host_is_f64 ? static_cast<const double *>(host)[i] : (double)static_cast<const float *>(host)[i];

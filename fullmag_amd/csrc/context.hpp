@@ -199,6 +199,9 @@ struct Context {
     void *adj_g = nullptr, *adj_q = nullptr, *adj_w = nullptr;                          // Real
     double *adj_lu = nullptr, *adj_lmt = nullptr;
 
+    // scratch of the AoS <-> SoA transfers (allocated by the first one)
+    void *d_xfer = nullptr;
+
     // scratch for previews
     void *d_preview = nullptr;
     uint64_t preview_bytes = 0;
@@ -331,6 +334,11 @@ int stack_step(Stack &s, double dt, uint64_t n_steps, fullmag_fdm_step_stats *st
 bool stack_refresh(Stack &s);
 bool preview_field(Context &c, const void *field, bool field_f64, uint32_t pnx, uint32_t pny, uint32_t pnz,
                    uint32_t z0, uint32_t zs, void *dev_out, bool out_f64);
+// Whole-field transfers between a host AoS array and a device SoA field,
+// converted on the device and complete on return: 1 done, -1 failed
+// (last_error), 0 no device memory for the scratch (convert on the host).
+int state_from_host(Context &c, const void *host, bool host_f64);
+int field_to_host(Context &c, const void *field, bool field_f64, void *out, bool out_f64);
 bool alloc_integrator_buffers(Context &c);
 int integrator_step_many(Context &c, double dt, uint64_t n, fullmag_fdm_step_stats *st);
 // Graph-captured batches: prepare (H_demag(m) valid, timing off), enqueue
