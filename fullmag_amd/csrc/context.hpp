@@ -29,7 +29,7 @@ enum Mode { MODE_SINGLE = 1, MODE_DOUBLE = 2, MODE_MIXED = 3 };
 // Launch-schedule knobs of the demag transforms (0 = automatic).  Settable
 // per backend from the FULLMAG_FDM_TUNE environment variable as a comma list
 // of key=value (x_radix, x_lanes, x_rows, y_radix, y_lanes, y_lpw, fixed,
-// xcd, y_pipe, y_pipe_f, z_tile, zc, y_split, pad).  x_radix, x_lanes,
+// xcd, y_pipe, y_pipe_f, z_tile, zc, y_split, slab, pad).  x_radix, x_lanes,
 // x_rows, y_radix, y_lanes, y_lpw, fixed, z_tile, y_split and pad shape the
 // plan made at set-up; the others are read at every launch.
 struct DemagTuning {
@@ -42,6 +42,7 @@ struct DemagTuning {
     int z_tile = 0;    // > 0: at most this many columns per long-z (LDS line) workgroup
     int zc = 0;        // z planes per workgroup of the cell kernels (0: automatic)
     int y_split = 0;   // 1: thin-film y convolution as separate line and tensor passes
+    int slab = 160;    // y and z passes in one kernel for kx slabs of at most this many KB of LDS (0: off)
     int pad = 1;       // 0: transform lengths 2n even where a longer scheduled length is faster
 };
 

@@ -241,6 +241,26 @@ __global__ void __launch_bounds__(256) boundary_corr_kernel(BoundaryCorrArgs<Rea
     }
 }
 
+// Whether the y and z passes run as one slab kernel: a short-z tensor, a
+// scheduled y length of at most 512 and a slab that fits the LDS (and the
+// `slab` knob's KB).  us per mixed Heun step, separate passes and slab:
+// 64x64x4 43.7 and 37.8, 128x128x4 51.8 and 41.7, 256x256x4 83.8 and 65.3,
+// 500x250x8 189 and 167, 256x256x8 116 and 108; FP64 128x128x4 67.8 and 49.5,
+// 128x128x8 90.3 and 67.2, 500x250x4 177 and 146.  With 5 to 8 layers and
+// lines of 32 lanes a workgroup has up to 24 wavefronts of at most 85 FP64
+// values: FP64 spills (250x150x6 108 and 151), and FP32 gains only where the
+// columns divide into full rounds of nz T lanes per component (256x256x6, 2.7
+// rounds, 99 and 102; 256x192x6, 2 rounds, 94 and 90).
+template <typename Real>
+bool use_slab(const DemagPlan &dp) {
+    if (dp.projection || dp.nz < 2 || dp.pz > z_reg_max<Real>() || !dp.ly.fixed || !slab_length(dp.py)) return false;
+    const size_t bytes = (size_t)3 * dp.nz * fx_size(dp.py) * sizeof(cplx<Real>);
+    if (bytes > (size_t)dp.tune.slab * 1024 || bytes > dp.lds_limit) return false;
+    if (dp.nz <= 4 || fx_lanes(dp.py) < 32) return true;
+    const int cols = dp.nz * fx_lanes(dp.py), rounds = (int)cdiv(dp.py, cols);
+    return sizeof(Real) == 4 && 10 * dp.py >= 9 * rounds * cols;
+}
+
 // x R2C of Ms src, the y and z transforms with the tensor product and the
 // inverse y and z transforms: everything up to the x C2R, in the spectrum.
 template <typename Real, typename S>
@@ -263,7 +283,20 @@ void demag_transform_t(Context &c, const S *src, const XArgs<Real> &xa, unsigned
             launch(ms);
     }
     const KernelView<Real> K = kview<Real>(c);
-    if (dp.three_d) {
+    if (dp.three_d && use_slab<Real>(dp)) {
+        SlabArgs<Real> sa{};
+        sa.data = spec;
+        sa.tw = static_cast<const cplx<Real> *>(dp.tw_y);
+        sa.twz = static_cast<const cplx<Real> *>(dp.tw_z);
+        sa.nz = dp.nz;
+        sa.ny = dp.ny;
+        sa.hx = dp.hx;
+        sa.pitch = dp.rows;
+        sa.plane_stride = (int64_t)dp.hx * dp.rows;
+        sa.K = K;
+        Timed t(c, "demag_yz_slab");
+        launch_slab<Real>(c, dp.ly, sa);
+    } else if (dp.three_d) {
         LineArgs<Real> la{};
         la.data = spec;
         la.tw = static_cast<const cplx<Real> *>(dp.tw_y);
@@ -477,6 +510,7 @@ void parse_tuning_string(DemagTuning &t, const char *text) {
             else if (k == "zc") t.zc = v;
             else if (k == "y_split") t.y_split = v;
             else if (k == "pad") t.pad = v;
+            else if (k == "slab") t.slab = v;
         }
         pos = end + 1;
     }

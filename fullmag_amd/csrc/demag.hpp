@@ -259,6 +259,20 @@ struct YConvArgs {
 
 // MAXB: kMaxBlock, or 1024 for lines too long for three of them in
 // ---------------------------------------------------------------------------
+// kx slabs: y transforms and z convolution together
+// ---------------------------------------------------------------------------
+template <typename Real>
+struct SlabArgs {
+    cplx<Real> *data;
+    const cplx<Real> *tw, *twz;  // roots of lengths py and 2 nz
+    int nz, ny, hx, pitch;
+    int64_t plane_stride;        // between the (component, z) planes of the spectrum
+    KernelView<Real> K;
+};
+// Padded y lengths with a slab kernel: 24 lines of 32 lanes are 768.
+constexpr bool slab_length(int n) { return fx_has(n) && fx_lanes(n) <= 32; }
+
+// ---------------------------------------------------------------------------
 // z passes
 // ---------------------------------------------------------------------------
 template <typename Real>
@@ -346,6 +360,9 @@ template <typename Real>
 void launch_yconv(Context &c, const YConvArgs<Real> &ya);
 template <typename Real>
 void launch_film_tensor(Context &c, cplx<Real> *spec, const KernelView<Real> &K, int hx, int py, int64_t rows);
+// demag_s.hip: the slab kernel (slab_length(lp.n), 2 <= nz <= 8, a tensor).
+template <typename Real>
+void launch_slab(Context &c, const LinePlan &lp, const SlabArgs<Real> &sa);
 // demag_z.hip: the register z convolution (pz <= 16) and the longer z lines
 // (convolution, or plain transforms of `comps` components).
 template <typename Real>

@@ -63,3 +63,13 @@ def test_masked(fa, monkeypatch, cells, precision):
 def test_unpadded_schedule_agrees(fa, monkeypatch, cells):
     """pad=0 keeps the transforms at 2n."""
     assert field_error(fa, monkeypatch, cells, "double", tune="pad=0") <= BAR["double"]
+
+
+# y and z passes in one slab kernel: every layer count, y lengths of 2, 16 and
+# 32 lanes per line, whole and partial rounds of columns
+@pytest.mark.parametrize("precision", ["double", "mixed", "single"])
+@pytest.mark.parametrize("nz", [2, 3, 4, 5, 6, 7, 8])
+@pytest.mark.parametrize("nx,ny", [(5, 13), (17, 10), (9, 100), (12, 160), (7, 256)])
+def test_slab_and_separate_passes(fa, monkeypatch, nx, ny, nz, precision):
+    for tune in ("", "slab=0"):
+        assert field_error(fa, monkeypatch, (nx, ny, nz), precision, tune=tune) <= BAR.get(precision, 2e-6)
