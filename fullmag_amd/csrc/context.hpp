@@ -319,11 +319,13 @@ bool demag_replan(Context &c, const DemagTuning &t, std::string &err);
 bool newell_spectra_full(uint32_t nx, uint32_t ny, uint32_t nz, double dx, double dy, double dz, bool thin_film_2d,
                          double *out, std::string &err);
 
-// newell.cpp: Newell tensor on the non-negative displacement octant,
+// newell.hip: Newell tensor on the non-negative displacement octant,
 // out[c][k][j][i] for i < nx, j < ny, k < nz, c = xx, yy, zz, xy, xz, yz, at
-// displacements (i dx, j dy, k dz + z_offset).
-void newell_octant(size_t nx, size_t ny, size_t nz, double dx, double dy, double dz, std::vector<double> &out,
-                   double z_offset = 0.0);
+// displacements (i dx, j dy, k dz + z_offset), enqueued on the context's
+// stream; `out` and `scratch` (newell_scratch doubles) are device arrays.
+size_t newell_scratch(int nx, int ny, int nz);
+bool newell_octant(Context &c, int nx, int ny, int nz, double dx, double dy, double dz, double z_offset,
+                   double *scratch, double *out, std::string &err);
 
 // llg.hip
 int integrator_step(Context &c, double dt, fullmag_fdm_step_stats *st);

@@ -446,17 +446,18 @@ void demag_eval_t(Context &c, const S *src, Real *out, bool weight_ms, int phase
     }
 }
 
+// Twiddle tables of the plan's lengths, in one allocation.
 template <typename Real>
-bool upload_twiddles(Context &c, int n, void **dst) {
-    std::vector<cplx<double>> w = twiddle_table(n);
-    const size_t bytes = w.size() * sizeof(cplx<Real>);
-    if (!ctx_alloc(c, dst, bytes, "twiddle table")) return false;
-    if (sizeof(Real) == sizeof(double)) {
-        return ctx_upload(c, *dst, w.data(), bytes, "hipMemcpy(twiddles)", c.last_error);
-    }
-    std::vector<cplx<float>> wf(w.size());
-    for (size_t i = 0; i < w.size(); ++i) wf[i] = {(float)w[i].x, (float)w[i].y};
-    return ctx_upload(c, *dst, wf.data(), bytes, "hipMemcpy(twiddles)", c.last_error);
+bool upload_twiddles(Context &c) {
+    DemagPlan &dp = c.dp;
+    std::vector<cplx<Real>> all;
+    for (int n : {dp.px, dp.py, dp.three_d ? dp.pz : 1})
+        for (const cplx<double> &w : twiddle_table(n)) all.push_back({(Real)w.x, (Real)w.y});
+    const size_t bytes = all.size() * sizeof(cplx<Real>);
+    if (!ctx_alloc(c, &dp.tw_x, bytes, "twiddle tables")) return false;
+    dp.tw_y = static_cast<cplx<Real> *>(dp.tw_x) + dp.px;
+    dp.tw_z = static_cast<cplx<Real> *>(dp.tw_y) + dp.py;
+    return ctx_upload(c, dp.tw_x, all.data(), bytes, "hipMemcpy(twiddles)", c.last_error);
 }
 
 // Transform lengths: 2n per axis where the tensor comes as spectra of that
@@ -522,22 +523,28 @@ void parse_tuning(DemagTuning &t) { parse_tuning_string(t, std::getenv("FULLMAG_
 
 // Padded forward transform of the Newell kernel, FP64, into a temporary
 // spectrum spec[6][pz][hx][py].
-bool newell_forward(Context &c, const DemagPlan &dp, const std::vector<double> &oct, cplx<double> **spec_out,
-                    std::string &err, bool z_even = false) {
-    void *d_oct = nullptr, *d_spec = nullptr, *twx = nullptr, *twy = nullptr, *twz = nullptr;
-    const int pz = dp.three_d ? dp.pz : 1;
+bool newell_forward(Context &c, const DemagPlan &dp, double z_offset, cplx<double> **spec_out, std::string &err,
+                    bool z_even = false) {
+    const int pz = dp.three_d ? dp.pz : 1, nzo = dp.three_d ? dp.nz : 1;
     const SpecGeom g{dp.hx, pz, dp.py};
-    const size_t spec_bytes = 6 * (size_t)pz * dp.hx * dp.py * sizeof(cplx<double>);
     const size_t ce = sizeof(cplx<double>);
-    bool ok = hip_ok(hipMalloc(&d_oct, oct.size() * sizeof(double)), "hipMalloc(newell octant)", err) &&
-              hip_ok(hipMalloc(&d_spec, spec_bytes), "hipMalloc(newell spectrum)", err) &&
-              ctx_upload(c, d_oct, oct.data(), oct.size() * sizeof(double), "hipMemcpy(newell octant)", err);
-    auto up = [&](int n, void **dst) {
-        std::vector<cplx<double>> w = twiddle_table(n);
-        return hip_ok(hipMalloc(dst, w.size() * sizeof(cplx<double>)), "hipMalloc(twiddles)", err) &&
-               ctx_upload(c, *dst, w.data(), w.size() * sizeof(cplx<double>), "hipMemcpy(twiddles)", err);
-    };
-    ok = ok && up(dp.px, &twx) && up(dp.py, &twy) && (!dp.three_d || up(dp.pz, &twz));
+    // one allocation: the spectrum (before it, the octant's tables), the
+    // octant and the twiddle tables
+    const size_t spec_bytes = std::max(6 * (size_t)pz * dp.hx * dp.py * ce,
+                                       (newell_scratch(dp.nx, dp.ny, nzo) * sizeof(double) + ce - 1) / ce * ce);
+    const size_t oct_bytes = 6 * (size_t)dp.nx * dp.ny * nzo * sizeof(double);
+    std::vector<cplx<double>> tw = twiddle_table(dp.px);
+    for (int n : {dp.py, pz}) {
+        const std::vector<cplx<double>> w = twiddle_table(n);
+        tw.insert(tw.end(), w.begin(), w.end());
+    }
+    void *d_spec = nullptr;
+    bool ok = hip_ok(hipMalloc(&d_spec, spec_bytes + oct_bytes + tw.size() * ce), "hipMalloc(newell)", err);
+    double *d_oct = reinterpret_cast<double *>(static_cast<char *>(d_spec) + spec_bytes);
+    cplx<double> *twx = reinterpret_cast<cplx<double> *>(static_cast<char *>(d_spec) + spec_bytes + oct_bytes);
+    cplx<double> *twy = twx + dp.px, *twz = twy + dp.py;
+    ok = ok && ctx_upload(c, twx, tw.data(), tw.size() * ce, "hipMemcpy(twiddles)", err);
+    ok = ok && newell_octant(c, dp.nx, dp.ny, nzo, c.dx, c.dy, c.dz, z_offset, static_cast<double *>(d_spec), d_oct, err);
     int xr = 2, xls = dp.px;
     LinePlan lx, ly, lz;
     ok = ok && plan_line(dp.px, lx, err) && plan_line(dp.py, ly, err) && (!dp.three_d || plan_line(dp.pz, lz, err));
@@ -547,10 +554,9 @@ bool newell_forward(Context &c, const DemagPlan &dp, const std::vector<double> &
     }
     if (ok) {
         cplx<double> *spec = static_cast<cplx<double> *>(d_spec);
-        NewellSource src{static_cast<const double *>(d_oct), dp.nx, dp.ny, dp.three_d ? dp.nz : 1, dp.px, dp.py, pz,
-                         z_even ? 1 : 0};
+        NewellSource src{d_oct, dp.nx, dp.ny, nzo, dp.px, dp.py, pz, z_even ? 1 : 0};
         XArgs<double> xa{};
-        xa.tw = static_cast<const cplx<double> *>(twx);
+        xa.tw = twx;
         xa.lp = lx;
         xa.rows = dp.py;
         xa.n_in = dp.px;
@@ -563,7 +569,7 @@ bool newell_forward(Context &c, const DemagPlan &dp, const std::vector<double> &
         launch_xfwd<double>(c, xa, src, spec, (unsigned)cdiv(dp.py, xr), (unsigned)pz, 6, (size_t)(xr / 2) * xls * ce);
         LineArgs<double> la{};
         la.data = spec;
-        la.tw = static_cast<const cplx<double> *>(twy);
+        la.tw = twy;
         la.lp = ly;
         la.lines = 6ll * pz * dp.hx;
         la.line_pitch = dp.py;
@@ -579,7 +585,7 @@ bool newell_forward(Context &c, const DemagPlan &dp, const std::vector<double> &
         if (ok && dp.three_d) {
             ZLdsArgs<double> za{};
             za.data = spec;
-            za.tw = static_cast<const cplx<double> *>(twz);
+            za.tw = twz;
             za.lp = lz;
             za.n_in = dp.pz;
             za.n_out = dp.pz;
@@ -600,10 +606,6 @@ bool newell_forward(Context &c, const DemagPlan &dp, const std::vector<double> &
         ok = ok && hip_ok(hipStreamSynchronize(c.stream), "Newell setup transform", err);
         ok = ok && hip_ok(hipGetLastError(), "Newell setup launch", err);
     }
-    if (d_oct) (void)hipFree(d_oct);
-    if (twx) (void)hipFree(twx);
-    if (twy) (void)hipFree(twy);
-    if (twz) (void)hipFree(twz);
     if (!ok) {
         if (d_spec) (void)hipFree(d_spec);
         return false;
@@ -747,8 +749,7 @@ bool setup_t(Context &c, const fullmag_fdm_plan_desc &plan) {
     DemagPlan &dp = c.dp;
     const size_t ce = sizeof(cplx<Real>);
     if (!plan_geometry<Real>(dp, c.last_error)) return false;
-    if (!upload_twiddles<Real>(c, dp.px, &dp.tw_x) || !upload_twiddles<Real>(c, dp.py, &dp.tw_y)) return false;
-    if (dp.three_d && !upload_twiddles<Real>(c, dp.pz, &dp.tw_z)) return false;
+    if (!upload_twiddles<Real>(c)) return false;
     dp.spec_elems = 3ull * (dp.three_d ? dp.nz : 1) * dp.hx * dp.rows;
     if (!ctx_alloc(c, &dp.spec, dp.spec_elems * ce, "demag spectrum")) return false;
     if (dp.projection) return true;
@@ -757,11 +758,9 @@ bool setup_t(Context &c, const fullmag_fdm_plan_desc &plan) {
         if (!host_octant_from_spectra(dp, plan, kern, c.last_error)) return false;
         return upload_kern<Real>(c, kern);
     }
-    // In-library Newell build: octant on the host, padded transform on the device.
-    std::vector<double> oct;
-    newell_octant(dp.nx, dp.ny, dp.three_d ? dp.nz : 1, c.dx, c.dy, c.dz, oct);
+    // In-library Newell build: octant, padded transform.
     cplx<double> *spec = nullptr;
-    if (!newell_forward(c, dp, oct, &spec, c.last_error)) return false;
+    if (!newell_forward(c, dp, 0.0, &spec, c.last_error)) return false;
     dp.kern_elems = (uint64_t)(dp.hx * dp.kl.skx);
     const int64_t entries = (int64_t)dp.kcomp * dp.kz_n * dp.hx * (dp.py / 2 + 1);
     bool ok = ctx_alloc(c, &dp.kern, dp.kern_elems * sizeof(Real), "demag tensor") &&
@@ -1052,11 +1051,7 @@ bool stack_setup_t(Stack &s, std::string &err) {
             return false;
         }
     }
-    if (!upload_twiddles<Real>(c, dp.px, &dp.tw_x) || !upload_twiddles<Real>(c, dp.py, &dp.tw_y)) {
-        err = c.last_error;
-        return false;
-    }
-    if (dp.three_d && !upload_twiddles<Real>(c, dp.pz, &dp.tw_z)) {
+    if (!upload_twiddles<Real>(c)) {
         err = c.last_error;
         return false;
     }
@@ -1098,10 +1093,8 @@ bool stack_setup_t(Stack &s, std::string &err) {
         !ctx_upload(c, s.d_kimag, kimag.data(), kimag.size() * sizeof(uint32_t), "hipMemcpy(parities)", err))
         return false;
     for (int u = 0; u < s.nkern; ++u) {
-        std::vector<double> oct;
-        newell_octant(dp.nx, dp.ny, dp.three_d ? dp.nz : 1, c.dx, c.dy, c.dz, oct, u == 0 ? 0.0 : shifts[u - 1]);
         cplx<double> *spec = nullptr;
-        if (!newell_forward(c, dp, oct, &spec, err, u > 0)) return false;
+        if (!newell_forward(c, dp, u == 0 ? 0.0 : shifts[u - 1], &spec, err, u > 0)) return false;
         Real *dst = static_cast<Real *>(s.kern) + (uint64_t)u * s.kern_stride;
         hipLaunchKernelGGL((spec_part_kernel<Real>), dim3((unsigned)cdiv(s.kern_stride, 256)), dim3(256), 0,
                            c.stream, spec, dst, (int64_t)points, kimag[u]);
@@ -1294,12 +1287,8 @@ bool newell_spectra_full(uint32_t nx, uint32_t ny, uint32_t nz, double dx, doubl
     dp.three_d = !thin_film_2d;
     pad_lengths(dp, false, 0);
     bool ok = true;
-    std::vector<double> oct;
     cplx<double> *spec = nullptr;
-    if (ok) {
-        newell_octant(nx, ny, dp.three_d ? nz : 1, dx, dy, dz, oct);
-        ok = newell_forward(c, dp, oct, &spec, err);
-    }
+    if (ok) ok = newell_forward(c, dp, 0.0, &spec, err);
     if (ok) {
         const int pz = dp.pz;
         const SpecGeom g{dp.hx, pz, dp.py};
