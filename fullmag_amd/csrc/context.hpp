@@ -248,6 +248,10 @@ struct Stack {
     void *spec_m = nullptr, *spec_h = nullptr;
     void *kern = nullptr;      // per kernel 6 components of one real per k-point
     uint64_t kern_stride = 0;  // reals per pair kernel
+    // thin layers coupled in the y pass (YStackArgs): kernels
+    // [kernel][kx][6][py / 2 + 1], no spec_h
+    bool fused = false;
+    int kpw = 1;              // kx columns per workgroup of that pass
     int nkern = 0;
     std::vector<int> pair;    // kernel of (dst, src) at dst * L + src
     int *d_pair = nullptr;

@@ -1011,6 +1011,18 @@ __global__ void __launch_bounds__(256) spec_part_kernel(const cplx<double> *in, 
     out[i] = Real(((imag >> c) & 1u) ? in[i].y : in[i].x);
 }
 
+// The ky octant of one kernel: out[kx][c][ky], ky <= py / 2.
+template <typename Real>
+__global__ void __launch_bounds__(256) stack_octant_kernel(const cplx<double> *in, Real *out, int hx, int py,
+                                                           uint32_t imag) {
+    const int hp = py / 2 + 1;
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= (int64_t)hx * 6 * hp) return;
+    const int ky = (int)(i % hp), c = (int)(i / hp % 6), kx = (int)(i / ((int64_t)hp * 6));
+    const cplx<double> v = in[((int64_t)c * hx + kx) * py + ky];
+    out[i] = Real(((imag >> c) & 1u) ? v.y : v.x);
+}
+
 GridXfer xfer_of(const Stack &s, const Context &l) {
     const Context &c = s.conv;
     return GridXfer{(int)l.nx, (int)l.ny, (int)l.nz, l.dx, l.dy, l.dz,
@@ -1029,6 +1041,9 @@ bool stack_setup_t(Stack &s, std::string &err) {
     dp.ny = c.ny;
     dp.nz = c.nz;
     dp.three_d = c.nz > 1;
+    DemagTuning tune;
+    parse_tuning(tune);
+    dp.tune.y_split = tune.y_split;
     pad_lengths(dp, true, 0);
     dp.rows = dp.py;
     dp.inv_npad = 1.0 / ((double)dp.px * dp.py * dp.pz);
@@ -1058,8 +1073,16 @@ bool stack_setup_t(Stack &s, std::string &err) {
     s.planes = dp.pz;
     const int64_t points = (int64_t)s.planes * dp.hx * dp.py;
     s.layer_spec = 3 * (uint64_t)points;
+    // The coupled y pass takes a thin stack whose column of 3 L lines fits one
+    // workgroup; several columns where they are short.  Against the separate
+    // passes, Heun steps of 2 to 5 layers of 64 x 64 to 512 x 512: 1.03 to
+    // 1.6 times as fast wherever it fits, FP32 and FP64.
+    s.kpw = std::max(1, 256 / (3 * L * dp.ly.threads));
+    s.fused = !dp.three_d && dp.ly.fixed && L <= kStackFused && !dp.tune.y_split &&
+              3 * L * dp.ly.threads <= 1024 &&
+              (size_t)3 * L * s.kpw * line_slots(dp.ly) * ce <= dp.lds_limit;
     if (!ctx_alloc(c, &s.spec_m, (size_t)L * s.layer_spec * ce, "stack spectra") ||
-        !ctx_alloc(c, &s.spec_h, (size_t)L * s.layer_spec * ce, "stack field spectra")) {
+        (!s.fused && !ctx_alloc(c, &s.spec_h, (size_t)L * s.layer_spec * ce, "stack field spectra"))) {
         err = c.last_error;
         return false;
     }
@@ -1079,7 +1102,7 @@ bool stack_setup_t(Stack &s, std::string &err) {
             s.pair[(size_t)d * L + q] = 1 + (int)(it - shifts.begin());
         }
     s.nkern = 1 + (int)shifts.size();
-    s.kern_stride = 6 * (uint64_t)points;
+    s.kern_stride = s.fused ? 6 * (uint64_t)dp.hx * (dp.py / 2 + 1) : 6 * (uint64_t)points;
     // components with an odd number of odd axes transform to imaginary
     // values: xz (odd in x) and yz (odd in y) of the shifted kernels, whose
     // z mirror keeps the sign, and of the thin self kernel (zero there); in
@@ -1096,8 +1119,13 @@ bool stack_setup_t(Stack &s, std::string &err) {
         cplx<double> *spec = nullptr;
         if (!newell_forward(c, dp, u == 0 ? 0.0 : shifts[u - 1], &spec, err, u > 0)) return false;
         Real *dst = static_cast<Real *>(s.kern) + (uint64_t)u * s.kern_stride;
-        hipLaunchKernelGGL((spec_part_kernel<Real>), dim3((unsigned)cdiv(s.kern_stride, 256)), dim3(256), 0,
-                           c.stream, spec, dst, (int64_t)points, kimag[u]);
+        const dim3 grid((unsigned)cdiv(s.kern_stride, 256));
+        if (s.fused)
+            hipLaunchKernelGGL((stack_octant_kernel<Real>), grid, dim3(256), 0, c.stream, spec, dst, dp.hx, dp.py,
+                               kimag[u]);
+        else
+            hipLaunchKernelGGL((spec_part_kernel<Real>), grid, dim3(256), 0, c.stream, spec, dst, (int64_t)points,
+                               kimag[u]);
         const bool ok = hip_ok(hipStreamSynchronize(c.stream), "stack kernel", err);
         (void)hipFree(spec);
         if (!ok) return false;
@@ -1117,16 +1145,16 @@ bool stack_setup_t(Stack &s, std::string &err) {
     return hip_ok(hipGetLastError(), "stack setup", err);
 }
 
-// y lines (3-D: per component, over the nz stored planes) and z lines of one
-// spectrum, forward or inverse.
+// y lines (3-D: per component, over the nz stored planes) and z lines of
+// `layers` spectra, forward or inverse.
 template <typename Real>
-void stack_yz(Stack &s, cplx<Real> *spec, bool inverse) {
+void stack_yz(Stack &s, cplx<Real> *spec, int layers, bool inverse) {
     Context &c = s.conv;
     const DemagPlan &dp = c.dp;
     const int64_t comp = (int64_t)s.planes * dp.hx * dp.py;
-    auto zpass = [&] {
+    auto zpass = [&](int l) {
         ZLdsArgs<Real> za{};
-        za.data = spec;
+        za.data = spec + l * 3 * comp;
         za.tw = static_cast<const cplx<Real> *>(dp.tw_z);
         za.lp = dp.lz;
         za.n_in = inverse ? dp.pz : dp.nz;
@@ -1141,7 +1169,7 @@ void stack_yz(Stack &s, cplx<Real> *spec, bool inverse) {
         za.pitch = dp.py;
         launch_zlds<Real>(c, za, 3);
     };
-    if (dp.three_d && inverse) zpass();
+    for (int l = 0; dp.three_d && inverse && l < layers; ++l) zpass(l);
     LineArgs<Real> la{};
     la.tw = static_cast<const cplx<Real> *>(dp.tw_y);
     la.lp = dp.ly;
@@ -1152,16 +1180,16 @@ void stack_yz(Stack &s, cplx<Real> *spec, bool inverse) {
     la.inverse = inverse ? 1 : 0;
     if (dp.three_d) {
         la.lines = (int64_t)dp.nz * dp.hx;
-        for (int k = 0; k < 3; ++k) {
+        for (int k = 0; k < 3 * layers; ++k) {
             la.data = spec + k * comp;
             launch_lines<Real>(c, dp.ly, la);
         }
     } else {
         la.data = spec;
-        la.lines = 3ll * dp.hx;
+        la.lines = 3ll * layers * dp.hx;
         launch_lines<Real>(c, dp.ly, la);
     }
-    if (dp.three_d && !inverse) zpass();
+    for (int l = 0; dp.three_d && !inverse && l < layers; ++l) zpass(l);
 }
 
 template <typename Real, typename S>
@@ -1183,10 +1211,33 @@ void stack_eval_t(Stack &s, const S *const *src) {
     const unsigned xgroups = (unsigned)cdiv(dp.ny, dp.xr);
     const size_t xlds = (size_t)(dp.xr / 2) * dp.x_ls * sizeof(cplx<Real>);
     const int64_t ncv = (int64_t)c.nx * c.ny * c.nz;
-    cplx<Real> *sm = static_cast<cplx<Real> *>(s.spec_m), *sh = static_cast<cplx<Real> *>(s.spec_h);
+    cplx<Real> *sm = static_cast<cplx<Real> *>(s.spec_m);
+    cplx<Real> *sh = s.fused ? sm : static_cast<cplx<Real> *>(s.spec_h);
+    // layers on the common grid go through the x passes together
+    bool together = true, masked = false;
+    for (int l = 0; l < L; ++l) {
+        together = together && !s.conv_m[l];
+        masked = masked || s.layers[l]->d_mask;
+    }
     {
         Timed t(c, "stack_forward");
-        for (int l = 0; l < L; ++l) {
+        for (int l0 = 0; together && l0 < L; l0 += kStackPack) {
+            StackMag<Real, S> ms{};
+            const int nl = std::min(kStackPack, L - l0);
+            for (int l = 0; l < nl; ++l) {
+                ms.m[l] = src[l0 + l];
+                ms.mask[l] = s.layers[l0 + l]->d_mask;
+                ms.ms[l] = s.layers[l0 + l]->ms;
+            }
+            ms.nx = dp.nx;
+            ms.ny = dp.ny;
+            ms.nz = dp.nz;
+            ms.n = ncv;
+            ms.layer_stride = (int64_t)s.layer_spec;
+            launch_xfwd_stack<Real, S>(c, xa, ms, masked, sm + (uint64_t)l0 * s.layer_spec, xgroups, (unsigned)dp.nz,
+                                       (unsigned)nl, xlds);
+        }
+        for (int l = 0; !together && l < L; ++l) {
             Context &lc = *s.layers[l];
             cplx<Real> *spec = sm + (uint64_t)l * s.layer_spec;
             if (s.conv_m[l]) {
@@ -1204,10 +1255,22 @@ void stack_eval_t(Stack &s, const S *const *src) {
                     launch_xfwd<Real>(c, xa, ms, spec, xgroups, (unsigned)dp.nz, 3, xlds);
                 }
             }
-            stack_yz<Real>(s, spec, false);
         }
+        if (!s.fused) stack_yz<Real>(s, sm, L, false);
     }
-    {
+    if (s.fused) {
+        Timed t(c, "stack_tensor");
+        YStackArgs<Real> ya{};
+        ya.data = sm;
+        ya.tw = static_cast<const cplx<Real> *>(dp.tw_y);
+        ya.kern = static_cast<const Real *>(s.kern);
+        ya.ny = dp.ny;
+        ya.hx = dp.hx;
+        ya.kpw = s.kpw;
+        for (int d = 0; d < L; ++d)
+            for (int q = 0; q < L; ++q) ya.kernel[d][q] = s.pair[(size_t)d * L + q];
+        launch_ystack<Real>(c, dp.ly, L, ya);
+    } else {
         Timed t(c, "stack_tensor");
         StackTensorArgs<Real> ta{};
         ta.m = sm;
@@ -1231,10 +1294,24 @@ void stack_eval_t(Stack &s, const S *const *src) {
     }
     {
         Timed t(c, "stack_inverse");
-        for (int l = 0; l < L; ++l) {
+        if (!s.fused) stack_yz<Real>(s, sh, L, true);
+        for (int l0 = 0; together && l0 < L; l0 += kStackPack) {
+            StackField<Real> sf{};
+            const int nl = std::min(kStackPack, L - l0);
+            for (int l = 0; l < nl; ++l) {
+                sf.out[l] = static_cast<Real *>(s.layers[l0 + l]->hd);
+                sf.mask[l] = s.layers[l0 + l]->d_mask;
+            }
+            sf.nx = dp.nx;
+            sf.ny = dp.ny;
+            sf.n = ncv;
+            sf.layer_stride = (int64_t)s.layer_spec;
+            launch_xinv_stack<Real>(c, xa, sh + (uint64_t)l0 * s.layer_spec, sf, xgroups, (unsigned)dp.nz,
+                                    (unsigned)nl, xlds);
+        }
+        for (int l = 0; !together && l < L; ++l) {
             Context &lc = *s.layers[l];
-            cplx<Real> *spec = sh + (uint64_t)l * s.layer_spec;
-            stack_yz<Real>(s, spec, true);
+            const cplx<Real> *spec = sh + (uint64_t)l * s.layer_spec;
             const bool xfer = s.conv_h[l] != nullptr;
             Real *out = xfer ? static_cast<Real *>(s.conv_h[l]) : static_cast<Real *>(lc.hd);
             FieldSink<Real> sink{out, xfer ? nullptr : lc.d_mask, dp.nx, dp.ny, ncv};

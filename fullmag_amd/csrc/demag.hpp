@@ -257,7 +257,41 @@ struct YConvArgs {
     KernelView<Real> K;
 };
 
-// MAXB: kMaxBlock, or 1024 for lines too long for three of them in
+// Layers of a stack handed to one launch.
+constexpr int kStackPack = 8;
+
+// Ms m of up to kStackPack layers on the common grid (a mask where there is
+// one), and where their fields go.
+template <typename Real, typename S>
+struct StackMag {
+    const S *m[kStackPack];
+    const uint8_t *mask[kStackPack];
+    double ms[kStackPack];
+    int nx, ny, nz;
+    int64_t n;
+    int64_t layer_stride;  // complex elements per layer spectrum
+};
+template <typename Real>
+struct StackField {
+    Real *out[kStackPack];
+    const uint8_t *mask[kStackPack];
+    int nx, ny;
+    int64_t n;
+    int64_t layer_stride;
+};
+
+// Thin stack of L <= kStackFused layers: per kx, the layers' 3 L ky lines are
+// transformed, coupled by the pair kernels and transformed back in place.
+constexpr int kStackFused = 5;
+template <typename Real>
+struct YStackArgs {
+    cplx<Real> *data;       // [layer][c][kx][ky]
+    const cplx<Real> *tw;
+    const Real *kern;       // [kernel][kx][6][py / 2 + 1], the ky octant
+    int ny, hx, kpw;        // kx columns per workgroup
+    int kernel[kStackFused][kStackFused];  // of (dst, src)
+};
+
 // ---------------------------------------------------------------------------
 // kx slabs: y transforms and z convolution together
 // ---------------------------------------------------------------------------
@@ -360,6 +394,16 @@ template <typename Real>
 void launch_yconv(Context &c, const YConvArgs<Real> &ya);
 template <typename Real>
 void launch_film_tensor(Context &c, cplx<Real> *spec, const KernelView<Real> &K, int hx, int py, int64_t rows);
+// The stack's: x passes of `layers` <= kStackPack layers (spectra layer_stride
+// apart), and the coupled y pass.
+template <typename Real, typename S>
+void launch_xfwd_stack(Context &c, const XArgs<Real> &xa, const StackMag<Real, S> &sm, bool masked, cplx<Real> *spec,
+                       unsigned row_groups, unsigned planes, unsigned layers, size_t lds);
+template <typename Real>
+void launch_xinv_stack(Context &c, const XArgs<Real> &xa, const cplx<Real> *spec, const StackField<Real> &sf,
+                       unsigned row_groups, unsigned planes, unsigned layers, size_t lds);
+template <typename Real>
+void launch_ystack(Context &c, const LinePlan &lp, int layers, const YStackArgs<Real> &ya);
 // demag_s.hip: the slab kernel (slab_length(lp.n), 2 <= nz <= 8, a tensor).
 template <typename Real>
 void launch_slab(Context &c, const LinePlan &lp, const SlabArgs<Real> &sa);

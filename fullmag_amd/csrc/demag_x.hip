@@ -170,6 +170,30 @@ __global__ void __launch_bounds__(kMaxBlock) xfwd_multi(const XFwdPack<Real, Src
     xfwd_body<Real, Src, N>(p.a, p.src, p.spec, (int)(blockIdx.z % zdiv));
 }
 
+// Entry l of an argument array, l uniform in the workgroup (selects of
+// scalars: an index that is not a constant would put the array in scratch).
+template <typename T>
+__device__ __forceinline__ T entry_of(const T (&v)[kStackPack], int l) {
+    T r = v[0];
+#pragma unroll
+    for (int q = 1; q < kStackPack; ++q) r = q == l ? v[q] : r;
+    return r;
+}
+
+// Layer blockIdx.z / 3 of a stack, component blockIdx.z % 3: one launch for
+// all layers, whose single passes of a few microseconds leave the chip partly
+// idle (three 512 x 512 films, FP32: 3 x 6.7 us one by one).
+template <typename Real, typename S, bool GATHER, int N>
+__global__ void __launch_bounds__(kMaxBlock) xfwd_stack_kernel(XArgs<Real> a, StackMag<Real, S> p, cplx<Real> *spec) {
+    using Src = MagSource<Real, S, GATHER>;
+    const int l = (int)blockIdx.z / 3, c = (int)blockIdx.z - 3 * l;
+    const Src src{entry_of(p.m, l), GATHER ? entry_of(p.mask, l) : nullptr, nullptr, entry_of(p.ms, l),
+                  p.nx, p.ny, p.nz, p.n, nullptr};
+    cplx<Real> *sp = spec + l * p.layer_stride;
+    if constexpr (N > 0) xfwd_body<Real, Src, N>(a, src, sp, c);
+    else xfwd_body_rt<Real, Src>(a, src, sp, c);
+}
+
 // Inverse complex-to-real along x: Z_k = A_k + i B_k for k <= N/2 and the
 // Hermitian continuation A_{N-k} = conj A_k; z = IFFT(Z); rows a = Re z,
 // b = Im z.  Reads spec[c][z][k][y0..y0+xr-1].
@@ -377,6 +401,17 @@ __global__ void __launch_bounds__(kMaxBlock) xinv_kernel(XArgs<Real> a, const cp
     else xinv_body_rt<Real, Sink>(a, spec, sink, (int)blockIdx.z);
 }
 
+template <typename Real, int N>
+__global__ void __launch_bounds__(kMaxBlock)
+    xinv_stack_kernel(XArgs<Real> a, const cplx<Real> *spec, StackField<Real> p) {
+    using Sink = FieldSink<Real>;
+    const int l = (int)blockIdx.z / 3, c = (int)blockIdx.z - 3 * l;
+    const Sink sink{entry_of(p.out, l), entry_of(p.mask, l), p.nx, p.ny, p.n};
+    const cplx<Real> *sp = spec + l * p.layer_stride;
+    if constexpr (N > 0) xinv_body<Real, Sink, N>(a, sp, sink, c);
+    else xinv_body_rt<Real, Sink>(a, sp, sink, c);
+}
+
 template <typename Real, class Sink>
 struct XInvPack {
     XArgs<Real> a;
@@ -426,6 +461,29 @@ void launch_xinv(Context &c, const XArgs<Real> &xa, const cplx<Real> *spec, cons
     });
 }
 
+template <typename Real, typename S>
+void launch_xfwd_stack(Context &c, const XArgs<Real> &xa, const StackMag<Real, S> &sm, bool masked, cplx<Real> *spec,
+                       unsigned row_groups, unsigned planes, unsigned layers, size_t lds) {
+    const dim3 grid(row_groups, planes, 3 * layers), block((unsigned)((xa.xr / 2) * xa.lp.threads));
+    with_line(xa.lp, [&](auto NC) {
+        constexpr int N = decltype(NC)::value;
+        if (masked)
+            hipLaunchKernelGGL((xfwd_stack_kernel<Real, S, true, N>), grid, block, lds, c.stream, xa, sm, spec);
+        else
+            hipLaunchKernelGGL((xfwd_stack_kernel<Real, S, false, N>), grid, block, lds, c.stream, xa, sm, spec);
+    });
+}
+
+template <typename Real>
+void launch_xinv_stack(Context &c, const XArgs<Real> &xa, const cplx<Real> *spec, const StackField<Real> &sf,
+                       unsigned row_groups, unsigned planes, unsigned layers, size_t lds) {
+    const dim3 grid(row_groups, planes, 3 * layers), block((unsigned)((xa.xr / 2) * xa.lp.threads));
+    with_line(xa.lp, [&](auto NC) {
+        constexpr int N = decltype(NC)::value;
+        hipLaunchKernelGGL((xinv_stack_kernel<Real, N>), grid, block, lds, c.stream, xa, spec, sf);
+    });
+}
+
 using R = FM_REAL;
 #define FM_XFWD(SRC) \
     template void launch_xfwd<R, SRC>(Context &, const XArgs<R> &, const SRC &, cplx<R> *, unsigned, unsigned, \
@@ -442,6 +500,14 @@ FM_XFWD(SrcStageG)
 #else
 FM_XFWD(NewellSource)
 #endif
+template void launch_xfwd_stack<R, double>(Context &, const XArgs<R> &, const StackMag<R, double> &, bool, cplx<R> *,
+                                           unsigned, unsigned, unsigned, size_t);
+#ifdef FM_REAL_IS_FLOAT
+template void launch_xfwd_stack<R, float>(Context &, const XArgs<R> &, const StackMag<R, float> &, bool, cplx<R> *,
+                                          unsigned, unsigned, unsigned, size_t);
+#endif
+template void launch_xinv_stack<R>(Context &, const XArgs<R> &, const cplx<R> *, const StackField<R> &, unsigned,
+                                   unsigned, unsigned, size_t);
 template void launch_xinv<R>(Context &, const XArgs<R> &, const cplx<R> *, const FieldSink<R> &, unsigned, unsigned,
                              size_t);
 

@@ -221,6 +221,99 @@ __global__ void __launch_bounds__(fx_lanes(N) > 64 ? 3 * fx_lanes(N) : 256)
     yconv_fx_body<Real, N>(a);
 }
 
+// acc += k m and acc += i k m for real k.
+template <typename T>
+__device__ __forceinline__ void mad_re(cplx<T> &acc, T k, const cplx<T> &m) {
+    acc.x += k * m.x;
+    acc.y += k * m.y;
+}
+template <typename T>
+__device__ __forceinline__ void mad_im(cplx<T> &acc, T k, const cplx<T> &m) {
+    acc.x -= k * m.y;
+    acc.y += k * m.x;
+}
+
+// Thin stack: the 3 L ky lines of a kx column in one workgroup, transformed,
+// coupled and transformed back without leaving LDS.  As line passes and a
+// tensor pass the layers' spectra cross memory six times and the pair kernels
+// are read at every ky; here twice, and the kernels on the ky octant.  Three
+// 512 x 512 films, FP32: 3 x (6.6 + 6.1) + 25.9 us as three passes, 33.6 us
+// here; bound by each workgroup's chain of load, transforms, coupling and
+// store with two of them on a CU (the 513th column alone costs 6 us).
+template <typename Real, int N, int L>
+__global__ void __launch_bounds__(3 * L * fx_lanes(N) > 256 ? 3 * L * fx_lanes(N) : 256)
+    ystack_kernel(YStackArgs<Real> a) {
+    using C = cplx<Real>;
+    constexpr int T = fx_lanes(N), E = fx_elems(N), ls = fx_size(N), NL = 3 * L, HP = N / 2 + 1;
+    extern __shared__ unsigned char smem_raw[];
+    C *lds = reinterpret_cast<C *>(smem_raw);
+    const int tid = threadIdx.x, nthr = blockDim.x;
+    const int kx0 = blockIdx.x * a.kpw;
+    const int s = tid / T, t = tid % T, j = s / NL, kxl = kx0 + j;
+    const bool live = kxl < a.hx;
+    C *line = lds + s * ls;
+    C *g = a.data + ((int64_t)(s - j * NL) * a.hx + (live ? kxl : kx0)) * N;
+    {
+        C v[E];
+#pragma unroll
+        for (int e = 0; e < E / 2; ++e) {
+            const int i = t + e * T;
+            const C q = g[i < a.ny ? i : 0];
+            v[e] = i < a.ny ? q : C{Real(0), Real(0)};
+        }
+#pragma unroll
+        for (int e = E / 2; e < E; ++e) v[e] = C{Real(0), Real(0)};
+        fx_first_pass<Real, N>(line, t, v, a.tw, false);
+    }
+    fx_rest<Real, N>(line, t, a.tw, false);
+    __syncthreads();
+    for (int idx = tid; idx < a.kpw * N; idx += nthr) {
+        const int jc = idx / N, ky = idx % N, kx = kx0 + jc < a.hx ? kx0 + jc : kx0;
+        const bool lo = ky <= N / 2;
+        const Real sy = lo ? Real(1) : Real(-1);
+        const int64_t o = (int64_t)kx * 6 * HP + (lo ? ky : N - ky), ks = (int64_t)a.hx * 6 * HP;
+        C *col = lds + jc * NL * ls + fxslot<N>(ky);
+        C m[L][3], h[L][3];
+#pragma unroll
+        for (int l = 0; l < L; ++l)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                m[l][c] = col[(3 * l + c) * ls];
+                h[l][c] = {Real(0), Real(0)};
+            }
+#pragma unroll
+        for (int d = 0; d < L; ++d)
+#pragma unroll
+            for (int q = 0; q < L; ++q) {
+                C *hh = h[d];
+                const C *mm = m[q];
+                const Real *K = a.kern + (q == d ? 0 : a.kernel[d][q]) * ks + o;  // 0: self
+                const Real kxx = K[0], kyy = K[HP], kzz = K[2 * HP], kxy = sy * K[3 * HP];
+                const Real kxz = K[4 * HP], kyz = sy * K[5 * HP];
+                mad_re(hh[0], kxx, mm[0]);
+                mad_re(hh[0], kxy, mm[1]);
+                mad_im(hh[0], kxz, mm[2]);
+                mad_re(hh[1], kxy, mm[0]);
+                mad_re(hh[1], kyy, mm[1]);
+                mad_im(hh[1], kyz, mm[2]);
+                mad_im(hh[2], kxz, mm[0]);
+                mad_im(hh[2], kyz, mm[1]);
+                mad_re(hh[2], kzz, mm[2]);
+            }
+#pragma unroll
+        for (int l = 0; l < L; ++l)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) col[(3 * l + c) * ls] = {-h[l][c].x, -h[l][c].y};
+    }
+    __syncthreads();
+    C v[E];
+    fx_load<Real, N>(line, t, v);
+    fx_first_pass<Real, N>(line, t, v, a.tw, true);
+    fx_rest_put<Real, N, 2>(line, t, a.tw, true, [&](int i, const C &q) {
+        if (live && i < a.ny) g[i] = q;
+    });
+}
+
 // Thin film, split form: the three components' ky spectra (all py entries,
 // rows `rows` apart) are multiplied by the tensor at kz = 0 in place; the y
 // transforms run before and after as line passes.  For films whose three
@@ -306,6 +399,28 @@ void launch_yconv(Context &c, const YConvArgs<Real> &ya) {
 }
 
 template <typename Real>
+void launch_ystack(Context &c, const LinePlan &lp, int layers, const YStackArgs<Real> &ya) {
+    const dim3 grid((unsigned)cdiv(ya.hx, ya.kpw)), block((unsigned)(3 * layers * ya.kpw * lp.threads));
+    const size_t lds = (size_t)3 * layers * ya.kpw * line_slots(lp) * sizeof(cplx<Real>);
+    with_line(lp, [&](auto NC) {
+        constexpr int N = decltype(NC)::value;
+        auto launch = [&](auto lc) {
+            constexpr int L = decltype(lc)::value;
+            // what the plan's rule can choose (160 KiB of LDS)
+            if constexpr (N > 0 && 3 * L * fx_lanes(N) <= 1024 && 3 * L * fx_size(N) * sizeof(cplx<Real>) <= 163840)
+                hipLaunchKernelGGL((ystack_kernel<Real, N, L>), grid, block, lds, c.stream, ya);
+        };
+        switch (layers) {
+            case 1: launch(std::integral_constant<int, 1>{}); break;
+            case 2: launch(std::integral_constant<int, 2>{}); break;
+            case 3: launch(std::integral_constant<int, 3>{}); break;
+            case 4: launch(std::integral_constant<int, 4>{}); break;
+            default: launch(std::integral_constant<int, 5>{}); break;
+        }
+    });
+}
+
+template <typename Real>
 void launch_film_tensor(Context &c, cplx<Real> *spec, const KernelView<Real> &K, int hx, int py, int64_t rows) {
     const dim3 g1((unsigned)cdiv((int64_t)hx * py, 256));
     launch_rec(c, nullptr, g1, dim3(256), 0, 1, K, [&] {
@@ -316,6 +431,7 @@ void launch_film_tensor(Context &c, cplx<Real> *spec, const KernelView<Real> &K,
 using R = FM_REAL;
 template void launch_lines<R>(Context &, const LinePlan &, LineArgs<R>);
 template void launch_yconv<R>(Context &, const YConvArgs<R> &);
+template void launch_ystack<R>(Context &, const LinePlan &, int, const YStackArgs<R> &);
 template void launch_film_tensor<R>(Context &, cplx<R> *, const KernelView<R> &, int, int, int64_t);
 
 }  // namespace fm

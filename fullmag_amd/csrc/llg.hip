@@ -201,8 +201,9 @@ struct Driver {
     }
 
     template <typename Src, typename Out>
-    void stage(const Src *src, Real *kout, Out *out, std::initializer_list<std::pair<int, double>> prev, double anew,
-               double dt) {
+    StageArgs<State, Real, Src, Out> stage_args(const Src *src, Real *kout, Out *out,
+                                                std::initializer_list<std::pair<int, double>> prev, double anew,
+                                                double dt) {
         StageArgs<State, Real, Src, Out> a = args<Src, Out>(src, hd());
         a.kout = kout;
         a.out = out;
@@ -213,6 +214,13 @@ struct Driver {
         }
         a.anew = anew;
         a.dt = dt;
+        return a;
+    }
+
+    template <typename Src, typename Out>
+    void stage(const Src *src, Real *kout, Out *out, std::initializer_list<std::pair<int, double>> prev, double anew,
+               double dt) {
+        const StageArgs<State, Real, Src, Out> a = stage_args<Src, Out>(src, kout, out, prev, anew, dt);
         Timed t(c, "llg_stage");
         const dim3 g(grid_stage()), b(kBlock);
         // the uniform kernel (or its multi-instance twin while a batch, which
@@ -793,6 +801,24 @@ double integrator_probe_ms(Context &c, int reps) {
     return (double)ms;
 }
 
+// One stage of every layer of a stack (equal grids), kStagePack to a launch.
+template <typename State, typename Real, typename Src, typename Out, int NPREV, bool M0_IS_SRC, class F>
+void stage_pack(std::vector<Driver<State, Real>> &d, F &&args_of) {
+    const bool masked = d[0].c.d_mask != nullptr;
+    for (size_t l0 = 0; l0 < d.size(); l0 += kStagePack) {
+        StagePack<State, Real, Src, Out> p{};
+        const size_t nl = std::min<size_t>(kStagePack, d.size() - l0);
+        for (size_t l = 0; l < nl; ++l) p.a[l] = args_of(d[l0 + l]);
+        const dim3 g(d[0].grid_stage(), (unsigned)nl), b(kBlock);
+        if (masked)
+            hipLaunchKernelGGL((stage_uniform_pack<State, Real, Src, Out, NPREV, M0_IS_SRC, true>), g, b, 0,
+                               d[0].c.stream, p);
+        else
+            hipLaunchKernelGGL((stage_uniform_pack<State, Real, Src, Out, NPREV, M0_IS_SRC, false>), g, b, 0,
+                               d[0].c.stream, p);
+    }
+}
+
 // Heun steps of a stack (crates/fullmag-runner/src/multilayer_reference.rs:
 // 543-589): every stage evaluates all layers, then the coupled demag of all
 // layers at the new points, then the next stage.  The stats pass at the new
@@ -817,15 +843,38 @@ int stack_step_t(Stack &s, double dt, uint64_t nsteps, fullmag_fdm_step_stats *s
         eval(true);
         for (Context *c : s.layers) c->pre_valid = false;
     }
+    // Layers of one grid whose stages are the uniform kernel's, all with or
+    // all without a mask, share each stage's launch (with per-kernel timing,
+    // which is kept by layer, they do not).
+    const FieldArgs f0 = field_args(*s.layers[0]);
+    bool together = L > 1;
+    for (Context *c : s.layers) {
+        const FieldArgs f = field_args(*c);
+        together = together && c->demag && !c->timing && !f.tier_ex && stage_uniform_ok(f, c->hd, 1) &&
+                   f.nx == f0.nx && f.ny == f0.ny && f.nz == f0.nz && (f.mask != nullptr) == (f0.mask != nullptr) &&
+                   stage_blocks(*c) == stage_blocks(*s.layers[0]);
+    }
     for (uint64_t k = 0; k < nsteps; ++k) {
+        bool fresh = true;  // every layer's predictor is still to be computed
+        for (Context *c : s.layers) fresh = fresh && !(c->pre_valid && c->pre_dt == dt);
+        if (together && fresh)
+            stage_pack<State, Real, State, Real, 0, true>(d, [&](Driver<State, Real> &q) {
+                return q.template stage_args<State, Real>(q.m(), q.k(0), q.mt(0), {}, 1.0, dt);
+            });
         for (size_t l = 0; l < L; ++l) {
             Context &c = *s.layers[l];
-            if (!(c.pre_valid && c.pre_dt == dt))
+            if (!(together && fresh) && !(c.pre_valid && c.pre_dt == dt))
                 d[l].template stage<State, Real>(d[l].m(), d[l].k(0), d[l].mt(0), {}, 1.0, dt);
             c.pre_valid = false;
         }
         eval(false);
-        for (size_t l = 0; l < L; ++l) d[l].template stage<Real, State>(d[l].mt(0), nullptr, d[l].m(), {{0, 0.5}}, 0.5, dt);
+        if (together)
+            stage_pack<State, Real, Real, State, 1, false>(d, [&](Driver<State, Real> &q) {
+                return q.template stage_args<Real, State>(q.mt(0), nullptr, q.m(), {{0, 0.5}}, 0.5, dt);
+            });
+        else
+            for (size_t l = 0; l < L; ++l)
+                d[l].template stage<Real, State>(d[l].mt(0), nullptr, d[l].m(), {{0, 0.5}}, 0.5, dt);
         eval(true);
     }
     for (size_t l = 0; l < L; ++l) {
