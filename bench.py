@@ -67,6 +67,7 @@ def alg_bytes(nx, ny, nz, q, r):
         "demag_x_r2c": 3 * n * (q + r) / 2 + 3 * a1 * c,
         "demag_y_fwd": 3 * a1 * c + 3 * a2 * c,
         "demag_z_conv": 3 * a2 * c + kern * r + 3 * a2 * c,
+        "demag_yz_class": 3 * a1 * c + kern * r + 3 * a2 * c,
         "demag_y_inv": 3 * a2 * c + 3 * a1 * c,
         "demag_x_c2r": 3 * a1 * c + 3 * n * r,
         # corrector: mt, Hd, m0, k1 -> m (the predictor runs in the stats

@@ -42,7 +42,7 @@ struct DemagTuning {
     int z_tile = 0;    // > 0: at most this many columns per long-z (LDS line) workgroup
     int zc = 0;        // z planes per workgroup of the cell kernels (0: automatic)
     int y_split = 0;   // 1: thin-film y convolution as separate line and tensor passes
-    int slab = 160;    // y and z passes in one kernel for kx slabs of at most this many KB of LDS (0: off)
+    int slab = 160;    // y and z passes in one kernel for kx slabs of at most this many KB of LDS (0: off, ky classes too)
     int pad = 1;       // 0: transform lengths 2n even where a longer scheduled length is faster
 };
 
@@ -58,6 +58,7 @@ void parse_tuning_string(DemagTuning &t, const char *text);
 // Films: the four components of an entry together.
 struct KernLayout {
     int64_t skx = 0, soy = 0, soz = 0, odd = 0, sc = 1;
+    int cls = 1, yw = 0;  // oy at (oy mod cls) yw + oy / cls, the ky classes of a row one after the other
 };
 
 struct DemagPlan {
@@ -83,6 +84,9 @@ struct DemagPlan {
     // device buffers (element type depends on Real)
     void *tw_x = nullptr, *tw_y = nullptr, *tw_z = nullptr;
     void *spec = nullptr;
+    void *xspec = nullptr;  // x passes' spectrum of rows of xrows entries (ky classes)
+    void *tw_c = nullptr;   // roots of length py / cls
+    int cls = 1, xrows = 0;  // ky classes (1: none), fixed at set-up
     void *kern = nullptr;
     uint64_t spec_elems = 0;  // complex elements
     uint64_t kern_elems = 0;  // real elements

@@ -20,7 +20,8 @@
 // kz = 0, inverse y in one kernel), x inv.
 //
 // Spectrum layout: spec[c][z][kx][ky] with z < nz (3-D) or a single plane
-// (2-D), kx <= nx, ky < pitch (2ny in 3-D, ny in 2-D).
+// (2-D), kx <= nx, ky < pitch (2ny in 3-D, ny in 2-D).  Slabs split into ky
+// classes have a second one of pitch ny for the x passes.
 // The Newell spectra are real (the padded kernel is even or odd along every
 // axis); the tensor is stored on the non-negative octant as
 // blocks per (kx, ky) column (kz <= nz, ky <= ny, kern_at) and mirrored with
@@ -261,6 +262,24 @@ bool use_slab(const DemagPlan &dp) {
     return sizeof(Real) == 4 && 10 * dp.py >= 9 * rounds * cols;
 }
 
+// Whether a slab's ky classes go through the y transform and the z
+// convolution in one kernel each: the plan's choice (class_rule, fixed at set-up
+// with the tensor's layout), its second spectrum, and the knobs.
+template <typename Real>
+bool use_class(const DemagPlan &dp) {
+    return dp.cls > 1 && dp.xspec && dp.ly.fixed && dp.tune.slab > 0;
+}
+
+// The x passes' spectrum.
+template <typename Real>
+SpecGeom x_geom(const DemagPlan &dp) {
+    return SpecGeom{dp.hx, dp.three_d ? dp.nz : 1, use_class<Real>(dp) ? dp.xrows : dp.rows};
+}
+template <typename Real>
+cplx<Real> *x_spec(const DemagPlan &dp) {
+    return static_cast<cplx<Real> *>(use_class<Real>(dp) ? dp.xspec : dp.spec);
+}
+
 // x R2C of Ms src, the y and z transforms with the tensor product and the
 // inverse y and z transforms: everything up to the x C2R, in the spectrum.
 template <typename Real, typename S>
@@ -275,7 +294,7 @@ void demag_transform_t(Context &c, const S *src, const XArgs<Real> &xa, unsigned
                                     (int64_t)c.n, weight_ms ? phi_array<Real>(c) : nullptr};
         Timed t(c, "demag_x_r2c");
         auto launch = [&](const auto &src_v) {
-            launch_xfwd<Real>(c, xa, src_v, spec, xgroups, (unsigned)dp.nz, 3, xlds);
+            launch_xfwd<Real>(c, xa, src_v, x_spec<Real>(dp), xgroups, (unsigned)dp.nz, 3, xlds);
         };
         if (ms.mask || ms.ms_cell || ms.phi)
             launch(MagSource<Real, S, true>{ms.m, ms.mask, ms.ms_cell, ms.ms, ms.nx, ms.ny, ms.nz, ms.n, ms.phi});
@@ -283,7 +302,39 @@ void demag_transform_t(Context &c, const S *src, const XArgs<Real> &xa, unsigned
             launch(ms);
     }
     const KernelView<Real> K = kview<Real>(c);
-    if (dp.three_d && use_slab<Real>(dp)) {
+    if (use_class<Real>(dp)) {
+        SlabArgs<Real> sa{};
+        sa.data = spec;
+        sa.tw = static_cast<const cplx<Real> *>(dp.tw_y);
+        sa.twz = static_cast<const cplx<Real> *>(dp.tw_z);
+        sa.twp = static_cast<const cplx<Real> *>(dp.tw_c);
+        sa.nz = dp.nz;
+        sa.ny = dp.ny;
+        sa.hx = dp.hx;
+        sa.pitch = dp.rows;
+        sa.plane_stride = (int64_t)dp.hx * dp.rows;
+        sa.in = static_cast<const cplx<Real> *>(dp.xspec);
+        sa.in_pitch = dp.xrows;
+        sa.in_plane = (int64_t)dp.hx * dp.xrows;
+        sa.K = K;
+        {
+            Timed t(c, "demag_yz_class");
+            launch_class<Real>(c, dp.ly, sa);
+        }
+        LineArgs<Real> la{};
+        la.in = spec;
+        la.in_pitch = dp.rows;
+        la.data = static_cast<cplx<Real> *>(dp.xspec);
+        la.line_pitch = dp.xrows;
+        la.tw = sa.tw;
+        la.lp = dp.ly;
+        la.lines = 3ll * dp.nz * dp.hx;
+        la.n_in = dp.py;
+        la.n_out = dp.ny;
+        la.inverse = 1;
+        Timed t(c, "demag_y_inv");
+        launch_class_inverse<Real>(c, dp.ly, la);
+    } else if (dp.three_d && use_slab<Real>(dp)) {
         SlabArgs<Real> sa{};
         sa.data = spec;
         sa.tw = static_cast<const cplx<Real> *>(dp.tw_y);
@@ -397,8 +448,8 @@ void demag_transform_t(Context &c, const S *src, const XArgs<Real> &xa, unsigned
 template <typename Real, typename S>
 void demag_eval_t(Context &c, const S *src, Real *out, bool weight_ms, int phase) {
     DemagPlan &dp = c.dp;
-    cplx<Real> *spec = static_cast<cplx<Real> *>(dp.spec);
-    const SpecGeom g{dp.hx, dp.three_d ? dp.nz : 1, dp.rows};
+    cplx<Real> *spec = x_spec<Real>(dp);
+    const SpecGeom g = x_geom<Real>(dp);
     const size_t ce = sizeof(cplx<Real>);
     XArgs<Real> xa{};
     xa.tw = static_cast<const cplx<Real> *>(dp.tw_x);
@@ -451,12 +502,13 @@ template <typename Real>
 bool upload_twiddles(Context &c) {
     DemagPlan &dp = c.dp;
     std::vector<cplx<Real>> all;
-    for (int n : {dp.px, dp.py, dp.three_d ? dp.pz : 1})
+    for (int n : {dp.px, dp.py, dp.three_d ? dp.pz : 1, dp.cls > 1 ? dp.py / dp.cls : 1})
         for (const cplx<double> &w : twiddle_table(n)) all.push_back({(Real)w.x, (Real)w.y});
     const size_t bytes = all.size() * sizeof(cplx<Real>);
     if (!ctx_alloc(c, &dp.tw_x, bytes, "twiddle tables")) return false;
     dp.tw_y = static_cast<cplx<Real> *>(dp.tw_x) + dp.px;
     dp.tw_z = static_cast<cplx<Real> *>(dp.tw_y) + dp.py;
+    dp.tw_c = static_cast<cplx<Real> *>(dp.tw_z) + (dp.three_d ? dp.pz : 1);
     return ctx_upload(c, dp.tw_x, all.data(), bytes, "hipMemcpy(twiddles)", c.last_error);
 }
 
@@ -678,6 +730,21 @@ bool upload_kern(Context &c, const std::vector<double> &kern) {
     return ctx_upload(c, dp.kern, f.data(), bytes, "hipMemcpy(tensor)", c.last_error);
 }
 
+// Whether the plan splits its slabs into ky classes: short z lines and a
+// scheduled y length of 320 to 1024 whose slab does not fit the slab kernel.
+// us per Heun step, separate passes and classes: mixed 512x512x4 187.1 and
+// 167.9, 400x400x2 115.8 and 105.0, 300x384x5 145.2 and 133.0, 250x150x6 102.5
+// and 94.8, 100x300x8 104.3 and 96.6, 512x512x8 348.7 and 344.5; FP64
+// 512x512x4 330.9 and 300.3, 200x400x3 126.5 and 118.0.  FP64 with more than
+// four layers needs a component per lane: 512x512x8 651 and 670.  Where both
+// fit, the slab kernel mostly wins (mixed 128x200x7 76.9 against 80.6,
+// 500x250x8 175.7 against 186.5; 256x224x7 119.5 against 108.2).
+template <typename Real>
+bool class_rule(const DemagPlan &dp) {
+    return dp.three_d && !dp.projection && dp.nz >= 2 && dp.nz <= (sizeof(Real) == 4 ? 8 : 4) && dp.ly.fixed &&
+           class_length(dp.py) && dp.tune.slab > 0 && !use_slab<Real>(dp);
+}
+
 // Launch geometry of the planned lines (no allocation): x rows per
 // workgroup, y lines per workgroup, long-z tile, thin-film y convolution
 // form.  `keep_split` >= 0 requires the thin-film form to stay as it is (a
@@ -689,9 +756,12 @@ bool plan_geometry(DemagPlan &dp, std::string &err, int keep_split = -1) {
         const int64_t ly = dp.py / 2 + 1, nzo = dp.kz_n;
         KernLayout &l = dp.kl;
         const bool planes = dp.three_d && dp.pz <= z_reg_max<Real>();
-        l.sc = planes ? ly : 1;
+        l.cls = dp.cls;
+        l.yw = (int)cdiv(ly, (int64_t)dp.cls);
+        const int64_t w = (int64_t)dp.cls * l.yw;
+        l.sc = planes ? w : 1;
         l.soy = planes ? 1 : dp.kcomp;
-        l.odd = ly * dp.kcomp;
+        l.odd = w * dp.kcomp;
         l.soz = 2 * l.odd;
         l.skx = nzo * l.odd;
     }
@@ -745,9 +815,10 @@ bool plan_geometry(DemagPlan &dp, std::string &err, int keep_split = -1) {
 }
 
 template <typename Real>
-bool setup_t(Context &c, const fullmag_fdm_plan_desc &plan) {
+bool setup_tensor_t(Context &c, const fullmag_fdm_plan_desc &plan) {
     DemagPlan &dp = c.dp;
     const size_t ce = sizeof(cplx<Real>);
+    dp.cls = class_rule<Real>(dp) ? kClasses : 1;
     if (!plan_geometry<Real>(dp, c.last_error)) return false;
     if (!upload_twiddles<Real>(c)) return false;
     dp.spec_elems = 3ull * (dp.three_d ? dp.nz : 1) * dp.hx * dp.rows;
@@ -775,6 +846,24 @@ bool setup_t(Context &c, const fullmag_fdm_plan_desc &plan) {
     }
     (void)hipFree(spec);
     return ok;
+}
+
+// The tensor first, then the classes' second spectrum: without memory for it
+// the separate passes run.
+template <typename Real>
+bool setup_t(Context &c, const fullmag_fdm_plan_desc &plan) {
+    DemagPlan &dp = c.dp;
+    if (!setup_tensor_t<Real>(c, plan)) return false;
+    if (dp.cls > 1) {
+        dp.xrows = dp.ny + (dp.ny & 1);
+        const std::string err = c.last_error;
+        if (!ctx_alloc(c, &dp.xspec, 3ull * dp.nz * dp.hx * dp.xrows * sizeof(cplx<Real>), "demag spectrum")) {
+            (void)hipGetLastError();
+            dp.xspec = nullptr;
+            c.last_error = err;
+        }
+    }
+    return true;
 }
 
 }  // namespace

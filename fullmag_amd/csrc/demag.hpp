@@ -52,9 +52,15 @@ struct KernelView {
     double kxs = 0, kys = 0, kzs = 0;  // 2 pi / (p d) per axis (projection)
 };
 
+// Position of oy within a row of the octant tensor (KernLayout): residue
+// classes mod cls (a power of two) one after the other.
+__host__ __device__ __forceinline__ int kern_y(const KernLayout &l, int oy) {
+    return (oy & (l.cls - 1)) * l.yw + oy / l.cls;
+}
+
 // Entry (kx, oy, oz), component c of the octant tensor (KernLayout).
 __host__ __device__ __forceinline__ int64_t kern_at(const KernLayout &l, int c, int oz, int kx, int oy) {
-    return kx * l.skx + oy * l.soy + ((oz & 1) ? l.odd : 0) + (oz >> 1) * l.soz + c * l.sc;
+    return kx * l.skx + kern_y(l, oy) * l.soy + ((oz & 1) ? l.odd : 0) + (oz >> 1) * l.soz + c * l.sc;
 }
 
 // t = (xx, yy, zz, xy, xz, yz) at frequency (kx, ky, kz); kx <= nx.
@@ -242,6 +248,8 @@ struct LineArgs {
     int n_in, n_out;
     int inverse;
     int iters;          // line_pipe_kernel: line groups per workgroup
+    const cplx<Real> *in;  // inverse from ky classes: rows of a class's entries after another's, in_pitch apart
+    int64_t in_pitch;
 };
 
 // Thin film: per kx, the three components' ky lines (ny of 2ny inputs) are
@@ -302,7 +310,18 @@ struct SlabArgs {
     int nz, ny, hx, pitch;
     int64_t plane_stride;        // between the (component, z) planes of the spectrum
     KernelView<Real> K;
+    // ky classes (class_kernel): the x passes' spectrum, read, and the roots of
+    // length py / kClasses
+    const cplx<Real> *in, *twp;
+    int in_pitch;
+    int64_t in_plane;
 };
+// Residue classes of ky that class_kernel splits a slab into, and the padded y
+// lengths it takes.
+constexpr int kClasses = 4;
+constexpr bool class_length(int n) {
+    return n % kClasses == 0 && fx_has(n) && fx_lanes(n) >= 32 && fx_has(n / kClasses) && fx_lanes(n / kClasses) <= 16;
+}
 // Padded y lengths with a slab kernel: 24 lines of 32 lanes are 768.
 constexpr bool slab_length(int n) { return fx_has(n) && fx_lanes(n) <= 32; }
 
@@ -407,6 +426,10 @@ void launch_ystack(Context &c, const LinePlan &lp, int layers, const YStackArgs<
 // demag_s.hip: the slab kernel (slab_length(lp.n), 2 <= nz <= 8, a tensor).
 template <typename Real>
 void launch_slab(Context &c, const LinePlan &lp, const SlabArgs<Real> &sa);
+template <typename Real>
+void launch_class(Context &c, const LinePlan &lp, const SlabArgs<Real> &sa);
+template <typename Real>
+void launch_class_inverse(Context &c, const LinePlan &lp, const LineArgs<Real> &la);
 // demag_z.hip: the register z convolution (pz <= 16) and the longer z lines
 // (convolution, or plain transforms of `comps` components).
 template <typename Real>

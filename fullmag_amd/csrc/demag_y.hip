@@ -37,7 +37,7 @@ __global__ void __launch_bounds__(kMaxBlock) line_kernel(LineArgs<Real> a) {
 // holds no prefetch registers and more waves share each SIMD instead.
 // Forward: N / 2 inputs per line (RAGGED: a.n_in, fewer), the rest zero, and N
 // outputs; inverse: N inputs, a.n_out <= N / 2 outputs.
-template <typename Real, int N, bool INV, bool PIPE, bool RAGGED>
+template <typename Real, int N, bool INV, bool PIPE, bool RAGGED, bool CLS = false>
 __device__ __forceinline__ void line_pipe_body(const LineArgs<Real> &a) {
     constexpr int T = fx_lanes(N), E = fx_elems(N);
     constexpr int G = T >= 64 ? 1 : 64 / T;
@@ -47,6 +47,10 @@ __device__ __forceinline__ void line_pipe_body(const LineArgs<Real> &a) {
     cplx<Real> *lds = reinterpret_cast<cplx<Real> *>(smem_raw);
     const int j = (int)threadIdx.x / T, t = (int)threadIdx.x - j * T;
     cplx<Real> *line = lds + j * fx_size(N);
+    // CLS: lane t takes the first pass of lane t1, so that neighbouring lanes
+    // read neighbouring entries of one class
+    constexpr int TC = T / kClasses;
+    const int t1 = CLS ? (t % TC) * kClasses + t / TC : t;
     const int64_t first = (int64_t)blockIdx.x * (PIPE ? a.iters : 1) * G + j;
     cplx<Real> buf[NI];
     auto fetch = [&](int64_t l) {
@@ -55,7 +59,13 @@ __device__ __forceinline__ void line_pipe_body(const LineArgs<Real> &a) {
         // a select becomes a branch, and the join waits for the loads
         // issued before it)
         const cplx<Real> *g = a.data + (l < a.lines ? l : 0) * a.line_pitch;
-        if constexpr (!RAGGED) {
+        if constexpr (CLS) {
+            // element i is entry i / kClasses of class i mod kClasses
+            static_assert(T % kClasses == 0, "a lane stays in its class");
+            g = a.in + (l < a.lines ? l : 0) * a.in_pitch + (t / TC) * (N / kClasses) + t % TC;
+#pragma unroll
+            for (int e = 0; e < NI; ++e) buf[e] = g[e * TC];
+        } else if constexpr (!RAGGED) {
 #pragma unroll
             for (int e = 0; e < NI; ++e) buf[e] = g[t + e * T];
         } else {
@@ -78,7 +88,7 @@ __device__ __forceinline__ void line_pipe_body(const LineArgs<Real> &a) {
 #pragma unroll
         for (int e = 0; e < E; ++e) v[e] = e < NI ? buf[e] : cplx<Real>{Real(0), Real(0)};
         if (PIPE && it + 1 < iters) fetch(l + G);
-        fx_first_pass<Real, N>(line, t, v, a.tw, INV);
+        fx_first_pass<Real, N>(line, t1, v, a.tw, INV);
         // the last pass stores from registers: consecutive lanes hold
         // consecutive elements, and the inverse produces only the half of
         // them that is kept
@@ -99,6 +109,16 @@ template <typename Real, int N, bool INV, bool PIPE, bool RAGGED>
 __global__ void __launch_bounds__(256) line_pipe_multi(const LineArgs<Real> *tab, int zdiv) {
     const LineArgs<Real> a = tab[blockIdx.z / zdiv];
     line_pipe_body<Real, N, INV, PIPE, RAGGED>(a);
+}
+
+template <typename Real, int N>
+__global__ void __launch_bounds__(256) line_class_kernel(LineArgs<Real> a) {
+    line_pipe_body<Real, N, true, false, false, true>(a);
+}
+template <typename Real, int N>
+__global__ void __launch_bounds__(256) line_class_multi(const LineArgs<Real> *tab, int zdiv) {
+    const LineArgs<Real> a = tab[blockIdx.z / zdiv];
+    line_pipe_body<Real, N, true, false, false, true>(a);
 }
 
 // MAXB: kMaxBlock, or 1024 for lines too long for three of them in
@@ -380,6 +400,21 @@ void launch_lines(Context &c, const LinePlan &lp, LineArgs<Real> la) {
 }
 
 template <typename Real>
+void launch_class_inverse(Context &c, const LinePlan &lp, const LineArgs<Real> &la) {
+    with_line(lp, [&](auto NC) {
+        constexpr int N = decltype(NC)::value;
+        if constexpr (class_length(N)) {
+            constexpr int T = fx_lanes(N), G = T >= 64 ? 1 : 64 / T;
+            const dim3 grid((unsigned)cdiv(la.lines, (int64_t)G)), block((unsigned)(G * T));
+            const size_t lds = (size_t)G * fx_size(N) * sizeof(cplx<Real>);
+            launch_rec(c, reinterpret_cast<const void *>(&line_class_multi<Real, N>), grid, block, lds, 1, la, [&] {
+                hipLaunchKernelGGL((line_class_kernel<Real, N>), grid, block, lds, c.stream, la);
+            });
+        }
+    });
+}
+
+template <typename Real>
 void launch_yconv(Context &c, const YConvArgs<Real> &ya) {
     const dim3 grid((unsigned)cdiv(ya.hx, ya.kpw)), block((unsigned)(3 * ya.kpw * ya.lp.threads));
     const size_t lds = (size_t)3 * ya.kpw * line_slots(ya.lp) * sizeof(cplx<Real>);
@@ -430,6 +465,7 @@ void launch_film_tensor(Context &c, cplx<Real> *spec, const KernelView<Real> &K,
 
 using R = FM_REAL;
 template void launch_lines<R>(Context &, const LinePlan &, LineArgs<R>);
+template void launch_class_inverse<R>(Context &, const LinePlan &, const LineArgs<R> &);
 template void launch_yconv<R>(Context &, const YConvArgs<R> &);
 template void launch_ystack<R>(Context &, const LinePlan &, int, const YStackArgs<R> &);
 template void launch_film_tensor<R>(Context &, cplx<R> *, const KernelView<R> &, int, int, int64_t);

@@ -54,7 +54,7 @@ __device__ __forceinline__ void zreg_body(const ZArgs<Real> &a) {
     const Real sy = ylo ? Real(1) : Real(-1);
     const int kx0 = __builtin_amdgcn_readfirstlane(kx);
     const Real *kb = a.K.k + kx0 * a.K.l.skx;
-    const uint32_t ko = (uint32_t)((kx - kx0) * (int)a.K.l.skx + (ylo ? ky : a.py - ky));
+    const uint32_t ko = (uint32_t)((kx - kx0) * (int)a.K.l.skx + kern_y(a.K.l, ylo ? ky : a.py - ky));
     auto load = [&](Real (*t)[6], int n, int64_t off) {
 #pragma unroll
         for (int i = 0; i < n; ++i)
@@ -151,7 +151,7 @@ __device__ __forceinline__ void zreg3_body(const ZArgs<Real> &a) {
     const bool ylo = ky <= a.K.ny;
     const int kx0 = __builtin_amdgcn_readfirstlane(kx);
     const Real *kb = a.K.k + kx0 * a.K.l.skx;
-    const uint32_t ko = (uint32_t)((kx - kx0) * (int)a.K.l.skx + (ylo ? ky : a.py - ky));
+    const uint32_t ko = (uint32_t)((kx - kx0) * (int)a.K.l.skx + kern_y(a.K.l, ylo ? ky : a.py - ky));
     const Real sy = ylo || c != 1 ? Real(1) : Real(-1), sz = c == 2 ? Real(-1) : Real(1);
     auto half = [&](C *v, int odd, int n, int64_t off) {
         Real t[NE][3];

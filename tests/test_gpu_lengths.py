@@ -73,3 +73,30 @@ def test_unpadded_schedule_agrees(fa, monkeypatch, cells):
 def test_slab_and_separate_passes(fa, monkeypatch, nx, ny, nz, precision):
     for tune in ("", "slab=0"):
         assert field_error(fa, monkeypatch, (nx, ny, nz), precision, tune=tune) <= BAR.get(precision, 2e-6)
+
+
+# ky classes of a slab: every layer count, P = 80, 160, 192, 224 and 256 entries
+# per class, ny at, below and far below half the padded length
+@pytest.mark.parametrize("precision", ["double", "mixed"])
+@pytest.mark.parametrize("nz", [2, 3, 4, 5, 6, 7, 8])
+@pytest.mark.parametrize("nx,ny", [(5, 149), (9, 320), (6, 384), (11, 385), (4, 449), (7, 512)])
+def test_class_and_separate_passes(fa, monkeypatch, nx, ny, nz, precision):
+    for tune in ("", "slab=0"):
+        assert field_error(fa, monkeypatch, (nx, ny, nz), precision, tune=tune) <= BAR[precision]
+
+
+@pytest.mark.parametrize("precision", ["double", "mixed", "single"])
+def test_classes_off_at_run_time(fa, precision):
+    """The tensor keeps its class order when a schedule turns the classes off."""
+    cells = (6, 300, 3)
+    n = int(np.prod(cells))
+    gpu = fa.NativeFdmBackend(fa.FdmPlan(cells=cells, cell_size=(4e-9, 3e-9, 2e-9),
+                                         initial_magnetization=fa.generate_random_unit_vectors(7, n),
+                                         saturation_magnetisation=8e5, exchange_stiffness=1e-11, damping=0.1,
+                                         precision=precision, demag_kernel="device"))
+    h = gpu.copy_h_demag()
+    for tune in ("slab=0", "fixed=0", "slab=160"):
+        gpu.set_schedule(tune)
+        gpu.refresh_observables()
+        assert np.abs(gpu.copy_h_demag() - h).max() <= BAR.get(precision, 2e-6) * np.abs(h).max()
+    gpu.close()
