@@ -52,6 +52,15 @@ __device__ __forceinline__ void xfwd_body_rt(const XArgs<Real> &a, const Src &sr
     }
 }
 
+// Roots ahead of the passes (FxRoots) for powers of two; the other lengths'
+// last pass has up to seven butterflies per lane (400x100x2 FP64, 896 points:
+// 66.2 us per step with the table, 67.7 with the roots ahead).
+template <typename Real, int N>
+__device__ __forceinline__ auto x_roots(int t, const cplx<Real> *tw) {
+    if constexpr (fx_odd(N) == 1) return FxRoots<Real, N>(t, tw);
+    else return tw;
+}
+
 // Scheduled lines.  A lane's loads are all in flight before the first pass,
 // which takes them from registers.  In the unpack a lane keeps its line (FP32:
 // pair of rows) and walks kx = k0 + u T, so each step is one pointer
@@ -92,8 +101,9 @@ __device__ __forceinline__ void xfwd_body(const XArgs<Real> &a, const Src &src, 
         }
 #pragma unroll
         for (int e = E / 2; e < E; ++e) v[e] = {Real(0), Real(0)};
+        const auto roots = x_roots<Real, N>(t, a.tw);
         fx_first_pass<Real, N>(line, t, v, a.tw, false);
-        fx_rest<Real, N>(line, t, a.tw, false);
+        fx_rest<Real, N>(line, t, roots, false);
     }
     __syncthreads();  // the unpack reads every line
     if constexpr (sizeof(Real) == 8) {
@@ -256,6 +266,7 @@ __device__ __forceinline__ void xinv_body(const XArgs<Real> &a, const cplx<Real>
     const int LINES = a.xr >> 1, ls = a.ls;
     const int tid = threadIdx.x;
     const int y0 = blockIdx.x * a.xr, z = blockIdx.y;
+    const auto roots = x_roots<Real, N>(tid % T, a.tw);
     {
         // lane (j, k0): rows 2j and 2j + 1; consecutive lanes read
         // consecutive rows of one kx column (a row pair is one 16-byte load
@@ -298,7 +309,7 @@ __device__ __forceinline__ void xinv_body(const XArgs<Real> &a, const cplx<Real>
         cplx<Real> v[E];
         fx_load<Real, N>(line, t, v);
         fx_first_pass<Real, N>(line, t, v, a.tw, true);
-        fx_rest<Real, N>(line, t, a.tw, true);
+        fx_rest<Real, N>(line, t, roots, true);
     }
     // the lanes of line jl store its rows 2 jl (real part) and 2 jl + 1
     const int ya = y0 + 2 * jl;

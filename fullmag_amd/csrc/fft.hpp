@@ -17,6 +17,7 @@
 
 #include "common.hpp"
 
+#include <type_traits>
 #include <vector>
 
 namespace fm {
@@ -264,27 +265,40 @@ __device__ __forceinline__ void dft_any(cplx<T> *v, const cplx<T> *tw, int n, bo
 // power-of-two R only the roots w^(2^b st) are read from the table; each
 // other power is one product of an earlier power and a table root, so no
 // twiddle carries more than three extra roundings.
+template <int R>
+constexpr int root_bits() {
+    return R == 2 ? 1 : R == 4 ? 2 : R == 8 ? 3 : 4;
+}
+// The same for power-of-two R with the roots w^(2^b st) in hand.
+template <typename T, int R>
+__device__ __forceinline__ void twiddle_by(cplx<T> *v, const cplx<T> *roots, bool inv) {
+    constexpr int LB = root_bits<R>();
+    // conjugation for the inverse as a product with -1 (exact), so the
+    // table loads stay out of any branch
+    const T sg = inv ? T(-1) : T(1);
+    cplx<T> pw[LB];
+#pragma unroll
+    for (int b = 0; b < LB; ++b) {
+        pw[b] = roots[b];
+        pw[b].y *= sg;
+    }
+    cplx<T> w[R];
+#pragma unroll
+    for (int r = 1; r < R; ++r) {
+        const int low = r & -r;
+        const int lb = low == 1 ? 0 : low == 2 ? 1 : low == 4 ? 2 : 3;
+        w[r] = (r == low) ? pw[lb] : cmul(w[r - low], pw[lb]);
+        v[r] = cmul(v[r], w[r]);
+    }
+}
 template <typename T, int R>
 __device__ __forceinline__ void twiddle(cplx<T> *v, const cplx<T> *tw, int st, bool inv) {
     if constexpr (R == 2 || R == 4 || R == 8 || R == 16) {
-        constexpr int LB = R == 2 ? 1 : R == 4 ? 2 : R == 8 ? 3 : 4;
-        // conjugation for the inverse as a product with -1 (exact), so the
-        // table loads stay out of any branch
-        const T sg = inv ? T(-1) : T(1);
+        constexpr int LB = root_bits<R>();
         cplx<T> pw[LB];
 #pragma unroll
-        for (int b = 0; b < LB; ++b) {
-            pw[b] = tw[st << b];
-            pw[b].y *= sg;
-        }
-        cplx<T> w[R];
-#pragma unroll
-        for (int r = 1; r < R; ++r) {
-            const int low = r & -r;
-            const int lb = low == 1 ? 0 : low == 2 ? 1 : low == 4 ? 2 : 3;
-            w[r] = (r == low) ? pw[lb] : cmul(w[r - low], pw[lb]);
-            v[r] = cmul(v[r], w[r]);
-        }
+        for (int b = 0; b < LB; ++b) pw[b] = tw[st << b];
+        twiddle_by<T, R>(v, pw, inv);
     } else {
         const T sg = inv ? T(-1) : T(1);
 #pragma unroll
@@ -489,10 +503,39 @@ __device__ __forceinline__ void pass_sync() {
     }
 }
 
+// The roots of a lane's butterflies in the passes after the first, loaded
+// beside the line's inputs; a pass takes the table or this.  A pass that reads
+// the table when it needs the roots waits for the L2 once more.  The x passes
+// carry them (their workgroups of up to 512 lanes leave few others to cover
+// the wait): per step 512x512x8 FP64 646.7 -> 637.7 us, mixed 345.9 -> 343.9,
+// 250x150x6 single 94.8 -> 93.5.  In the film's y convolution they cost
+// registers (512x512x1 FP64 90.1 -> 91.9 us) and in the slab kernel they gave
+// nothing.
+template <typename T, int N>
+struct FxRoots {
+    static_assert(fx_npass(N) <= 3, "two passes of roots");
+    cplx<T> w[2][8];
+    __device__ __forceinline__ FxRoots(int t, const cplx<T> *tw) {
+        if constexpr (fx_npass(N) > 1) fetch<1, fx_radix(N, 0)>(t, tw);
+        if constexpr (fx_npass(N) > 2) fetch<2, fx_radix(N, 0) * fx_radix(N, 1)>(t, tw);
+    }
+    template <int P, int NS>
+    __device__ __forceinline__ void fetch(int t, const cplx<T> *tw) {
+        constexpr int R = fx_radix(N, P), NT = fx_lanes(N), NR = N / R, MB = (NR + NT - 1) / NT, LB = root_bits<R>();
+        static_assert(MB * LB <= 8, "roots of one pass");
+#pragma unroll
+        for (int b = 0; b < MB; ++b) {
+            const int j0 = t + b * NT, j = MB * NT == NR || j0 < NR ? j0 : 0;
+#pragma unroll
+            for (int i = 0; i < LB; ++i) w[P - 1][b * LB + i] = tw[((j % NS) * (N / (NS * R))) << i];
+        }
+    }
+};
+
 // One pass.  LAST: output element i goes to put(i, value) instead of LDS, and
 // only the elements i < N / OUT_DIV are produced.
-template <typename T, int N, int R, int NS, bool LAST, int OUT_DIV, class Put>
-__device__ __forceinline__ void fx_pass(cplx<T> *line, int t, const cplx<T> *tw, bool inv, Put &&put) {
+template <typename T, int N, int P, int R, int NS, bool LAST, int OUT_DIV, class Tw, class Put>
+__device__ __forceinline__ void fx_pass(cplx<T> *line, int t, const Tw &tw, bool inv, Put &&put) {
     constexpr int G = fx_pad(N), NT = fx_lanes(N), NR = N / R, ST = N / (NS * R);
     constexpr int MB = (NR + NT - 1) / NT;  // butterflies per lane; the last may be beyond NR
     constexpr bool FULL = MB * NT == NR;
@@ -509,8 +552,9 @@ __device__ __forceinline__ void fx_pass(cplx<T> *line, int t, const cplx<T> *tw,
         for (int r = 0; r < R; ++r) v[b][r] = p[r * (NR + NR / G)];
         // k = 0 multiplies by the table's exact w^0 = 1 (no branch: lanes of
         // one wave differ in k, and a branch would split the table loads)
-        twiddle<T, R>(v[b], tw, k * ST, inv);
-        dft_any<T, R>(v[b], tw, N, inv);
+        if constexpr (std::is_same<Tw, FxRoots<T, N>>::value) twiddle_by<T, R>(v[b], tw.w[P - 1] + b * root_bits<R>(), inv);
+        else twiddle<T, R>(v[b], tw, k * ST, inv);
+        dft_any<T, R>(v[b], nullptr, N, inv);
         base[b] = (j / NS) * NS * R + k;
     }
     if constexpr (!LAST) pass_sync<N>();
@@ -535,11 +579,11 @@ struct FxNoPut {
 };
 
 // Passes P.. of the schedule; the last through `put` when STORE.
-template <typename T, int N, int P, int NS, bool STORE, int OUT_DIV, class Put>
-__device__ __forceinline__ void fx_passes(cplx<T> *line, int t, const cplx<T> *tw, bool inv, Put &&put) {
+template <typename T, int N, int P, int NS, bool STORE, int OUT_DIV, class Tw, class Put>
+__device__ __forceinline__ void fx_passes(cplx<T> *line, int t, const Tw &tw, bool inv, Put &&put) {
     if constexpr (P < fx_npass(N)) {
         constexpr int R = fx_radix(N, P);
-        fx_pass<T, N, R, NS, STORE && P + 1 == fx_npass(N), OUT_DIV>(line, t, tw, inv, put);
+        fx_pass<T, N, P, R, NS, STORE && P + 1 == fx_npass(N), OUT_DIV>(line, t, tw, inv, put);
         fx_passes<T, N, P + 1, NS * R, STORE, OUT_DIV>(line, t, tw, inv, put);
     }
 }
@@ -564,12 +608,12 @@ __device__ __forceinline__ void fx_first_pass(cplx<T> *line, int t, const cplx<T
     }
     pass_sync<N>();
 }
-template <typename T, int N>
-__device__ __forceinline__ void fx_rest(cplx<T> *line, int t, const cplx<T> *tw, bool inv) {
+template <typename T, int N, class Tw>
+__device__ __forceinline__ void fx_rest(cplx<T> *line, int t, const Tw &tw, bool inv) {
     fx_passes<T, N, 1, fx_radix(N, 0), false, 1>(line, t, tw, inv, FxNoPut{});
 }
-template <typename T, int N, int OUT_DIV, class Put>
-__device__ __forceinline__ void fx_rest_put(cplx<T> *line, int t, const cplx<T> *tw, bool inv, Put &&put) {
+template <typename T, int N, int OUT_DIV, class Tw, class Put>
+__device__ __forceinline__ void fx_rest_put(cplx<T> *line, int t, const Tw &tw, bool inv, Put &&put) {
     fx_passes<T, N, 1, fx_radix(N, 0), true, OUT_DIV>(line, t, tw, inv, put);
 }
 
