@@ -745,6 +745,19 @@ bool class_rule(const DemagPlan &dp) {
            class_length(dp.py) && dp.tune.slab > 0 && !use_slab<Real>(dp);
 }
 
+// Rows per x workgroup where full workgroups are few: with fewer than 64 of more
+// than one wavefront each, halving the rows (down to 4) spreads the same lanes
+// over twice the CUs, for shorter runs per column.  us per step: 500x125x1
+// mixed 53.6 with 16 rows (24 workgroups of 512 lanes), 51.3 with 8, 50.5 with
+// 4; 200x30x2 mixed 48.1, 46.1, 44.6.  Not beyond: 256x256x1 mixed (48
+// workgroups of 256) 49.8 with 16 and with 8, 512x512x1 mixed (96) 75.4 and
+// 76.6, 64x64x1 FP64 (12 of one wavefront) 42.5 and 43.5.
+int spread_rows(int xr, int threads, int rows, int planes) {
+    while (xr > 4 && xr / 2 * threads > 64 && cdiv(rows, xr) * planes < 64)
+        xr >>= 1;
+    return xr;
+}
+
 // Launch geometry of the planned lines (no allocation): x rows per
 // workgroup, y lines per workgroup, long-z tile, thin-film y convolution
 // form.  `keep_split` >= 0 requires the thin-film form to stay as it is (a
@@ -769,6 +782,7 @@ bool plan_geometry(DemagPlan &dp, std::string &err, int keep_split = -1) {
         err = "x line FFT does not fit in one workgroup";
         return false;
     }
+    if (dp.lx.fixed && dp.tune.x_rows <= 0) dp.xr = spread_rows(dp.xr, dp.lx.threads, dp.ny, 3 * dp.nz);
     if (dp.three_d) {
         dp.y_lines_per_wg = pick_lpw(dp.ly, ce);
         if (dp.tune.y_lpw > 0) dp.y_lines_per_wg = std::min(dp.y_lines_per_wg, dp.tune.y_lpw);
