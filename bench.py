@@ -68,6 +68,7 @@ def alg_bytes(nx, ny, nz, q, r):
         "demag_y_fwd": 3 * a1 * c + 3 * a2 * c,
         "demag_z_conv": 3 * a2 * c + kern * r + 3 * a2 * c,
         "demag_yz_class": 3 * a1 * c + kern * r + 3 * a2 * c,
+        "demag_yz_slab": 3 * a1 * c + kern * r + 3 * a1 * c,
         "demag_y_inv": 3 * a2 * c + 3 * a1 * c,
         "demag_x_c2r": 3 * a1 * c + 3 * n * r,
         # corrector: mt, Hd, m0, k1 -> m (the predictor runs in the stats

@@ -29,8 +29,8 @@ enum Mode { MODE_SINGLE = 1, MODE_DOUBLE = 2, MODE_MIXED = 3 };
 // Launch-schedule knobs of the demag transforms (0 = automatic).  Settable
 // per backend from the FULLMAG_FDM_TUNE environment variable as a comma list
 // of key=value (x_radix, x_lanes, x_rows, y_radix, y_lanes, y_lpw, fixed,
-// xcd, y_pipe, y_pipe_f, z_tile, zc, y_split, slab, pad).  x_radix, x_lanes,
-// x_rows, y_radix, y_lanes, y_lpw, fixed, z_tile, y_split and pad shape the
+// xcd, y_pipe, y_pipe_f, z_tile, zc, y_split, slab, pad, skew).  x_radix, x_lanes,
+// x_rows, y_radix, y_lanes, y_lpw, fixed, z_tile, y_split, pad and skew shape the
 // plan made at set-up; the others are read at every launch.
 struct DemagTuning {
     int x_radix = 16, x_lanes = 0, x_rows = 0;
@@ -43,6 +43,7 @@ struct DemagTuning {
     int zc = 0;        // z planes per workgroup of the cell kernels (0: automatic)
     int y_split = 0;   // 1: thin-film y convolution as separate line and tensor passes
     int slab = 160;    // y and z passes in one kernel for kx slabs of at most this many KB of LDS (0: off, ky classes too)
+    int skew = 1;      // 0: x transforms at the integer frequencies
     int pad = 1;       // 0: transform lengths 2n even where a longer scheduled length is faster
 };
 
@@ -68,7 +69,8 @@ struct DemagPlan {
     bool projection = false;  // no tensor: k-space projection fallback
     int nx = 0, ny = 0, nz = 0;
     int px = 0, py = 0, pz = 1;
-    int hx = 0;    // px / 2 + 1 columns of the half spectrum
+    bool skew = false;  // x frequencies k + 1/2 (skew-cyclic convolution along x), fixed at set-up
+    int hx = 0;    // columns of the half spectrum: px / 2 (skew), px / 2 + 1
     size_t lds_limit = 65536;  // LDS bytes one workgroup may allocate on this device
     bool y_split = false;      // thin film: y lines, tensor and inverse y lines as three passes
     int rows = 0;  // rows per plane of `spec`
@@ -85,6 +87,7 @@ struct DemagPlan {
     void *tw_x = nullptr, *tw_y = nullptr, *tw_z = nullptr;
     void *spec = nullptr;
     void *xspec = nullptr;  // x passes' spectrum of rows of xrows entries (ky classes)
+    void *sw = nullptr;     // exp(-i pi d / px) of the displacement d(x) (skew)
     void *tw_c = nullptr;   // roots of length py / cls
     int cls = 1, xrows = 0;  // ky classes (1: none), fixed at set-up
     void *kern = nullptr;

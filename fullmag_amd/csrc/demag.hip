@@ -262,6 +262,33 @@ bool use_slab(const DemagPlan &dp) {
     return sizeof(Real) == 4 && 10 * dp.py >= 9 * rounds * cols;
 }
 
+// Whether px / 2 workgroups of `lds` bytes, one per column, take fewer rounds
+// over the chip than px / 2 + 1.
+bool saves_round(const DemagPlan &dp, size_t lds, int per_group = 1) {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+        return false;
+    const int64_t slots = cus * std::max<int64_t>(1, (int64_t)(dp.lds_limit / lds)), h = dp.px / 2;
+    return cdiv(cdiv(h + 1, per_group), slots) > cdiv(cdiv(h, per_group), slots);
+}
+
+// Whether the x transforms run at the frequencies k + 1/2 (plans with the
+// library's own tensor): the padded rows leave room for a skew-cyclic
+// convolution, whose spectrum has px / 2 columns and no Nyquist one, so the
+// slab kernel's workgroups, one to three per CU, come to whole rounds where
+// px does.  us per mixed Heun step without and with: 256x256x8 117.6 and 94.2
+// (257 slabs of 104 KB are two rounds), 500x250x8 175.3 and 152.5, 256x256x4
+// 73.4 and 71.1, 128x128x8 55.1 and 53.6.  Elsewhere the factors in the x
+// passes cost more than a column: 512x512x8 340 and 345, 512x512x1 73.8 and
+// 75.5, 256x256x64 756 and 768.  In FP64 they cost 2 to 3 us per pass
+// (128x128x4 52 and 57), which only a round saved gives back.
+template <typename Real>
+bool skew_rule(const DemagPlan &dp) {
+    if (dp.tune.skew == 0 || !dp.three_d || !use_slab<Real>(dp)) return false;
+    return sizeof(Real) == 4 || saves_round(dp, (size_t)3 * dp.nz * fx_size(dp.py) * sizeof(cplx<Real>));
+}
+
 // Whether a slab's ky classes go through the y transform and the z
 // convolution in one kernel each: the plan's choice (class_rule, fixed at set-up
 // with the tensor's layout), its second spectrum, and the knobs.
@@ -453,6 +480,7 @@ void demag_eval_t(Context &c, const S *src, Real *out, bool weight_ms, int phase
     const size_t ce = sizeof(cplx<Real>);
     XArgs<Real> xa{};
     xa.tw = static_cast<const cplx<Real> *>(dp.tw_x);
+    xa.sw = static_cast<const cplx<Real> *>(dp.sw);
     xa.lp = dp.lx;
     xa.rows = dp.ny;
     xa.n_in = dp.nx;
@@ -497,6 +525,15 @@ void demag_eval_t(Context &c, const S *src, Real *out, bool weight_ms, int phase
     }
 }
 
+// exp(-i pi d / px) at x, d = x up to px / 2 and x - px beyond: the factors
+// that shift a row's x frequencies by 1/2.
+std::vector<cplx<double>> skew_table(int px) {
+    std::vector<cplx<double>> w = twiddle_table(2 * px);
+    w.resize(px);
+    for (int x = px / 2 + 1; x < px; ++x) w[x] = {-w[x].x, -w[x].y};
+    return w;
+}
+
 // Twiddle tables of the plan's lengths, in one allocation.
 template <typename Real>
 bool upload_twiddles(Context &c) {
@@ -504,9 +541,13 @@ bool upload_twiddles(Context &c) {
     std::vector<cplx<Real>> all;
     for (int n : {dp.px, dp.py, dp.three_d ? dp.pz : 1, dp.cls > 1 ? dp.py / dp.cls : 1})
         for (const cplx<double> &w : twiddle_table(n)) all.push_back({(Real)w.x, (Real)w.y});
+    const size_t roots = all.size();
+    if (dp.skew)
+        for (const cplx<double> &w : skew_table(dp.px)) all.push_back({(Real)w.x, (Real)w.y});
     const size_t bytes = all.size() * sizeof(cplx<Real>);
     if (!ctx_alloc(c, &dp.tw_x, bytes, "twiddle tables")) return false;
     dp.tw_y = static_cast<cplx<Real> *>(dp.tw_x) + dp.px;
+    dp.sw = dp.skew ? static_cast<cplx<Real> *>(dp.tw_x) + roots : nullptr;
     dp.tw_z = static_cast<cplx<Real> *>(dp.tw_y) + dp.py;
     dp.tw_c = static_cast<cplx<Real> *>(dp.tw_z) + (dp.three_d ? dp.pz : 1);
     return ctx_upload(c, dp.tw_x, all.data(), bytes, "hipMemcpy(twiddles)", c.last_error);
@@ -520,7 +561,7 @@ void pad_lengths(DemagPlan &dp, bool free, int z_keep) {
     dp.px = free ? pick_padded(dp.nx) : 2 * dp.nx;
     dp.py = free ? pick_padded(dp.ny) : 2 * dp.ny;
     dp.pz = !dp.three_d ? 1 : free && 2 * dp.nz > z_keep ? pick_padded(dp.nz) : 2 * dp.nz;
-    dp.hx = dp.px / 2 + 1;
+    dp.hx = dp.px / 2 + (dp.skew ? 0 : 1);
 }
 
 bool plan_lines(DemagPlan &dp, std::string &err) {
@@ -564,6 +605,7 @@ void parse_tuning_string(DemagTuning &t, const char *text) {
             else if (k == "y_split") t.y_split = v;
             else if (k == "pad") t.pad = v;
             else if (k == "slab") t.slab = v;
+            else if (k == "skew") t.skew = v;
         }
         pos = end + 1;
     }
@@ -590,6 +632,11 @@ bool newell_forward(Context &c, const DemagPlan &dp, double z_offset, cplx<doubl
         const std::vector<cplx<double>> w = twiddle_table(n);
         tw.insert(tw.end(), w.begin(), w.end());
     }
+    const size_t roots = tw.size();
+    if (dp.skew) {
+        const std::vector<cplx<double>> w = skew_table(dp.px);
+        tw.insert(tw.end(), w.begin(), w.end());
+    }
     void *d_spec = nullptr;
     bool ok = hip_ok(hipMalloc(&d_spec, spec_bytes + oct_bytes + tw.size() * ce), "hipMalloc(newell)", err);
     double *d_oct = reinterpret_cast<double *>(static_cast<char *>(d_spec) + spec_bytes);
@@ -609,6 +656,7 @@ bool newell_forward(Context &c, const DemagPlan &dp, double z_offset, cplx<doubl
         NewellSource src{d_oct, dp.nx, dp.ny, nzo, dp.px, dp.py, pz, z_even ? 1 : 0};
         XArgs<double> xa{};
         xa.tw = twx;
+        xa.sw = dp.skew ? twx + roots : nullptr;
         xa.lp = lx;
         xa.rows = dp.py;
         xa.n_in = dp.px;
@@ -904,6 +952,9 @@ bool demag_setup(Context &c, const fullmag_fdm_plan_desc &plan, bool newell_on_d
     dp.inv_npad = 1.0 / ((double)dp.px * dp.py * dp.pz);
     dp.lds_limit = device_lds_limit(c.device);
     if (!plan_lines(dp, c.last_error)) return false;
+    dp.skew = !have_spectra && newell_on_device &&
+              (c.mode == MODE_DOUBLE ? skew_rule<double>(dp) : skew_rule<float>(dp));
+    dp.hx = dp.px / 2 + (dp.skew ? 0 : 1);
     if (c.mode == MODE_DOUBLE) return setup_t<double>(c, plan);
     return setup_t<float>(c, plan);
 }
@@ -1152,6 +1203,20 @@ bool stack_setup_t(Stack &s, std::string &err) {
     dp.inv_npad = 1.0 / ((double)dp.px * dp.py * dp.pz);
     dp.lds_limit = device_lds_limit(c.device);
     if (!plan_lines(dp, err)) return false;
+    // The coupled y pass takes a thin stack whose column of 3 L lines fits one
+    // workgroup; several columns where they are short.  Against the separate
+    // passes, Heun steps of 2 to 5 layers of 64 x 64 to 512 x 512: 1.03 to
+    // 1.6 times as fast wherever it fits, FP32 and FP64.
+    s.kpw = std::max(1, 256 / (3 * L * dp.ly.threads));
+    s.fused = !dp.three_d && dp.ly.fixed && L <= kStackFused && !dp.tune.y_split &&
+              3 * L * dp.ly.threads <= 1024 &&
+              (size_t)3 * L * s.kpw * line_slots(dp.ly) * ce <= dp.lds_limit;
+    // Frequencies k + 1/2 along x (skew_rule) where that saves a round: 3 films
+    // of 512x512, 513 workgroups, mixed 138.3 and 123.7 us per step, FP64 214.8
+    // and 203.1; without one saved, 100x300 four films FP64 79.5 and 83.0.
+    dp.skew = tune.skew != 0 && s.fused &&
+              saves_round(dp, (size_t)3 * L * s.kpw * line_slots(dp.ly) * ce, s.kpw);
+    dp.hx = dp.px / 2 + (dp.skew ? 0 : 1);
     if (!pick_x(dp.lx, ce, dp.xr, dp.x_ls, 16, dp.lds_limit)) {
         err = "stack: x line FFT does not fit in one workgroup";
         return false;
@@ -1176,14 +1241,6 @@ bool stack_setup_t(Stack &s, std::string &err) {
     s.planes = dp.pz;
     const int64_t points = (int64_t)s.planes * dp.hx * dp.py;
     s.layer_spec = 3 * (uint64_t)points;
-    // The coupled y pass takes a thin stack whose column of 3 L lines fits one
-    // workgroup; several columns where they are short.  Against the separate
-    // passes, Heun steps of 2 to 5 layers of 64 x 64 to 512 x 512: 1.03 to
-    // 1.6 times as fast wherever it fits, FP32 and FP64.
-    s.kpw = std::max(1, 256 / (3 * L * dp.ly.threads));
-    s.fused = !dp.three_d && dp.ly.fixed && L <= kStackFused && !dp.tune.y_split &&
-              3 * L * dp.ly.threads <= 1024 &&
-              (size_t)3 * L * s.kpw * line_slots(dp.ly) * ce <= dp.lds_limit;
     if (!ctx_alloc(c, &s.spec_m, (size_t)L * s.layer_spec * ce, "stack spectra") ||
         (!s.fused && !ctx_alloc(c, &s.spec_h, (size_t)L * s.layer_spec * ce, "stack field spectra"))) {
         err = c.last_error;
@@ -1302,6 +1359,7 @@ void stack_eval_t(Stack &s, const S *const *src) {
     const int L = (int)s.layers.size();
     XArgs<Real> xa{};
     xa.tw = static_cast<const cplx<Real> *>(dp.tw_x);
+    xa.sw = static_cast<const cplx<Real> *>(dp.sw);
     xa.lp = dp.lx;
     xa.rows = dp.ny;
     xa.n_in = dp.nx;

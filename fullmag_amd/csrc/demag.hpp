@@ -139,6 +139,7 @@ struct XArgs {
     int n_in;         // forward: inputs loaded per row
     int n_out;        // inverse: outputs stored per row
     Real scale;       // inverse: 1/Npad
+    const cplx<Real> *sw;  // frequencies k + 1/2: exp(-i pi d / px) of the displacement d(x) (null: k)
     SpecGeom g;
 };
 

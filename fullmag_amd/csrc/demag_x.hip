@@ -34,6 +34,7 @@ __device__ __forceinline__ void xfwd_body_rt(const XArgs<Real> &a, const Src &sr
         if (x < a.n_in) {
             if (ya < a.rows) v.x = src(c, z, ya, x);
             if (ya + 1 < a.rows) v.y = src(c, z, ya + 1, x);
+            if (a.sw) v = cmul(v, a.sw[x]);
         }
         line[lslot(a.lp, x)] = v;
     }
@@ -45,7 +46,7 @@ __device__ __forceinline__ void xfwd_body_rt(const XArgs<Real> &a, const Src &sr
         const int j = idx & (LINES - 1), k = idx >> (a.xr_log2 - 1), y = y0 + 2 * j;
         if (y >= a.rows) continue;
         cplx<Real> A, B;
-        xfwd_split(lds[j * ls + lslot(a.lp, k)], lds[j * ls + lslot(a.lp, k == 0 ? 0 : n - k)], A, B);
+        xfwd_split(lds[j * ls + lslot(a.lp, k)], lds[j * ls + lslot(a.lp, a.sw ? n - 1 - k : k == 0 ? 0 : n - k)], A, B);
         cplx<Real> *dst = spec + a.g.at(c, z, k, y);
         dst[0] = A;
         if (y + 1 < a.rows) dst[1] = B;
@@ -65,7 +66,7 @@ __device__ __forceinline__ auto x_roots(int t, const cplx<Real> *tw) {
 // which takes them from registers.  In the unpack a lane keeps its line (FP32:
 // pair of rows) and walks kx = k0 + u T, so each step is one pointer
 // increment and one LDS read per side at a fixed distance.
-template <typename Real, class Src, int N>
+template <typename Real, class Src, int N, bool SKEW>
 __device__ __forceinline__ void xfwd_body(const XArgs<Real> &a, const Src &src, cplx<Real> *spec, int c) {
     constexpr int E = fx_elems(N), T = fx_lanes(N);
     extern __shared__ unsigned char smem_raw[];
@@ -101,6 +102,13 @@ __device__ __forceinline__ void xfwd_body(const XArgs<Real> &a, const Src &src, 
         }
 #pragma unroll
         for (int e = E / 2; e < E; ++e) v[e] = {Real(0), Real(0)};
+        if constexpr (SKEW) {
+            cplx<Real> w[E / 2];
+#pragma unroll
+            for (int e = 0; e < E / 2; ++e) w[e] = a.sw[t + e * T];
+#pragma unroll
+            for (int e = 0; e < E / 2; ++e) v[e] = cmul(v[e], w[e]);
+        }
         const auto roots = x_roots<Real, N>(t, a.tw);
         fx_first_pass<Real, N>(line, t, v, a.tw, false);
         fx_rest<Real, N>(line, t, roots, false);
@@ -125,9 +133,9 @@ __device__ __forceinline__ void xfwd_body(const XArgs<Real> &a, const Src &src, 
 #pragma unroll
         for (int u = 0; u < E; ++u) {
             const int k = k0 + u * KS;
-            one(k, u == 0 && k0 == 0 ? 0 : N - k, dst + (int64_t)(u * KS) * a.g.pitch);
+            one(k, SKEW ? N - 1 - k : u == 0 && k0 == 0 ? 0 : N - k, dst + (int64_t)(u * KS) * a.g.pitch);
         }
-        if (k0 == 0) one(N / 2, N / 2, dst + (int64_t)(N / 2) * a.g.pitch);
+        if (!SKEW && k0 == 0) one(N / 2, N / 2, dst + (int64_t)(N / 2) * a.g.pitch);
     } else {
         // lane (j, k) splits line j into rows 2j (A) and 2j + 1 (B); the two
         // are adjacent in memory (one 16-byte store when the row pitch is even)
@@ -149,16 +157,16 @@ __device__ __forceinline__ void xfwd_body(const XArgs<Real> &a, const Src &src, 
 #pragma unroll
         for (int u = 0; u < E / 2; ++u) {
             const int k = k0 + u * T;
-            one(k, u == 0 && k0 == 0 ? 0 : N - k, dst + (int64_t)(u * T) * a.g.pitch);
+            one(k, SKEW ? N - 1 - k : u == 0 && k0 == 0 ? 0 : N - k, dst + (int64_t)(u * T) * a.g.pitch);
         }
-        if (k0 == 0) one(N / 2, N / 2, dst + (int64_t)(N / 2) * a.g.pitch);
+        if (!SKEW && k0 == 0) one(N / 2, N / 2, dst + (int64_t)(N / 2) * a.g.pitch);
     }
 }
 
 // Component c = blockIdx.z.
-template <typename Real, class Src, int N = 0>
+template <typename Real, class Src, int N = 0, bool SKEW = false>
 __global__ void __launch_bounds__(kMaxBlock) xfwd_kernel(XArgs<Real> a, Src src, cplx<Real> *spec) {
-    if constexpr (N > 0) xfwd_body<Real, Src, N>(a, src, spec, (int)blockIdx.z);
+    if constexpr (N > 0) xfwd_body<Real, Src, N, SKEW>(a, src, spec, (int)blockIdx.z);
     else xfwd_body_rt<Real, Src>(a, src, spec, (int)blockIdx.z);
 }
 
@@ -174,10 +182,10 @@ struct XFwdPack {
     Src src;
     cplx<Real> *spec;
 };
-template <typename Real, class Src, int N>
+template <typename Real, class Src, int N, bool SKEW>
 __global__ void __launch_bounds__(kMaxBlock) xfwd_multi(const XFwdPack<Real, Src> *tab, int zdiv) {
     const XFwdPack<Real, Src> p = tab[blockIdx.z / zdiv];
-    xfwd_body<Real, Src, N>(p.a, p.src, p.spec, (int)(blockIdx.z % zdiv));
+    xfwd_body<Real, Src, N, SKEW>(p.a, p.src, p.spec, (int)(blockIdx.z % zdiv));
 }
 
 // Entry l of an argument array, l uniform in the workgroup (selects of
@@ -193,14 +201,14 @@ __device__ __forceinline__ T entry_of(const T (&v)[kStackPack], int l) {
 // Layer blockIdx.z / 3 of a stack, component blockIdx.z % 3: one launch for
 // all layers, whose single passes of a few microseconds leave the chip partly
 // idle (three 512 x 512 films, FP32: 3 x 6.7 us one by one).
-template <typename Real, typename S, bool GATHER, int N>
+template <typename Real, typename S, bool GATHER, int N, bool SKEW>
 __global__ void __launch_bounds__(kMaxBlock) xfwd_stack_kernel(XArgs<Real> a, StackMag<Real, S> p, cplx<Real> *spec) {
     using Src = MagSource<Real, S, GATHER>;
     const int l = (int)blockIdx.z / 3, c = (int)blockIdx.z - 3 * l;
     const Src src{entry_of(p.m, l), GATHER ? entry_of(p.mask, l) : nullptr, nullptr, entry_of(p.ms, l),
                   p.nx, p.ny, p.nz, p.n, nullptr};
     cplx<Real> *sp = spec + l * p.layer_stride;
-    if constexpr (N > 0) xfwd_body<Real, Src, N>(a, src, sp, c);
+    if constexpr (N > 0) xfwd_body<Real, Src, N, SKEW>(a, src, sp, c);
     else xfwd_body_rt<Real, Src>(a, src, sp, c);
 }
 
@@ -239,7 +247,7 @@ __device__ __forceinline__ void xinv_body_rt(const XArgs<Real> &a, const cplx<Re
             if (idx >= hx * LINES) break;
             const int j = idx & (LINES - 1), k = idx >> (a.xr_log2 - 1);
             lds[j * ls + lslot(a.lp, k)] = {A[u].x - B[u].y, A[u].y + B[u].x};
-            if (k > 0 && k < n - k) lds[j * ls + lslot(a.lp, n - k)] = {A[u].x + B[u].y, B[u].x - A[u].y};
+            if (a.sw || (k > 0 && k < n - k)) lds[j * ls + lslot(a.lp, a.sw ? n - 1 - k : n - k)] = {A[u].x + B[u].y, B[u].x - A[u].y};
         }
     }
     __syncthreads();
@@ -249,7 +257,8 @@ __device__ __forceinline__ void xinv_body_rt(const XArgs<Real> &a, const cplx<Re
     // the lanes of line jl store its rows 2 jl (real part) and 2 jl + 1
     const int ya = y0 + 2 * jl;
     for (int x = t; x < a.n_out; x += T) {
-        const cplx<Real> v = line[lslot(a.lp, x)];
+        cplx<Real> v = line[lslot(a.lp, x)];
+        if (a.sw) v = cmul(v, cconj(a.sw[x]));
         if (ya < a.rows) sink(c, z, ya, x, v.x * a.scale);
         if (ya + 1 < a.rows) sink(c, z, ya + 1, x, v.y * a.scale);
     }
@@ -258,9 +267,9 @@ __device__ __forceinline__ void xinv_body_rt(const XArgs<Real> &a, const cplx<Re
 // Scheduled lines.  Every load of a lane (kx = k0 + u T of one row pair) is in
 // flight before the first LDS write; the addresses and LDS slots advance by
 // fixed steps.
-template <typename Real, class Sink, int N>
+template <typename Real, class Sink, int N, bool SKEW>
 __device__ __forceinline__ void xinv_body(const XArgs<Real> &a, const cplx<Real> *spec, const Sink &sink, int c) {
-    constexpr int E = fx_elems(N), T = fx_lanes(N), H = E / 2;
+    constexpr int E = fx_elems(N), T = fx_lanes(N), H = E / 2, U = SKEW ? H : H + 1;
     extern __shared__ unsigned char smem_raw[];
     cplx<Real> *lds = reinterpret_cast<cplx<Real> *>(smem_raw);
     const int LINES = a.xr >> 1, ls = a.ls;
@@ -274,11 +283,11 @@ __device__ __forceinline__ void xinv_body(const XArgs<Real> &a, const cplx<Real>
         const int j = tid & (LINES - 1), k0 = tid >> (a.xr_log2 - 1), ya = y0 + 2 * j;
         const bool oka = ya < a.rows, okb = ya + 1 < a.rows;
         const cplx<Real> *s = spec + a.g.at(c, z, k0, oka ? ya : 0);
-        cplx<Real> A[H + 1], B[H + 1];
+        cplx<Real> A[U], B[U];
         auto off = [&](int u) { return (int64_t)(u < H ? u * T : k0 == 0 ? N / 2 : 0) * a.g.pitch; };
         if (sizeof(Real) == 4 && (a.g.pitch & 1) == 0) {
 #pragma unroll
-            for (int u = 0; u <= H; ++u) {
+            for (int u = 0; u < U; ++u) {
                 // an even row pitch and an even ya keep the pair 16-byte aligned
                 const float4 q = *reinterpret_cast<const float4 *>(s + off(u));
                 A[u] = {Real(q.x), Real(q.y)};
@@ -287,19 +296,20 @@ __device__ __forceinline__ void xinv_body(const XArgs<Real> &a, const cplx<Real>
         } else {
             const int nb = okb ? 1 : 0;
 #pragma unroll
-            for (int u = 0; u <= H; ++u) {
+            for (int u = 0; u < U; ++u) {
                 A[u] = s[off(u)];
                 B[u] = s[off(u) + nb];
             }
         }
         cplx<Real> *ln = lds + j * ls;
 #pragma unroll
-        for (int u = 0; u <= H; ++u) {
+        for (int u = 0; u < U; ++u) {
             const int k = u < H ? k0 + u * T : N / 2;
             if (!oka) A[u] = {Real(0), Real(0)};
             if (!okb) B[u] = {Real(0), Real(0)};
             if (u < H || k0 == 0) ln[fxslot<N>(k)] = {A[u].x - B[u].y, A[u].y + B[u].x};
-            if (u < H && (u > 0 || k0 > 0)) ln[fxslot<N>(N - k)] = {A[u].x + B[u].y, B[u].x - A[u].y};
+            if (SKEW || (u < H && (u > 0 || k0 > 0)))
+                ln[fxslot<N>(SKEW ? N - 1 - k : N - k)] = {A[u].x + B[u].y, B[u].x - A[u].y};
         }
     }
     __syncthreads();
@@ -311,6 +321,10 @@ __device__ __forceinline__ void xinv_body(const XArgs<Real> &a, const cplx<Real>
         fx_first_pass<Real, N>(line, t, v, a.tw, true);
         fx_rest<Real, N>(line, t, roots, true);
     }
+    auto out = [&](int x) -> cplx<Real> {
+        if constexpr (SKEW) return cmul(line[fxslot<N>(x)], cconj(a.sw[x]));
+        else return line[fxslot<N>(x)];
+    };
     // the lanes of line jl store its rows 2 jl (real part) and 2 jl + 1
     const int ya = y0 + 2 * jl;
     if constexpr (std::is_same<Sink, FieldSink<float>>::value) {
@@ -336,7 +350,7 @@ __device__ __forceinline__ void xinv_body(const XArgs<Real> &a, const cplx<Real>
                 if (x < a.n_out) {
                     cplx<Real> v[4];
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] = line[fxslot<N>(x + e)];
+                    for (int e = 0; e < 4; ++e) v[e] = out(x + e);
                     auto row = [&](uint32_t k, int part) {
                         float o[4];
 #pragma unroll
@@ -371,7 +385,7 @@ __device__ __forceinline__ void xinv_body(const XArgs<Real> &a, const cplx<Real>
             for (int e = 0; e < H; ++e) {
                 const int x = t + e * T;
                 if (x < a.n_out) {
-                    const cplx<Real> v = line[fxslot<N>(x)];
+                    const cplx<Real> v = out(x);
                     if (oka) sink.put(c, z, ya, x, v.x * a.scale, ka[e]);
                     if (okb) sink.put(c, z, ya + 1, x, v.y * a.scale, kb[e]);
                 }
@@ -387,7 +401,7 @@ __device__ __forceinline__ void xinv_body(const XArgs<Real> &a, const cplx<Real>
             for (int x = 4 * t; x < a.n_out; x += 4 * T) {
                 cplx<Real> v[4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = line[fxslot<N>(x + e)];
+                for (int e = 0; e < 4; ++e) v[e] = out(x + e);
                 const int64_t i = ((int64_t)z * sink.ny + ya) * sink.nx + x;
                 if (ya < a.rows)
                     *reinterpret_cast<float4 *>(sink.out + (int64_t)c * sink.n + i) =
@@ -400,26 +414,26 @@ __device__ __forceinline__ void xinv_body(const XArgs<Real> &a, const cplx<Real>
         }
     }
     for (int x = t; x < a.n_out; x += T) {
-        const cplx<Real> v = line[fxslot<N>(x)];
+        const cplx<Real> v = out(x);
         if (ya < a.rows) sink(c, z, ya, x, v.x * a.scale);
         if (ya + 1 < a.rows) sink(c, z, ya + 1, x, v.y * a.scale);
     }
 }
 
-template <typename Real, class Sink, int N = 0>
+template <typename Real, class Sink, int N = 0, bool SKEW = false>
 __global__ void __launch_bounds__(kMaxBlock) xinv_kernel(XArgs<Real> a, const cplx<Real> *spec, Sink sink) {
-    if constexpr (N > 0) xinv_body<Real, Sink, N>(a, spec, sink, (int)blockIdx.z);
+    if constexpr (N > 0) xinv_body<Real, Sink, N, SKEW>(a, spec, sink, (int)blockIdx.z);
     else xinv_body_rt<Real, Sink>(a, spec, sink, (int)blockIdx.z);
 }
 
-template <typename Real, int N>
+template <typename Real, int N, bool SKEW>
 __global__ void __launch_bounds__(kMaxBlock)
     xinv_stack_kernel(XArgs<Real> a, const cplx<Real> *spec, StackField<Real> p) {
     using Sink = FieldSink<Real>;
     const int l = (int)blockIdx.z / 3, c = (int)blockIdx.z - 3 * l;
     const Sink sink{entry_of(p.out, l), entry_of(p.mask, l), p.nx, p.ny, p.n};
     const cplx<Real> *sp = spec + l * p.layer_stride;
-    if constexpr (N > 0) xinv_body<Real, Sink, N>(a, sp, sink, c);
+    if constexpr (N > 0) xinv_body<Real, Sink, N, SKEW>(a, sp, sink, c);
     else xinv_body_rt<Real, Sink>(a, sp, sink, c);
 }
 
@@ -429,10 +443,10 @@ struct XInvPack {
     const cplx<Real> *spec;
     Sink sink;
 };
-template <typename Real, class Sink, int N>
+template <typename Real, class Sink, int N, bool SKEW>
 __global__ void __launch_bounds__(kMaxBlock) xinv_multi(const XInvPack<Real, Sink> *tab, int zdiv) {
     const XInvPack<Real, Sink> p = tab[blockIdx.z / zdiv];
-    xinv_body<Real, Sink, N>(p.a, p.spec, p.sink, (int)(blockIdx.z % zdiv));
+    xinv_body<Real, Sink, N, SKEW>(p.a, p.spec, p.sink, (int)(blockIdx.z % zdiv));
 }
 
 }  // namespace
@@ -447,11 +461,16 @@ void launch_xfwd(Context &c, const XArgs<Real> &xa, const Src &src, cplx<Real> *
         with_line(xa.lp, [&](auto NC) {
             constexpr int N = decltype(NC)::value;
             const XFwdPack<Real, Src> pk{xa, src, spec};
-            const void *multi = nullptr;
-            if constexpr (N > 0) multi = reinterpret_cast<const void *>(&xfwd_multi<Real, Src, N>);
-            launch_rec(c, multi, grid, block, lds, (int)comps, pk, [&] {
-                           hipLaunchKernelGGL((xfwd_kernel<Real, Src, N>), grid, block, lds, c.stream, xa, src, spec);
-                       });
+            auto launch = [&](auto skew) {
+                constexpr bool SK = decltype(skew)::value;
+                const void *multi = nullptr;
+                if constexpr (N > 0) multi = reinterpret_cast<const void *>(&xfwd_multi<Real, Src, N, SK>);
+                launch_rec(c, multi, grid, block, lds, (int)comps, pk, [&] {
+                    hipLaunchKernelGGL((xfwd_kernel<Real, Src, N, SK>), grid, block, lds, c.stream, xa, src, spec);
+                });
+            };
+            if (xa.sw) launch(std::true_type{});
+            else launch(std::false_type{});
         });
     }
 }
@@ -463,12 +482,17 @@ void launch_xinv(Context &c, const XArgs<Real> &xa, const cplx<Real> *spec, cons
     with_line(xa.lp, [&](auto NC) {
         constexpr int N = decltype(NC)::value;
         const XInvPack<Real, FieldSink<Real>> pk{xa, spec, sink};
-        const void *multi = nullptr;
-        if constexpr (N > 0) multi = reinterpret_cast<const void *>(&xinv_multi<Real, FieldSink<Real>, N>);
-        launch_rec(c, multi, grid, block, lds, 3, pk, [&] {
-                       hipLaunchKernelGGL((xinv_kernel<Real, FieldSink<Real>, N>), grid, block, lds, c.stream, xa,
-                                          spec, sink);
-                   });
+        auto launch = [&](auto skew) {
+            constexpr bool SK = decltype(skew)::value;
+            const void *multi = nullptr;
+            if constexpr (N > 0) multi = reinterpret_cast<const void *>(&xinv_multi<Real, FieldSink<Real>, N, SK>);
+            launch_rec(c, multi, grid, block, lds, 3, pk, [&] {
+                hipLaunchKernelGGL((xinv_kernel<Real, FieldSink<Real>, N, SK>), grid, block, lds, c.stream, xa, spec,
+                                   sink);
+            });
+        };
+        if (xa.sw) launch(std::true_type{});
+        else launch(std::false_type{});
     });
 }
 
@@ -478,10 +502,15 @@ void launch_xfwd_stack(Context &c, const XArgs<Real> &xa, const StackMag<Real, S
     const dim3 grid(row_groups, planes, 3 * layers), block((unsigned)((xa.xr / 2) * xa.lp.threads));
     with_line(xa.lp, [&](auto NC) {
         constexpr int N = decltype(NC)::value;
-        if (masked)
-            hipLaunchKernelGGL((xfwd_stack_kernel<Real, S, true, N>), grid, block, lds, c.stream, xa, sm, spec);
-        else
-            hipLaunchKernelGGL((xfwd_stack_kernel<Real, S, false, N>), grid, block, lds, c.stream, xa, sm, spec);
+        auto launch = [&](auto skew) {
+            constexpr bool SK = decltype(skew)::value;
+            if (masked)
+                hipLaunchKernelGGL((xfwd_stack_kernel<Real, S, true, N, SK>), grid, block, lds, c.stream, xa, sm, spec);
+            else
+                hipLaunchKernelGGL((xfwd_stack_kernel<Real, S, false, N, SK>), grid, block, lds, c.stream, xa, sm, spec);
+        };
+        if (xa.sw) launch(std::true_type{});
+        else launch(std::false_type{});
     });
 }
 
@@ -491,7 +520,10 @@ void launch_xinv_stack(Context &c, const XArgs<Real> &xa, const cplx<Real> *spec
     const dim3 grid(row_groups, planes, 3 * layers), block((unsigned)((xa.xr / 2) * xa.lp.threads));
     with_line(xa.lp, [&](auto NC) {
         constexpr int N = decltype(NC)::value;
-        hipLaunchKernelGGL((xinv_stack_kernel<Real, N>), grid, block, lds, c.stream, xa, spec, sf);
+        if (xa.sw)
+            hipLaunchKernelGGL((xinv_stack_kernel<Real, N, true>), grid, block, lds, c.stream, xa, spec, sf);
+        else
+            hipLaunchKernelGGL((xinv_stack_kernel<Real, N, false>), grid, block, lds, c.stream, xa, spec, sf);
     });
 }
 

@@ -100,3 +100,13 @@ def test_classes_off_at_run_time(fa, precision):
         gpu.refresh_observables()
         assert np.abs(gpu.copy_h_demag() - h).max() <= BAR.get(precision, 2e-6) * np.abs(h).max()
     gpu.close()
+
+
+# x frequencies k + 1/2 (slab plans) and integer ones
+@pytest.mark.parametrize("precision", ["double", "mixed", "single"])
+@pytest.mark.parametrize("cells", [(5, 13, 2), (33, 17, 5), (40, 100, 3), (256, 250, 8), (256, 256, 4), (512, 100, 7)])
+def test_skewed_x_frequencies(fa, monkeypatch, cells, precision):
+    n = int(np.prod(cells))
+    mask = (np.random.default_rng(5).random(n) < 0.8).astype(np.uint8) if cells[0] == 33 else None
+    for tune in ("", "skew=0", "fixed=0"):
+        assert field_error(fa, monkeypatch, cells, precision, mask, tune=tune) <= BAR.get(precision, 2e-6)
