@@ -69,6 +69,7 @@ struct DemagPlan {
     bool projection = false;  // no tensor: k-space projection fallback
     int nx = 0, ny = 0, nz = 0;
     int px = 0, py = 0, pz = 1;
+    bool own = false;   // the library's own Newell tensor
     bool skew = false;  // x frequencies k + 1/2 (skew-cyclic convolution along x), fixed at set-up
     int hx = 0;    // columns of the half spectrum: px / 2 (skew), px / 2 + 1
     size_t lds_limit = 65536;  // LDS bytes one workgroup may allocate on this device

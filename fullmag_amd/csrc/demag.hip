@@ -249,9 +249,13 @@ __global__ void __launch_bounds__(256) boundary_corr_kernel(BoundaryCorrArgs<Rea
 // 500x250x8 189 and 167, 256x256x8 116 and 108; FP64 128x128x4 67.8 and 49.5,
 // 128x128x8 90.3 and 67.2, 500x250x4 177 and 146.  With 5 to 8 layers and
 // lines of 32 lanes a workgroup has up to 24 wavefronts of at most 85 FP64
-// values: FP64 spills (250x150x6 108 and 151), and FP32 gains only where the
-// columns divide into full rounds of nz T lanes per component (256x256x6, 2.7
-// rounds, 99 and 102; 256x192x6, 2 rounds, 94 and 90).
+// values: FP64 spills (250x150x6 108 and 151).  FP32 there takes one round of
+// one workgroup per CU for up to 256 slabs, which the skewed x frequencies give
+// (classes and slab: 250x150x6 93.5 and 79.4, 256x256x6 102.2 and 86.8,
+// 500x250x6 153.5 and 140.6, 100x150x7 71.3 and 66.5); a caller's spectra keep
+// px / 2 + 1 slabs, and there it gains only where the columns divide into full
+// rounds of nz T lanes per component (256x256x6, 2.7 rounds, 99 separate and
+// 102; 256x192x6, 2 rounds, 94 and 90).
 template <typename Real>
 bool use_slab(const DemagPlan &dp) {
     if (dp.projection || dp.nz < 2 || dp.pz > z_reg_max<Real>() || !dp.ly.fixed || !slab_length(dp.py)) return false;
@@ -259,7 +263,7 @@ bool use_slab(const DemagPlan &dp) {
     if (bytes > (size_t)dp.tune.slab * 1024 || bytes > dp.lds_limit) return false;
     if (dp.nz <= 4 || fx_lanes(dp.py) < 32) return true;
     const int cols = dp.nz * fx_lanes(dp.py), rounds = (int)cdiv(dp.py, cols);
-    return sizeof(Real) == 4 && 10 * dp.py >= 9 * rounds * cols;
+    return sizeof(Real) == 4 && (dp.own || 10 * dp.py >= 9 * rounds * cols);
 }
 
 // Whether px / 2 workgroups of `lds` bytes, one per column, take fewer rounds
@@ -781,12 +785,12 @@ bool upload_kern(Context &c, const std::vector<double> &kern) {
 // Whether the plan splits its slabs into ky classes: short z lines and a
 // scheduled y length of 320 to 1024 whose slab does not fit the slab kernel.
 // us per Heun step, separate passes and classes: mixed 512x512x4 187.1 and
-// 167.9, 400x400x2 115.8 and 105.0, 300x384x5 145.2 and 133.0, 250x150x6 102.5
-// and 94.8, 100x300x8 104.3 and 96.6, 512x512x8 348.7 and 344.5; FP64
+// 167.9, 400x400x2 115.8 and 105.0, 300x384x5 145.2 and 133.0, 100x300x8 104.3
+// and 96.6, 512x512x8 348.7 and 344.5; FP64
 // 512x512x4 330.9 and 300.3, 200x400x3 126.5 and 118.0.  FP64 with more than
 // four layers needs a component per lane: 512x512x8 651 and 670.  Where both
 // fit, the slab kernel mostly wins (mixed 128x200x7 76.9 against 80.6,
-// 500x250x8 175.7 against 186.5; 256x224x7 119.5 against 108.2).
+// 500x250x8 175.7 against 186.5).
 template <typename Real>
 bool class_rule(const DemagPlan &dp) {
     return dp.three_d && !dp.projection && dp.nz >= 2 && dp.nz <= (sizeof(Real) == 4 ? 8 : 4) && dp.ly.fixed &&
@@ -943,6 +947,7 @@ bool demag_setup(Context &c, const fullmag_fdm_plan_desc &plan, bool newell_on_d
     dp.projection = !have_spectra && !newell_on_device;
     dp.three_d = !(c.nz == 1 && ((have_spectra && plan.demag_kernel_spectrum_len == len2d) ||
                                  (!have_spectra && newell_on_device)));
+    dp.own = !have_spectra && newell_on_device;
     parse_tuning(dp.tune);
     pad_lengths(dp, !have_spectra && newell_on_device && dp.tune.pad != 0, z_reg_max<double>());
     // an even row count keeps two rows of a spectrum column in one 16-byte access
