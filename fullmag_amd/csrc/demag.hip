@@ -266,15 +266,18 @@ bool use_slab(const DemagPlan &dp) {
     return sizeof(Real) == 4 && (dp.own || 10 * dp.py >= 9 * rounds * cols);
 }
 
-// Whether px / 2 workgroups of `lds` bytes, one per column, take fewer rounds
-// over the chip than px / 2 + 1.
-bool saves_round(const DemagPlan &dp, size_t lds, int per_group = 1) {
+template <typename Real>
+bool class_rule(const DemagPlan &dp);
+// Whether workgroups of `lds` bytes, `per_column` for each column or one for
+// `per_group` of them, take fewer rounds over the chip for px / 2 columns than
+// for px / 2 + 1.
+bool saves_round(const DemagPlan &dp, size_t lds, int per_group = 1, int per_column = 1) {
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
         return false;
     const int64_t slots = cus * std::max<int64_t>(1, (int64_t)(dp.lds_limit / lds)), h = dp.px / 2;
-    return cdiv(cdiv(h + 1, per_group), slots) > cdiv(cdiv(h, per_group), slots);
+    return cdiv(per_column * cdiv(h + 1, per_group), slots) > cdiv(per_column * cdiv(h, per_group), slots);
 }
 
 // Whether the x transforms run at the frequencies k + 1/2 (plans with the
@@ -283,13 +286,17 @@ bool saves_round(const DemagPlan &dp, size_t lds, int per_group = 1) {
 // slab kernel's workgroups, one to three per CU, come to whole rounds where
 // px does.  us per mixed Heun step without and with: 256x256x8 117.6 and 94.2
 // (257 slabs of 104 KB are two rounds), 500x250x8 175.3 and 152.5, 256x256x4
-// 73.4 and 71.1, 128x128x8 55.1 and 53.6.  Elsewhere the factors in the x
+// 73.4 and 71.1, 128x128x8 55.1 and 53.6; ky classes where that saves a round,
+// 256x300x8 139.2 and 132.0.  Elsewhere the factors in the x
 // passes cost more than a column: 512x512x8 340 and 345, 512x512x1 73.8 and
 // 75.5, 256x256x64 756 and 768.  In FP64 they cost 2 to 3 us per pass
 // (128x128x4 52 and 57), which only a round saved gives back.
 template <typename Real>
 bool skew_rule(const DemagPlan &dp) {
-    if (dp.tune.skew == 0 || !dp.three_d || !use_slab<Real>(dp)) return false;
+    if (dp.tune.skew == 0 || !dp.three_d) return false;
+    if (!use_slab<Real>(dp))
+        return sizeof(Real) == 4 && class_rule<Real>(dp) &&
+               saves_round(dp, (size_t)3 * dp.nz * fx_size(dp.py / kClasses) * sizeof(cplx<Real>), 1, kClasses);
     return sizeof(Real) == 4 || saves_round(dp, (size_t)3 * dp.nz * fx_size(dp.py) * sizeof(cplx<Real>));
 }
 

@@ -276,6 +276,16 @@ __device__ __forceinline__ void xinv_body(const XArgs<Real> &a, const cplx<Real>
     const int tid = threadIdx.x;
     const int y0 = blockIdx.x * a.xr, z = blockIdx.y;
     const auto roots = x_roots<Real, N>(tid % T, a.tw);
+    // SKEW, FP32: the factors of the outputs a lane stores, ahead of the passes
+    // (128x128x8 mixed 53.4 and 52.4 us per step, 256x256x4 71.1 and 70.5)
+    constexpr int Q4 = SKEW && sizeof(Real) == 4 ? (N / 2 + 4 * T - 1) / (4 * T) : 1;
+    cplx<Real> wq[Q4][4];
+    if constexpr (SKEW && sizeof(Real) == 4) {
+#pragma unroll
+        for (int q = 0; q < Q4; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) wq[q][e] = a.sw[4 * (tid % T + q * T) + e];
+    }
     {
         // lane (j, k0): rows 2j and 2j + 1; consecutive lanes read
         // consecutive rows of one kx column (a row pair is one 16-byte load
@@ -350,7 +360,10 @@ __device__ __forceinline__ void xinv_body(const XArgs<Real> &a, const cplx<Real>
                 if (x < a.n_out) {
                     cplx<Real> v[4];
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] = out(x + e);
+                    for (int e = 0; e < 4; ++e) {
+                        v[e] = line[fxslot<N>(x + e)];
+                        if constexpr (SKEW) v[e] = cmul(v[e], cconj(wq[q][e]));
+                    }
                     auto row = [&](uint32_t k, int part) {
                         float o[4];
 #pragma unroll
@@ -394,14 +407,21 @@ __device__ __forceinline__ void xinv_body(const XArgs<Real> &a, const cplx<Real>
         }
     }
     if constexpr (std::is_same<Sink, FieldSink<float>>::value) {
-        if (!sink.masked() && (a.n_out & 3) == 0 && (sink.n & 3) == 0) {
+        if (2 * a.n_out <= N && !sink.masked() && (a.n_out & 3) == 0 && (sink.n & 3) == 0) {
             // four consecutive outputs of a row per lane and one 16-byte
             // store (rows start on 16-byte boundaries: nx = n_out and n are
             // multiples of four)
-            for (int x = 4 * t; x < a.n_out; x += 4 * T) {
+            constexpr int TT = T, Q = (N / 2 + 4 * TT - 1) / (4 * TT);
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                const int x = 4 * (t + q * TT);
+                if (x >= a.n_out) break;
                 cplx<Real> v[4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = out(x + e);
+                for (int e = 0; e < 4; ++e) {
+                    v[e] = line[fxslot<N>(x + e)];
+                    if constexpr (SKEW) v[e] = cmul(v[e], cconj(wq[q][e]));
+                }
                 const int64_t i = ((int64_t)z * sink.ny + ya) * sink.nx + x;
                 if (ya < a.rows)
                     *reinterpret_cast<float4 *>(sink.out + (int64_t)c * sink.n + i) =

@@ -105,7 +105,7 @@ def test_classes_off_at_run_time(fa, precision):
 # x frequencies k + 1/2 (slab plans) and integer ones
 @pytest.mark.parametrize("precision", ["double", "mixed", "single"])
 @pytest.mark.parametrize("cells", [(5, 13, 2), (33, 17, 5), (40, 100, 3), (256, 250, 8), (256, 256, 4), (512, 100, 7),
-                                   (12, 150, 6), (20, 256, 5)])
+                                   (12, 150, 6), (20, 256, 5), (256, 300, 8), (250, 149, 3)])
 def test_skewed_x_frequencies(fa, monkeypatch, cells, precision):
     n = int(np.prod(cells))
     mask = (np.random.default_rng(5).random(n) < 0.8).astype(np.uint8) if cells[0] == 33 else None
