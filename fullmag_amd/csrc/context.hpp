@@ -88,7 +88,7 @@ struct DemagPlan {
     void *tw_x = nullptr, *tw_y = nullptr, *tw_z = nullptr;
     void *spec = nullptr;
     void *xspec = nullptr;  // x passes' spectrum of rows of xrows entries (ky classes)
-    void *sw = nullptr;     // exp(-i pi d / px) of the displacement d(x) (skew)
+    void *sw = nullptr, *sw64 = nullptr;  // exp(-i pi d / px) of the displacement d(x) (skew), and in FP64
     void *tw_c = nullptr;   // roots of length py / cls
     int cls = 1, xrows = 0;  // ky classes (1: none), fixed at set-up
     void *kern = nullptr;

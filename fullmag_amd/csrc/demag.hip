@@ -492,6 +492,7 @@ void demag_eval_t(Context &c, const S *src, Real *out, bool weight_ms, int phase
     XArgs<Real> xa{};
     xa.tw = static_cast<const cplx<Real> *>(dp.tw_x);
     xa.sw = static_cast<const cplx<Real> *>(dp.sw);
+    xa.sw64 = static_cast<const cplx<double> *>(dp.sw64);
     xa.lp = dp.lx;
     xa.rows = dp.ny;
     xa.n_in = dp.nx;
@@ -553,12 +554,24 @@ bool upload_twiddles(Context &c) {
     for (int n : {dp.px, dp.py, dp.three_d ? dp.pz : 1, dp.cls > 1 ? dp.py / dp.cls : 1})
         for (const cplx<double> &w : twiddle_table(n)) all.push_back({(Real)w.x, (Real)w.y});
     const size_t roots = all.size();
-    if (dp.skew)
-        for (const cplx<double> &w : skew_table(dp.px)) all.push_back({(Real)w.x, (Real)w.y});
+    // FP32: the inputs' factors in FP64 after the tables, on a 16-byte boundary
+    size_t at64 = 0;
+    if (dp.skew) {
+        const std::vector<cplx<double>> w = skew_table(dp.px);
+        for (const cplx<double> &v : w) all.push_back({(Real)v.x, (Real)v.y});
+        if (sizeof(Real) == 4) {
+            at64 = (all.size() + 1) / 2 * 2;
+            all.resize(at64 + 2 * w.size());
+            std::memcpy(&all[at64], w.data(), w.size() * sizeof(w[0]));
+        } else {
+            at64 = roots;
+        }
+    }
     const size_t bytes = all.size() * sizeof(cplx<Real>);
     if (!ctx_alloc(c, &dp.tw_x, bytes, "twiddle tables")) return false;
     dp.tw_y = static_cast<cplx<Real> *>(dp.tw_x) + dp.px;
     dp.sw = dp.skew ? static_cast<cplx<Real> *>(dp.tw_x) + roots : nullptr;
+    dp.sw64 = dp.skew ? static_cast<cplx<Real> *>(dp.tw_x) + at64 : nullptr;
     dp.tw_z = static_cast<cplx<Real> *>(dp.tw_y) + dp.py;
     dp.tw_c = static_cast<cplx<Real> *>(dp.tw_z) + (dp.three_d ? dp.pz : 1);
     return ctx_upload(c, dp.tw_x, all.data(), bytes, "hipMemcpy(twiddles)", c.last_error);
@@ -667,7 +680,7 @@ bool newell_forward(Context &c, const DemagPlan &dp, double z_offset, cplx<doubl
         NewellSource src{d_oct, dp.nx, dp.ny, nzo, dp.px, dp.py, pz, z_even ? 1 : 0};
         XArgs<double> xa{};
         xa.tw = twx;
-        xa.sw = dp.skew ? twx + roots : nullptr;
+        xa.sw = xa.sw64 = dp.skew ? twx + roots : nullptr;
         xa.lp = lx;
         xa.rows = dp.py;
         xa.n_in = dp.px;
@@ -1372,6 +1385,7 @@ void stack_eval_t(Stack &s, const S *const *src) {
     XArgs<Real> xa{};
     xa.tw = static_cast<const cplx<Real> *>(dp.tw_x);
     xa.sw = static_cast<const cplx<Real> *>(dp.sw);
+    xa.sw64 = static_cast<const cplx<double> *>(dp.sw64);
     xa.lp = dp.lx;
     xa.rows = dp.ny;
     xa.n_in = dp.nx;

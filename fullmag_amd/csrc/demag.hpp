@@ -139,7 +139,10 @@ struct XArgs {
     int n_in;         // forward: inputs loaded per row
     int n_out;        // inverse: outputs stored per row
     Real scale;       // inverse: 1/Npad
-    const cplx<Real> *sw;  // frequencies k + 1/2: exp(-i pi d / px) of the displacement d(x) (null: k)
+    // frequencies k + 1/2: exp(-i pi d / px) of the displacement d(x) (null: k),
+    // and the same in FP64 for the inputs
+    const cplx<Real> *sw;
+    const cplx<double> *sw64;
     SpecGeom g;
 };
 
@@ -158,32 +161,27 @@ struct MagSource {
     // boundary tiers: every cell packs phi Ms m, mask or not (the volume
     // fraction in the field's precision)
     const Real *phi;
-    __device__ Real operator()(int c, int z, int y, int x) const {
+    __device__ double at(int c, int z, int y, int x) const {
         const int64_t i = ((int64_t)z * ny + y) * nx + x;
-        if (phi) return Real(double(m[(int64_t)c * n + i]) * (double(phi[i]) * (ms_cell ? ms_cell[i] : ms)));
-        if (mask && !mask[i]) return Real(0);
+        if (phi) return double(m[(int64_t)c * n + i]) * (double(phi[i]) * (ms_cell ? ms_cell[i] : ms));
+        if (mask && !mask[i]) return 0.0;
         const double w = ms_cell ? ms_cell[i] : ms;
-        return Real(double(m[(int64_t)c * n + i]) * w);
+        return double(m[(int64_t)c * n + i]) * w;
     }
-    // No mask and no per-cell Ms: the value is one unconditional load, so a
-    // lane's loads can all be issued before any of them is used.
-    __device__ bool uniform() const { return !mask && !ms_cell && !phi; }
-    __device__ Real uniform_at(int c, int z, int y, int x) const {
-        return Real(double(m[(int64_t)c * n + ((int64_t)z * ny + y) * nx + x]) * ms);
-    }
-    // operator()'s value with every load unconditional (an absent array is
-    // read from a stand-in and its value replaced after the load), so a
-    // lane's loads all issue before the first is used.
-    static constexpr bool kGather = GATHER;
-    __device__ Real gather_at(int c, int z, int y, int x) const {
+    // The value with every load unconditional, so that a lane's loads all issue
+    // before the first is used.  Without GATHER (no mask, no per-cell Ms) that is
+    // one load; with it an absent array is read from a stand-in and its value
+    // replaced after the load.
+    __device__ double load(int c, int z, int y, int x) const {
         const int64_t i = ((int64_t)z * ny + y) * nx + x;
         const double mv = double(m[(int64_t)c * n + i]);
+        if constexpr (!GATHER) return mv * ms;
         const double pv = double(*(phi ? phi + i : no_array<Real>()));
         const double cv = *(ms_cell ? ms_cell + i : &kNoArrayF64);
         const uint8_t kv = *(mask ? mask + i : &kNoMask);
         const double w = ms_cell ? cv : ms;
         const bool live = phi || kv != 0;
-        return live ? Real(mv * (phi ? pv * w : w)) : Real(0);
+        return live ? mv * (phi ? pv * w : w) : 0.0;
     }
 };
 
@@ -195,11 +193,7 @@ struct NewellSource {
     const double *oct;  // [6][nz][ny][nx]
     int nx, ny, nz, px, py, pz;
     int z_even;  // the cross-layer kernel: mirrored z slots keep every sign (newell.rs:630-647)
-    __device__ bool uniform() const { return false; }
-    __device__ double uniform_at(int, int, int, int) const { return 0.0; }
-    [[maybe_unused]] static constexpr bool kGather = false;  // read by the fixed-length x pass only
-    __device__ double gather_at(int, int, int, int) const { return 0.0; }
-    __device__ double operator()(int c, int zz, int yy, int x) const {
+    __device__ double at(int c, int zz, int yy, int x) const {
         if ((x >= nx && x <= px - nx) || (yy >= ny && yy <= py - ny) || (pz > 1 && zz >= nz && zz <= pz - nz))
             return 0.0;
         const int xi = x < nx ? x : px - x;

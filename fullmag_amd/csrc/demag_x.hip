@@ -17,6 +17,16 @@ __device__ __forceinline__ void xfwd_split(cplx<Real> zk, cplx<Real> zn, cplx<Re
     B = {h * (zk.y + zn.y), h * (zn.x - zk.x)};
 }
 
+// (a + i b) w, rounded once, as the inputs of a plan at integer frequencies
+// are: Ms m rounded to FP32 and multiplied by an FP32 factor gave smooth states
+// up to a fifth more error (rms of H_demag against FP64, 128x128x4 mixed: 3.0e-7
+// at integer frequencies, 3.6e-7 so, 3.4e-7 with this product and 3.2e-7 with the
+// exact powers of x_roots as well; 44.3, 44.3, 45.0 and 44.9 us per step).
+template <typename Real>
+__device__ __forceinline__ cplx<Real> skewed(double a, double b, const cplx<double> &w) {
+    return {Real(a * w.x - b * w.y), Real(a * w.y + b * w.x)};
+}
+
 // Runtime-planned lines.
 template <typename Real, class Src>
 __device__ __forceinline__ void xfwd_body_rt(const XArgs<Real> &a, const Src &src, cplx<Real> *spec, int c) {
@@ -32,9 +42,10 @@ __device__ __forceinline__ void xfwd_body_rt(const XArgs<Real> &a, const Src &sr
     for (int x = t; x < n; x += T) {
         cplx<Real> v = {Real(0), Real(0)};
         if (x < a.n_in) {
-            if (ya < a.rows) v.x = src(c, z, ya, x);
-            if (ya + 1 < a.rows) v.y = src(c, z, ya + 1, x);
-            if (a.sw) v = cmul(v, a.sw[x]);
+            const double va = ya < a.rows ? src.at(c, z, ya, x) : 0.0;
+            const double vb = ya + 1 < a.rows ? src.at(c, z, ya + 1, x) : 0.0;
+            if (a.sw64) v = skewed<Real>(va, vb, a.sw64[x]);
+            else v = {Real(va), Real(vb)};
         }
         line[lslot(a.lp, x)] = v;
     }
@@ -55,10 +66,16 @@ __device__ __forceinline__ void xfwd_body_rt(const XArgs<Real> &a, const Src &sr
 
 // Roots ahead of the passes (FxRoots) for powers of two; the other lengths'
 // last pass has up to seven butterflies per lane (400x100x2 FP64, 896 points:
-// 66.2 us per step with the table, 67.7 with the roots ahead).
-template <typename Real, int N>
+// 66.2 us per step with the table, 67.7 with the roots ahead).  FP32 at the
+// frequencies k + 1/2 forms EXACT powers: a state's mean, which integer
+// frequencies keep at k = 0 away from every twiddle, spreads over all of them
+// there.  At integer frequencies they would cost more than they give (all lines
+// so: 512x512x1 mixed 74.3 -> 76.2 us per step, 512x512x8 341 -> 349).
+template <typename Real, int N, bool SKEW>
 __device__ __forceinline__ auto x_roots(int t, const cplx<Real> *tw) {
-    if constexpr (fx_odd(N) == 1) return FxRoots<Real, N>(t, tw);
+    constexpr bool EXACT = SKEW && sizeof(Real) == 4;
+    if constexpr (fx_odd(N) == 1) return FxRoots<Real, N, EXACT>(t, tw);
+    else if constexpr (EXACT) return FxTable<Real>{tw};
     else return tw;
 }
 
@@ -83,33 +100,29 @@ __device__ __forceinline__ void xfwd_body(const XArgs<Real> &a, const Src &src, 
         // (n_in <= N / 2) and are not loaded
         const bool oka = ya < a.rows, okb = ya + 1 < a.rows;
         const int yA = oka ? ya : 0, yB = okb ? ya + 1 : 0;
+        double va[E / 2], vb[E / 2];
 #pragma unroll
         for (int e = 0; e < E / 2; ++e) {
             const int x = t + e * T;
             const bool okx = x < a.n_in;
             const int xs = okx ? x : 0;
-            Real va, vb;
-            if constexpr (Src::kGather) {
-                // the mask, volume fraction and per-cell Ms are read beside
-                // each element, all unconditionally
-                va = src.gather_at(c, z, yA, xs);
-                vb = src.gather_at(c, z, yB, xs);
-            } else {
-                va = src.uniform_at(c, z, yA, xs);
-                vb = src.uniform_at(c, z, yB, xs);
-            }
-            v[e] = {(okx && oka) ? va : Real(0), (okx && okb) ? vb : Real(0)};
+            const double qa = src.load(c, z, yA, xs), qb = src.load(c, z, yB, xs);
+            va[e] = (okx && oka) ? qa : 0.0;
+            vb[e] = (okx && okb) ? qb : 0.0;
+        }
+        if constexpr (SKEW) {
+            cplx<double> w[E / 2];
+#pragma unroll
+            for (int e = 0; e < E / 2; ++e) w[e] = a.sw64[t + e * T];
+#pragma unroll
+            for (int e = 0; e < E / 2; ++e) v[e] = skewed<Real>(va[e], vb[e], w[e]);
+        } else {
+#pragma unroll
+            for (int e = 0; e < E / 2; ++e) v[e] = {Real(va[e]), Real(vb[e])};
         }
 #pragma unroll
         for (int e = E / 2; e < E; ++e) v[e] = {Real(0), Real(0)};
-        if constexpr (SKEW) {
-            cplx<Real> w[E / 2];
-#pragma unroll
-            for (int e = 0; e < E / 2; ++e) w[e] = a.sw[t + e * T];
-#pragma unroll
-            for (int e = 0; e < E / 2; ++e) v[e] = cmul(v[e], w[e]);
-        }
-        const auto roots = x_roots<Real, N>(t, a.tw);
+        const auto roots = x_roots<Real, N, SKEW>(t, a.tw);
         fx_first_pass<Real, N>(line, t, v, a.tw, false);
         fx_rest<Real, N>(line, t, roots, false);
     }
@@ -275,7 +288,7 @@ __device__ __forceinline__ void xinv_body(const XArgs<Real> &a, const cplx<Real>
     const int LINES = a.xr >> 1, ls = a.ls;
     const int tid = threadIdx.x;
     const int y0 = blockIdx.x * a.xr, z = blockIdx.y;
-    const auto roots = x_roots<Real, N>(tid % T, a.tw);
+    const auto roots = x_roots<Real, N, SKEW>(tid % T, a.tw);
     // SKEW, FP32: the factors of the outputs a lane stores, ahead of the passes
     // (128x128x8 mixed 53.4 and 52.4 us per step, 256x256x4 71.1 and 70.5)
     constexpr int Q4 = SKEW && sizeof(Real) == 4 ? (N / 2 + 4 * T - 1) / (4 * T) : 1;

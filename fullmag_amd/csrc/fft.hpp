@@ -262,43 +262,46 @@ __device__ __forceinline__ void dft_any(cplx<T> *v, const cplx<T> *tw, int n, bo
 }
 
 // v[r] *= w^(r st), r = 1..R-1, where w^t = tw[t] (r st < n).  For
-// power-of-two R only the roots w^(2^b st) are read from the table; each
-// other power is one product of an earlier power and a table root, so no
-// twiddle carries more than three extra roundings.
-template <int R>
-constexpr int root_bits() {
-    return R == 2 ? 1 : R == 4 ? 2 : R == 8 ? 3 : 4;
+// power-of-two R the roots w^(2^b st) are read from the table; each other power
+// is one product of an earlier power and a table root, so no twiddle carries
+// more than three extra roundings.  EXACT reads w^3 and w^12 too and forms the
+// others as one product of w^1, w^2 or w^3 and w^4, w^8 or w^12.
+template <int R, bool EXACT>
+constexpr int root_count() {
+    return R == 2 ? 1 : R == 4 ? 2 : R == 8 ? (EXACT ? 4 : 3) : EXACT ? 6 : 4;
 }
-// The same for power-of-two R with the roots w^(2^b st) in hand.
-template <typename T, int R>
+template <bool EXACT>
+constexpr int root_power(int i) {
+    return !EXACT ? 1 << i : i < 3 ? i + 1 : 4 * (i - 2);
+}
+// The same for power-of-two R with the roots in hand.
+template <typename T, int R, bool EXACT = false>
 __device__ __forceinline__ void twiddle_by(cplx<T> *v, const cplx<T> *roots, bool inv) {
-    constexpr int LB = root_bits<R>();
     // conjugation for the inverse as a product with -1 (exact), so the
     // table loads stay out of any branch
     const T sg = inv ? T(-1) : T(1);
-    cplx<T> pw[LB];
-#pragma unroll
-    for (int b = 0; b < LB; ++b) {
-        pw[b] = roots[b];
-        pw[b].y *= sg;
-    }
     cplx<T> w[R];
+#pragma unroll
+    for (int i = 0; i < root_count<R, EXACT>(); ++i) w[root_power<EXACT>(i)] = {roots[i].x, sg * roots[i].y};
 #pragma unroll
     for (int r = 1; r < R; ++r) {
         const int low = r & -r;
-        const int lb = low == 1 ? 0 : low == 2 ? 1 : low == 4 ? 2 : 3;
-        w[r] = (r == low) ? pw[lb] : cmul(w[r - low], pw[lb]);
+        if (!EXACT || R == 4) {
+            if (r != low) w[r] = cmul(w[r - low], w[low]);
+        } else if (r > 4 && r % 4 != 0) {
+            w[r] = cmul(w[r & ~3], w[r & 3]);
+        }
         v[r] = cmul(v[r], w[r]);
     }
 }
-template <typename T, int R>
+template <typename T, int R, bool EXACT = false>
 __device__ __forceinline__ void twiddle(cplx<T> *v, const cplx<T> *tw, int st, bool inv) {
     if constexpr (R == 2 || R == 4 || R == 8 || R == 16) {
-        constexpr int LB = root_bits<R>();
+        constexpr int LB = root_count<R, EXACT>();
         cplx<T> pw[LB];
 #pragma unroll
-        for (int b = 0; b < LB; ++b) pw[b] = tw[st << b];
-        twiddle_by<T, R>(v, pw, inv);
+        for (int b = 0; b < LB; ++b) pw[b] = tw[root_power<EXACT>(b) * st];
+        twiddle_by<T, R, EXACT>(v, pw, inv);
     } else {
         const T sg = inv ? T(-1) : T(1);
 #pragma unroll
@@ -511,7 +514,7 @@ __device__ __forceinline__ void pass_sync() {
 // 250x150x6 single 94.8 -> 93.5.  In the film's y convolution they cost
 // registers (512x512x1 FP64 90.1 -> 91.9 us) and in the slab kernel they gave
 // nothing.
-template <typename T, int N>
+template <typename T, int N, bool EXACT = false>
 struct FxRoots {
     static_assert(fx_npass(N) <= 3, "two passes of roots");
     cplx<T> w[2][8];
@@ -521,15 +524,22 @@ struct FxRoots {
     }
     template <int P, int NS>
     __device__ __forceinline__ void fetch(int t, const cplx<T> *tw) {
-        constexpr int R = fx_radix(N, P), NT = fx_lanes(N), NR = N / R, MB = (NR + NT - 1) / NT, LB = root_bits<R>();
+        constexpr int R = fx_radix(N, P), NT = fx_lanes(N), NR = N / R, MB = (NR + NT - 1) / NT;
+        constexpr int LB = root_count<R, EXACT>();
         static_assert(MB * LB <= 8, "roots of one pass");
 #pragma unroll
         for (int b = 0; b < MB; ++b) {
             const int j0 = t + b * NT, j = MB * NT == NR || j0 < NR ? j0 : 0;
 #pragma unroll
-            for (int i = 0; i < LB; ++i) w[P - 1][b * LB + i] = tw[((j % NS) * (N / (NS * R))) << i];
+            for (int i = 0; i < LB; ++i) w[P - 1][b * LB + i] = tw[root_power<EXACT>(i) * ((j % NS) * (N / (NS * R)))];
         }
     }
+};
+
+// The table, its powers EXACT.
+template <typename T>
+struct FxTable {
+    const cplx<T> *tw;
 };
 
 // One pass.  LAST: output element i goes to put(i, value) instead of LDS, and
@@ -552,8 +562,14 @@ __device__ __forceinline__ void fx_pass(cplx<T> *line, int t, const Tw &tw, bool
         for (int r = 0; r < R; ++r) v[b][r] = p[r * (NR + NR / G)];
         // k = 0 multiplies by the table's exact w^0 = 1 (no branch: lanes of
         // one wave differ in k, and a branch would split the table loads)
-        if constexpr (std::is_same<Tw, FxRoots<T, N>>::value) twiddle_by<T, R>(v[b], tw.w[P - 1] + b * root_bits<R>(), inv);
-        else twiddle<T, R>(v[b], tw, k * ST, inv);
+        if constexpr (std::is_same<Tw, FxRoots<T, N, true>>::value)
+            twiddle_by<T, R, true>(v[b], tw.w[P - 1] + b * root_count<R, true>(), inv);
+        else if constexpr (std::is_same<Tw, FxRoots<T, N>>::value)
+            twiddle_by<T, R>(v[b], tw.w[P - 1] + b * root_count<R, false>(), inv);
+        else if constexpr (std::is_same<Tw, FxTable<T>>::value)
+            twiddle<T, R, true>(v[b], tw.tw, k * ST, inv);
+        else
+            twiddle<T, R>(v[b], tw, k * ST, inv);
         dft_any<T, R>(v[b], nullptr, N, inv);
         base[b] = (j / NS) * NS * R + k;
     }
