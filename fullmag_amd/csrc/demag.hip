@@ -63,8 +63,12 @@ size_t lds_budget() { return 65536; }
 // Rows per x workgroup: the largest power of two <= 16 whose packed lines fit
 // in 64 KB of LDS (padded stride when that still fits) and 512 lanes; a line
 // longer than 64 KB takes one packed line (two rows) per workgroup when it
-// fits in `limit`, the device's LDS per workgroup (160 KB on gfx950).
+// fits in `limit`, the device's LDS per workgroup (160 KB on gfx950).  The
+// kernels take pairs of rows, a power of two of them: `max_rows` is rounded
+// down to one, and at least 2.
 bool pick_x(const LinePlan &lp, size_t ce, int &xr, int &ls, int max_rows = 16, size_t limit = 65536) {
+    while (max_rows & (max_rows - 1)) max_rows &= max_rows - 1;
+    max_rows = std::max(2, max_rows);
     if (lp.fixed) {
         // two workgroups of a CU's 160 KB; a line distance of 4 mod 32 slots
         // puts eight lines read at one element index on different banks
