@@ -262,7 +262,9 @@ __global__ void __launch_bounds__(256) boundary_corr_kernel(BoundaryCorrArgs<Rea
 // 102; 256x192x6, 2 rounds, 94 and 90).
 template <typename Real>
 bool use_slab(const DemagPlan &dp) {
-    if (dp.projection || dp.nz < 2 || dp.pz > z_reg_max<Real>() || !dp.ly.fixed || !slab_length(dp.py)) return false;
+    if (dp.tune.slab <= 0 || dp.projection || dp.nz < 2 || dp.pz > z_reg_max<Real>() || !dp.ly.fixed ||
+        !slab_length(dp.py))
+        return false;
     const size_t bytes = (size_t)3 * dp.nz * fx_size(dp.py) * sizeof(cplx<Real>);
     if (bytes > (size_t)dp.tune.slab * 1024 || bytes > dp.lds_limit) return false;
     if (dp.nz <= 4 || fx_lanes(dp.py) < 32) return true;

@@ -39,3 +39,22 @@ def test_rows_per_x_workgroup(fa, monkeypatch, rows, cells, more, precision):
     gpu = backend(fa, cells, precision)
     assert np.abs(gpu.copy_h_demag() - h).max() <= bar
     gpu.close()
+
+
+@pytest.mark.parametrize("precision", ["double", "mixed"])
+@pytest.mark.parametrize("slab", [-1, 0, 1, 160])
+def test_slab_kernel_by_its_knob(fa, monkeypatch, slab, precision):
+    """The slab kernel runs where its 17 KB (FP64: 34) fit the knob's KB; 0 and
+    below turn it off."""
+    monkeypatch.setenv("FULLMAG_FDM_TUNE", "skew=0")
+    gpu = backend(fa, (40, 100, 3), precision)
+    h = gpu.copy_h_demag()
+    gpu.set_schedule(f"slab={slab}")
+    gpu.set_timing(True)
+    gpu.refresh_observables()
+    gpu.step(1e-14)
+    assert ("demag_yz_slab" in gpu.timings()) == (slab == 160)
+    gpu.upload_magnetization(fa.generate_random_unit_vectors(17 + 12000, 12000))
+    gpu.refresh_observables()
+    assert np.abs(gpu.copy_h_demag() - h).max() <= BAR[precision] * np.abs(h).max()
+    gpu.close()
