@@ -19,6 +19,7 @@
 #include "fullmag_fdm_ext.h"
 
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -208,8 +209,11 @@ struct Context {
     void *adj_g = nullptr, *adj_q = nullptr, *adj_w = nullptr;                          // Real
     double *adj_lu = nullptr, *adj_lmt = nullptr;
 
-    // scratch of the AoS <-> SoA transfers (allocated by the first one)
+    // scratch of the AoS <-> SoA transfers (allocated by the first one, the
+    // upload of the initial m), held by one transfer at a time: several host
+    // threads may copy fields of one backend
     void *d_xfer = nullptr;
+    std::mutex xfer_mutex;
 
     // scratch for previews
     void *d_preview = nullptr;

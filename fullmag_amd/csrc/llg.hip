@@ -974,6 +974,7 @@ static bool xfer_scratch(Context &c) {
 }
 
 int state_from_host(Context &c, const void *host, bool host_f64) {
+    const std::lock_guard<std::mutex> lock(c.xfer_mutex);
     if (!xfer_scratch(c)) return 0;
     const size_t hb = host_f64 ? 8 : 4;
     const int64_t n = (int64_t)c.n;
@@ -1002,6 +1003,7 @@ int state_from_host(Context &c, const void *host, bool host_f64) {
 }
 
 int field_to_host(Context &c, const void *field, bool field_f64, void *out, bool out_f64) {
+    const std::lock_guard<std::mutex> lock(c.xfer_mutex);
     if (!xfer_scratch(c)) return 0;
     const size_t ob = out_f64 ? 8 : 4;
     const int64_t n = (int64_t)c.n;
