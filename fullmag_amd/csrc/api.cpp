@@ -11,6 +11,7 @@
 #include <cstddef>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <new>
 #include <optional>
@@ -356,24 +357,18 @@ template <typename T>
 bool download_soa(Context &c, const void *dev, size_t elem, T *out) {
     if (const int done = field_to_host(c, dev, elem == 8, out, sizeof(T) == 8)) return done > 0;
     const uint64_t n = c.n;
-    if (elem == 8) {
-        std::vector<double> h(3 * n);
-        if (!hip_ok(hipMemcpyAsync(h.data(), dev, h.size() * 8, hipMemcpyDeviceToHost, c.stream), "hipMemcpy(field)",
-                    c.last_error) ||
+    auto convert = [&](auto real) {
+        using Real = decltype(real);
+        const std::unique_ptr<Real[]> h(new Real[3 * n]);
+        if (!hip_ok(hipMemcpyAsync(h.get(), dev, 3 * n * sizeof(Real), hipMemcpyDeviceToHost, c.stream),
+                    "hipMemcpy(field)", c.last_error) ||
             !hip_ok(hipStreamSynchronize(c.stream), "hipMemcpy(field)", c.last_error))
             return false;
         for (uint64_t i = 0; i < n; ++i)
             for (int k = 0; k < 3; ++k) out[3 * i + k] = (T)h[k * n + i];
-    } else {
-        std::vector<float> h(3 * n);
-        if (!hip_ok(hipMemcpyAsync(h.data(), dev, h.size() * 4, hipMemcpyDeviceToHost, c.stream), "hipMemcpy(field)",
-                    c.last_error) ||
-            !hip_ok(hipStreamSynchronize(c.stream), "hipMemcpy(field)", c.last_error))
-            return false;
-        for (uint64_t i = 0; i < n; ++i)
-            for (int k = 0; k < 3; ++k) out[3 * i + k] = (T)h[k * n + i];
-    }
-    return true;
+        return true;
+    };
+    return elem == 8 ? convert(double()) : convert(float());
 }
 
 // Resolves an observable to its device buffer; null buffer means all-zero.

@@ -3,6 +3,7 @@
 #include "context.hpp"
 
 #include <cstring>
+#include <memory>
 
 namespace fm {
 
@@ -56,30 +57,21 @@ void ctx_free_all(Context &c) {
 bool ctx_upload_m(Context &c, const void *host, bool host_is_f64) {
     if (const int done = state_from_host(c, host, host_is_f64)) return done > 0;
     const uint64_t n = c.n;
-    auto get = [&](uint64_t i) -> double {
-        return host_is_f64 ? static_cast<const double *>(host)[i] : (double)static_cast<const float *>(host)[i];
+    auto convert = [&](auto state) {
+        using State = decltype(state);
+        const std::unique_ptr<State[]> s(new State[3 * n]);
+        for (uint64_t i = 0; i < n; ++i) {
+            const bool act = !c.has_mask || c.mask_host[i] != 0;
+            for (int k = 0; k < 3; ++k)
+                s[k * n + i] = !act          ? State(0)
+                               : host_is_f64 ? State(static_cast<const double *>(host)[3 * i + k])
+                                             : State(static_cast<const float *>(host)[3 * i + k]);
+        }
+        return hip_ok(hipMemcpyAsync(c.m, s.get(), 3 * n * sizeof(State), hipMemcpyHostToDevice, c.stream),
+                      "hipMemcpy(m)", c.last_error) &&
+               hip_ok(hipStreamSynchronize(c.stream), "hipMemcpy(m)", c.last_error);
     };
-    bool ok;
-    if (c.state_bytes() == 8) {
-        std::vector<double> s(3 * n);
-        for (uint64_t i = 0; i < n; ++i) {
-            const bool act = !c.has_mask || c.mask_host[i] != 0;
-            for (int k = 0; k < 3; ++k) s[k * n + i] = act ? get(3 * i + k) : 0.0;
-        }
-        ok = hip_ok(hipMemcpyAsync(c.m, s.data(), s.size() * sizeof(double), hipMemcpyHostToDevice, c.stream),
-                    "hipMemcpy(m)", c.last_error);
-        ok = ok && hip_ok(hipStreamSynchronize(c.stream), "hipMemcpy(m)", c.last_error);
-    } else {
-        std::vector<float> s(3 * n);
-        for (uint64_t i = 0; i < n; ++i) {
-            const bool act = !c.has_mask || c.mask_host[i] != 0;
-            for (int k = 0; k < 3; ++k) s[k * n + i] = act ? (float)get(3 * i + k) : 0.0f;
-        }
-        ok = hip_ok(hipMemcpyAsync(c.m, s.data(), s.size() * sizeof(float), hipMemcpyHostToDevice, c.stream),
-                    "hipMemcpy(m)", c.last_error);
-        ok = ok && hip_ok(hipStreamSynchronize(c.stream), "hipMemcpy(m)", c.last_error);
-    }
-    return ok;
+    return c.state_bytes() == 8 ? convert(double()) : convert(float());
 }
 
 bool ctx_query_device_info(Context &c) {

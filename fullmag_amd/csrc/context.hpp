@@ -209,9 +209,9 @@ struct Context {
     void *adj_g = nullptr, *adj_q = nullptr, *adj_w = nullptr;                          // Real
     double *adj_lu = nullptr, *adj_lmt = nullptr;
 
-    // scratch of the AoS <-> SoA transfers (allocated by the first one, the
-    // upload of the initial m), held by one transfer at a time: several host
-    // threads may copy fields of one backend
+    // scratch of the AoS <-> SoA transfers (allocated by the first one that
+    // converts on the device, 24 bytes per cell up to 48 MiB), held by one
+    // transfer at a time: several host threads may copy fields of one backend
     void *d_xfer = nullptr;
     std::mutex xfer_mutex;
 
@@ -355,7 +355,8 @@ bool preview_field(Context &c, const void *field, bool field_f64, uint32_t pnx, 
                    uint32_t z0, uint32_t zs, void *dev_out, bool out_f64);
 // Whole-field transfers between a host AoS array and a device SoA field,
 // converted on the device and complete on return: 1 done, -1 failed
-// (last_error), 0 no device memory for the scratch (convert on the host).
+// (last_error), 0 for the host to convert: few cells, or no device memory for
+// the scratch.
 int state_from_host(Context &c, const void *host, bool host_f64);
 int field_to_host(Context &c, const void *field, bool field_f64, void *out, bool out_f64);
 bool alloc_integrator_buffers(Context &c);

@@ -119,7 +119,8 @@ __global__ void __launch_bounds__(256) preview_kernel(const In *fx, const In *fy
 
 // Host arrays are AoS, device fields SoA: these two convert between a raw copy
 // of the host array and a field, in the precisions of both, so that the host
-// touches every value once, in the copy (converting on one host thread took
+// touches every value once, in the copy (for fields large enough, kUploadCells
+// and kCopyCells; converting on one host thread took
 // 2.9 ms for the upload and two field copies of a 256x256x8 backend that its
 // GPU work fills for 0.1 ms).  Inactive cells of an uploaded state are zero.
 template <typename In, typename State>
@@ -963,6 +964,18 @@ bool materialize_observables(Context &c) {
 // Cells converted per pass: bounds the transfer scratch to 48 MiB.
 constexpr uint64_t kXferCells = uint64_t(1) << 21;
 
+// Cells from which a whole-field transfer converts on the device, by the FP64
+// (1) or FP32 (0) scalars of the device's side and the host's.  Below them the
+// conversion's launch costs more than the host's loop.  us per call, host and
+// device: upload of FP64 to FP64 1024 cells 11 and 23, 28672 42 and 45, 40960 57
+// and 55; copy FP64 to FP64 1024 cells 11 and 28, 40960 67 and 70, 49152 104 and
+// 99; FP32 to FP32 65536 cells 57 and 61, 98304 104 and 98.  A copy of an FP32
+// field to FP64 moves twice the bytes when the device widens it (1048576 cells
+// 1284 and 1517, 2097152 cells 4207 and 4839), until the host's array is one
+// that malloc maps anew on each call (3145728 cells 13455 and 7152).
+constexpr uint64_t kUploadCells[2][2] = {{32768, 98304}, {16384, 32768}};
+constexpr uint64_t kCopyCells[2][2] = {{81920, 2621440}, {24576, 45056}};
+
 static bool xfer_scratch(Context &c) {
     if (c.d_xfer) return true;
     const uint64_t cells = std::min<uint64_t>(c.n, kXferCells);
@@ -974,6 +987,7 @@ static bool xfer_scratch(Context &c) {
 }
 
 int state_from_host(Context &c, const void *host, bool host_f64) {
+    if (c.n < kUploadCells[c.state_bytes() == 8][host_f64]) return 0;
     const std::lock_guard<std::mutex> lock(c.xfer_mutex);
     if (!xfer_scratch(c)) return 0;
     const size_t hb = host_f64 ? 8 : 4;
@@ -1003,6 +1017,7 @@ int state_from_host(Context &c, const void *host, bool host_f64) {
 }
 
 int field_to_host(Context &c, const void *field, bool field_f64, void *out, bool out_f64) {
+    if (c.n < kCopyCells[field_f64][out_f64]) return 0;
     const std::lock_guard<std::mutex> lock(c.xfer_mutex);
     if (!xfer_scratch(c)) return 0;
     const size_t ob = out_f64 ? 8 : 4;
