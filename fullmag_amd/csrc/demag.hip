@@ -594,6 +594,24 @@ void pad_lengths(DemagPlan &dp, bool free, int z_keep) {
     dp.hx = dp.px / 2 + (dp.skew ? 0 : 1);
 }
 
+// Device bytes that the Newell set-up holds at once: the FP64 spectrum of the
+// padded tensor and its octant, and `kept` complex and `tensor` real values of
+// `real` bytes per component, plane and column that stay.
+size_t setup_bytes(const DemagPlan &dp, size_t kept, size_t tensor, size_t real) {
+    const size_t hx = dp.px / 2 + 1, cells = (size_t)dp.nx * dp.ny * dp.nz;
+    return 6 * (size_t)dp.pz * hx * dp.py * sizeof(cplx<double>) + 6 * cells * sizeof(double) +
+           (2 * kept + tensor) * hx * real;
+}
+
+// Whether `bytes` and a margin for the small tables are free on the device.
+// Lines longer than 2n take up to 4/3 of the memory per axis (800 cells along
+// each of three axes: 413 GB for the set-up's spectrum at 2048 points, 197 GB at
+// 1600), so a grid whose padded set-up does not fit keeps 2n.
+bool fits_device(size_t bytes) {
+    size_t free = 0, total = 0;
+    return hipMemGetInfo(&free, &total) != hipSuccess || bytes + (size_t(64) << 20) <= free;
+}
+
 bool plan_lines(DemagPlan &dp, std::string &err) {
     const DemagTuning &t = dp.tune;
     const bool fx = t.fixed != 0;
@@ -975,7 +993,12 @@ bool demag_setup(Context &c, const fullmag_fdm_plan_desc &plan, bool newell_on_d
                                  (!have_spectra && newell_on_device)));
     dp.own = !have_spectra && newell_on_device;
     parse_tuning(dp.tune);
-    pad_lengths(dp, !have_spectra && newell_on_device && dp.tune.pad != 0, z_reg_max<double>());
+    pad_lengths(dp, dp.own && dp.tune.pad != 0, z_reg_max<double>());
+    if (dp.own && (dp.px > 2 * dp.nx || dp.py > 2 * dp.ny || (dp.three_d && dp.pz > 2 * dp.nz))) {
+        const size_t planes = dp.three_d ? 3 * (size_t)dp.nz : 3, oy = dp.py / 2 + 1, oz = dp.three_d ? dp.pz / 2 + 1 : 1;
+        const size_t need = setup_bytes(dp, planes * dp.py, (dp.three_d ? 6 : 4) * oz * oy, c.real_bytes());
+        if (!fits_device(need)) pad_lengths(dp, false, 0);
+    }
     // an even row count keeps two rows of a spectrum column in one 16-byte access
     dp.rows = dp.three_d ? dp.py : dp.ny + (dp.ny & 1);
     dp.kcomp = dp.three_d ? 6 : 4;
@@ -1229,7 +1252,27 @@ bool stack_setup_t(Stack &s, std::string &err) {
     DemagTuning tune;
     parse_tuning(tune);
     dp.tune.y_split = tune.y_split;
+    // pair kernels: the self kernel once, one shifted kernel per distinct
+    // z distance dst - src (compared exactly)
+    std::vector<double> shifts;
+    s.pair.assign((size_t)L * L, 0);
+    for (int d = 0; d < L; ++d)
+        for (int q = 0; q < L; ++q) {
+            if (d == q) continue;
+            const double sh = s.oz[d] - s.oz[q];
+            auto it = std::find(shifts.begin(), shifts.end(), sh);
+            if (it == shifts.end()) {
+                shifts.push_back(sh);
+                it = shifts.end() - 1;
+            }
+            s.pair[(size_t)d * L + q] = 1 + (int)(it - shifts.begin());
+        }
+    s.nkern = 1 + (int)shifts.size();
     pad_lengths(dp, true, 0);
+    if (dp.px > 2 * dp.nx || dp.py > 2 * dp.ny || (dp.three_d && dp.pz > 2 * dp.nz)) {
+        const size_t points = (size_t)dp.pz * dp.py;
+        if (!fits_device(setup_bytes(dp, 6 * points * L, 6 * points * s.nkern, c.real_bytes()))) pad_lengths(dp, false, 0);
+    }
     dp.rows = dp.py;
     dp.inv_npad = 1.0 / ((double)dp.px * dp.py * dp.pz);
     dp.lds_limit = device_lds_limit(c.device);
@@ -1277,22 +1320,6 @@ bool stack_setup_t(Stack &s, std::string &err) {
         err = c.last_error;
         return false;
     }
-    // pair kernels: the self kernel once, one shifted kernel per distinct
-    // z distance dst - src (compared exactly)
-    std::vector<double> shifts;
-    s.pair.assign((size_t)L * L, 0);
-    for (int d = 0; d < L; ++d)
-        for (int q = 0; q < L; ++q) {
-            if (d == q) continue;
-            const double sh = s.oz[d] - s.oz[q];
-            auto it = std::find(shifts.begin(), shifts.end(), sh);
-            if (it == shifts.end()) {
-                shifts.push_back(sh);
-                it = shifts.end() - 1;
-            }
-            s.pair[(size_t)d * L + q] = 1 + (int)(it - shifts.begin());
-        }
-    s.nkern = 1 + (int)shifts.size();
     s.kern_stride = s.fused ? 6 * (uint64_t)dp.hx * (dp.py / 2 + 1) : 6 * (uint64_t)points;
     // components with an odd number of odd axes transform to imaginary
     // values: xz (odd in x) and yz (odd in y) of the shifted kernels, whose
