@@ -57,6 +57,7 @@ struct FastDiv {
 // Records a HIP failure into `err` and returns false.
 inline bool hip_ok(hipError_t e, const char *what, std::string &err) {
     if (e == hipSuccess) return true;
+    (void)hipGetLastError();  // reported here, not by a later launch's check
     err = std::string(what) + ": " + hipGetErrorString(e);
     return false;
 }

@@ -11,6 +11,7 @@ bool ctx_alloc(Context &c, void **ptr, size_t bytes, const char *what) {
     void *p = nullptr;
     hipError_t e = hipMalloc(&p, bytes ? bytes : 1);
     if (e != hipSuccess) {
+        (void)hipGetLastError();  // see hip_ok
         c.last_error = std::string("hipMalloc(") + what + ", " + std::to_string(bytes) + " bytes): " +
                        hipGetErrorString(e);
         return false;

@@ -968,7 +968,6 @@ bool setup_t(Context &c, const fullmag_fdm_plan_desc &plan) {
         dp.xrows = dp.ny + (dp.ny & 1);
         const std::string err = c.last_error;
         if (!ctx_alloc(c, &dp.xspec, 3ull * dp.nz * dp.hx * dp.xrows * sizeof(cplx<Real>), "demag spectrum")) {
-            (void)hipGetLastError();
             dp.xspec = nullptr;
             c.last_error = err;
         }

@@ -981,9 +981,16 @@ static bool xfer_scratch(Context &c) {
     const uint64_t cells = std::min<uint64_t>(c.n, kXferCells);
     const std::string keep = c.last_error;
     if (ctx_alloc(c, &c.d_xfer, cells * 3 * sizeof(double), "transfer scratch")) return true;
-    (void)hipGetLastError();  // the caller converts on the host instead
-    c.last_error = keep;
+    c.last_error = keep;  // the caller converts on the host instead
     return false;
+}
+
+// Launches `k` and takes this launch's own status: an error that an earlier call
+// of the thread left (a failed allocation) is not the transfer's.
+template <typename... P>
+static bool launch_xfer(Context &c, void (*k)(P...), dim3 g, dim3 b, const char *what, P... p) {
+    void *args[] = {&p...};
+    return hip_ok(hipLaunchKernel(reinterpret_cast<const void *>(k), g, b, args, 0, c.stream), what, c.last_error);
 }
 
 int state_from_host(Context &c, const void *host, bool host_f64) {
@@ -1002,18 +1009,15 @@ int state_from_host(Context &c, const void *host, bool host_f64) {
         auto launch = [&](auto in, auto state) {
             using In = decltype(in);
             using State = decltype(state);
-            hipLaunchKernelGGL((aos_to_soa_kernel<In, State>), g, b, 0, c.stream, static_cast<const In *>(c.d_xfer),
-                               c.d_mask, (int64_t)first, (int64_t)count, n, static_cast<State *>(c.m));
+            return launch_xfer(c, aos_to_soa_kernel<In, State>, g, b, "magnetization upload",
+                               static_cast<const In *>(c.d_xfer), (const uint8_t *)c.d_mask, (int64_t)first,
+                               (int64_t)count, n, static_cast<State *>(c.m));
         };
-        if (host_f64 && c.state_bytes() == 8) launch(double(), double());
-        else if (host_f64) launch(double(), float());
-        else if (c.state_bytes() == 8) launch(float(), double());
-        else launch(float(), float());
+        const bool ok = host_f64 ? (c.state_bytes() == 8 ? launch(double(), double()) : launch(double(), float()))
+                                 : (c.state_bytes() == 8 ? launch(float(), double()) : launch(float(), float()));
+        if (!ok) return -1;
     }
-    return hip_ok(hipStreamSynchronize(c.stream), "hipMemcpy(m)", c.last_error) &&
-                   hip_ok(hipGetLastError(), "magnetization upload", c.last_error)
-               ? 1
-               : -1;
+    return hip_ok(hipStreamSynchronize(c.stream), "hipMemcpy(m)", c.last_error) ? 1 : -1;
 }
 
 int field_to_host(Context &c, const void *field, bool field_f64, void *out, bool out_f64) {
@@ -1028,22 +1032,18 @@ int field_to_host(Context &c, const void *field, bool field_f64, void *out, bool
         auto launch = [&](auto in, auto o) {
             using In = decltype(in);
             using Out = decltype(o);
-            hipLaunchKernelGGL((soa_to_aos_kernel<In, Out>), g, b, 0, c.stream, static_cast<const In *>(field),
+            return launch_xfer(c, soa_to_aos_kernel<In, Out>, g, b, "field copy", static_cast<const In *>(field),
                                (int64_t)first, (int64_t)count, n, static_cast<Out *>(c.d_xfer));
         };
-        if (field_f64 && out_f64) launch(double(), double());
-        else if (field_f64) launch(double(), float());
-        else if (out_f64) launch(float(), double());
-        else launch(float(), float());
+        const bool ok = field_f64 ? (out_f64 ? launch(double(), double()) : launch(double(), float()))
+                                  : (out_f64 ? launch(float(), double()) : launch(float(), float()));
+        if (!ok) return -1;
         if (!hip_ok(hipMemcpyAsync(static_cast<char *>(out) + 3 * first * ob, c.d_xfer, 3 * count * ob,
                                    hipMemcpyDeviceToHost, c.stream),
                     "hipMemcpy(field)", c.last_error))
             return -1;
     }
-    return hip_ok(hipStreamSynchronize(c.stream), "hipMemcpy(field)", c.last_error) &&
-                   hip_ok(hipGetLastError(), "field copy", c.last_error)
-               ? 1
-               : -1;
+    return hip_ok(hipStreamSynchronize(c.stream), "hipMemcpy(field)", c.last_error) ? 1 : -1;
 }
 
 bool preview_field(Context &c, const void *field, bool field_f64, uint32_t pnx, uint32_t pny, uint32_t pnz,
