@@ -1281,9 +1281,8 @@ bool stack_setup_t(Stack &s, std::string &err) {
     // passes, Heun steps of 2 to 5 layers of 64 x 64 to 512 x 512: 1.03 to
     // 1.6 times as fast wherever it fits, FP32 and FP64.
     s.kpw = std::max(1, 256 / (3 * L * dp.ly.threads));
-    s.fused = !dp.three_d && dp.ly.fixed && L <= kStackFused && !dp.tune.y_split &&
-              3 * L * dp.ly.threads <= 1024 &&
-              (size_t)3 * L * s.kpw * line_slots(dp.ly) * ce <= dp.lds_limit;
+    s.fused = !dp.three_d && dp.ly.fixed && !dp.tune.y_split &&
+              ystack_fits<Real>(dp.py, L, s.kpw, std::min(dp.lds_limit, kLdsMax));
     // Frequencies k + 1/2 along x (skew_rule) where that saves a round: 3 films
     // of 512x512, 513 workgroups, mixed 138.3 and 123.7 us per step, FP64 214.8
     // and 203.1; without one saved, 100x300 four films FP64 79.5 and 83.0.

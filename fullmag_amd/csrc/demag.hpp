@@ -286,6 +286,13 @@ struct StackField {
 // Thin stack of L <= kStackFused layers: per kx, the layers' 3 L ky lines are
 // transformed, coupled by the pair kernels and transformed back in place.
 constexpr int kStackFused = 5;
+constexpr size_t kLdsMax = 163840;  // LDS of a CU, the most that a workgroup may take
+// Whether `kpw` columns of L layers' scheduled lines fit a workgroup of `lds` bytes.
+template <typename Real>
+constexpr bool ystack_fits(int n, int L, int kpw = 1, size_t lds = kLdsMax) {
+    return fx_has(n) && L <= kStackFused && 3 * L * fx_lanes(n) <= 1024 && lds <= kLdsMax &&
+           (size_t)3 * L * kpw * fx_size(n) * sizeof(cplx<Real>) <= lds;
+}
 template <typename Real>
 struct YStackArgs {
     cplx<Real> *data;       // [layer][c][kx][ky]
@@ -370,14 +377,24 @@ struct Timed {
     }
 };
 
+constexpr int scheduled_lengths() {
+    int k = 0;
+    for (int n = 1; n <= 4096; ++n) k += fx_has(n) ? 1 : 0;
+    return k;
+}
+
 // Calls f(std::integral_constant<int, N>) with N the line length when `lp`
 // has a compile-time schedule, else with N = 0 (runtime plan).
 template <class F>
 void with_line(const LinePlan &lp, F &&f) {
+    static_assert(scheduled_lengths() == 26, "every length of fx_has is listed here");
     if (lp.fixed) {
         switch (lp.n) {
-#define FM_LINE(N) \
-    case N: f(std::integral_constant<int, N>{}); return;
+#define FM_LINE(N)                             \
+    case N:                                    \
+        static_assert(fx_has(N), "scheduled"); \
+        f(std::integral_constant<int, N>{});   \
+        return;
             FM_LINE(20) FM_LINE(24) FM_LINE(28) FM_LINE(32) FM_LINE(40) FM_LINE(48) FM_LINE(56) FM_LINE(64)
             FM_LINE(80) FM_LINE(96) FM_LINE(112) FM_LINE(128) FM_LINE(160) FM_LINE(192) FM_LINE(224) FM_LINE(256)
             FM_LINE(320) FM_LINE(384) FM_LINE(448) FM_LINE(512) FM_LINE(640) FM_LINE(768) FM_LINE(896)

@@ -441,8 +441,7 @@ void launch_ystack(Context &c, const LinePlan &lp, int layers, const YStackArgs<
         constexpr int N = decltype(NC)::value;
         auto launch = [&](auto lc) {
             constexpr int L = decltype(lc)::value;
-            // what the plan's rule can choose (160 KiB of LDS)
-            if constexpr (N > 0 && 3 * L * fx_lanes(N) <= 1024 && 3 * L * fx_size(N) * sizeof(cplx<Real>) <= 163840)
+            if constexpr (ystack_fits<Real>(N, L))  // the plan's rule
                 hipLaunchKernelGGL((ystack_kernel<Real, N, L>), grid, block, lds, c.stream, ya);
         };
         switch (layers) {
