@@ -58,3 +58,22 @@ def test_slab_kernel_by_its_knob(fa, monkeypatch, slab, precision):
     gpu.refresh_observables()
     assert np.abs(gpu.copy_h_demag() - h).max() <= BAR[precision] * np.abs(h).max()
     gpu.close()
+
+
+# the knobs that choose between the demag routes, against the oracle (the bars
+# of test_gpu_parity.py: FP64 1e-11 of the largest value, FP32 2e-6): slabs and
+# their separate passes, padded and at 2n, ky classes and theirs, long z lines
+@pytest.mark.parametrize("precision", ["double", "mixed"])
+@pytest.mark.parametrize("cells", [(32, 16, 4), (64, 32, 8), (16, 16, 6), (64, 48, 8), (13, 37, 5), (5, 160, 6),
+                                   (6, 300, 3), (9, 20, 11)])
+@pytest.mark.parametrize("tune", ["slab=0", "skew=0", "slab=0,pad=0", "skew=0,pad=0", "pad=0"])
+def test_routes_match_oracle(fa, oracle_mod, monkeypatch, cells, precision, tune):
+    monkeypatch.setenv("FULLMAG_FDM_TUNE", tune)
+    nx, ny, nz = cells
+    gpu = backend(fa, cells, precision)
+    n = int(np.prod(cells))
+    cfg = oracle_mod.OracleConfig(nx=nx, ny=ny, nz=nz, dx=4e-9, dy=3e-9, dz=2e-9, ms=8e5, a=1e-11, alpha=0.1)
+    want = oracle_mod.OracleProblem(cfg, fa.generate_random_unit_vectors(17 + n, n)).observe()["h_demag"]
+    bar = 1e-11 if precision == "double" else 2e-6
+    np.testing.assert_allclose(gpu.copy_h_demag(), want, rtol=0, atol=bar * np.abs(want).max())
+    gpu.close()
