@@ -252,7 +252,7 @@ __global__ void __launch_bounds__(256) boundary_corr_kernel(BoundaryCorrArgs<Rea
 // 64x64x4 43.7 and 37.8, 128x128x4 51.8 and 41.7, 256x256x4 83.8 and 65.3,
 // 500x250x8 189 and 167, 256x256x8 116 and 108; FP64 128x128x4 67.8 and 49.5,
 // 128x128x8 90.3 and 67.2, 500x250x4 177 and 146.  With 5 to 8 layers and
-// lines of 32 lanes a workgroup has up to 24 wavefronts of at most 85 FP64
+// lines of 32 lanes a workgroup has up to 12 wavefronts of at most 85 FP64
 // values: FP64 spills (250x150x6 108 and 151).  FP32 there takes one round of
 // one workgroup per CU for up to 256 slabs, which the skewed x frequencies give
 // (classes and slab: 250x150x6 93.5 and 79.4, 256x256x6 102.2 and 86.8,
@@ -276,7 +276,10 @@ template <typename Real>
 bool class_rule(const DemagPlan &dp);
 // Whether workgroups of `lds` bytes, `per_column` for each column or one for
 // `per_group` of them, take fewer rounds over the chip for px / 2 columns than
-// for px / 2 + 1.
+// for px / 2 + 1, as many to a CU as its LDS holds.  A kernel's registers can
+// hold it to fewer (class_kernel: three wavefronts per SIMD, 512 workgroups of
+// 8 layers where the LDS counts 768 or 1024), so for ky classes this is where
+// the columns divide into whole rounds by the LDS, not the rounds that run.
 bool saves_round(const DemagPlan &dp, size_t lds, int per_group = 1, int per_column = 1) {
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
@@ -292,9 +295,11 @@ bool saves_round(const DemagPlan &dp, size_t lds, int per_group = 1, int per_col
 // slab kernel's workgroups, one to three per CU, come to whole rounds where
 // px does.  us per mixed Heun step without and with: 256x256x8 117.6 and 94.2
 // (257 slabs of 104 KB are two rounds), 500x250x8 175.3 and 152.5, 256x256x4
-// 73.4 and 71.1, 128x128x8 55.1 and 53.6; ky classes where that saves a round,
-// 256x300x8 139.2 and 132.0.  Elsewhere the factors in the x
-// passes cost more than a column: 512x512x8 340 and 345, 512x512x1 73.8 and
+// 73.4 and 71.1, 128x128x8 55.1 and 53.6; ky classes where saves_round
+// counts one less, 256x300x8 138.9 and 132.2, 384x500x7 217.6 and 210.5.  It does
+// not for others that gain (256x512x8 176.1 and 170.7, 64x400x8 90.0 and 80.6) and
+// does for one that does not (384x512x8 238 and 238).  Elsewhere the factors in
+// the x passes cost more than a column: 512x512x8 342 and 346, 512x512x1 73.8 and
 // 75.5, 256x256x64 756 and 768.  In FP64 they cost 2 to 3 us per pass
 // (128x128x4 52 and 57), which only a round saved gives back.
 template <typename Real>

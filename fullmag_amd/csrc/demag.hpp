@@ -25,8 +25,9 @@ __device__ __forceinline__ const T *no_array() {
     else return &kNoArrayF64;
 }
 constexpr int kMaxBlock = 512;  // lanes per workgroup for FFT kernels
-// largest padded z length done in registers (a lane pair per column holds
-// 3 x pz complex values)
+// largest padded z length done in registers (a lane holds a column's 3 pz / 2
+// inputs and one half of its padded spectrum; FP64 spreads the components over
+// three wavefronts)
 template <typename Real>
 constexpr int z_reg_max() {
     return 16;
@@ -118,7 +119,7 @@ __device__ __forceinline__ void apply_tensor(const Real t[6], cplx<Real> &mx, cp
 // Spectrum addressing: spec[c][z][kx][ky], `planes` z-planes, ky pitch.
 // ---------------------------------------------------------------------------
 struct SpecGeom {
-    int hx;       // half-spectrum width px / 2 + 1
+    int hx;       // half-spectrum width px / 2 + 1, or px / 2 at the frequencies k + 1/2
     int planes;   // z planes stored
     int pitch;    // ky line length stored
     __device__ __host__ int64_t at(int c, int z, int kx, int ky) const {
