@@ -79,16 +79,13 @@ def alg_bytes(nx, ny, nz, q, r):
 
 
 def step_bytes(nx, ny, nz, q, r):
-    """Algorithmic bytes of one Heun step: two demag evaluations plus the
-    torque/predictor and corrector passes, stats fused."""
-    n = nx * ny * nz
-    c = 2 * r
-    h = nx + 1
-    a1, a2 = h * ny * nz, h * 2 * ny * nz
-    kern = 6 * (nx + 1) * (ny + 1) * (nz + 1)
-    d = (3 * n * q + 3 * a1 * c) + (3 * a1 * c + 3 * a2 * c) + (3 * a2 * c + kern * r + 3 * a2 * c) \
-        + (3 * a2 * c + 3 * a1 * c) + (3 * a1 * c + 3 * n * r)
-    return 2 * d + 3 * n * (2 * q + 2 * r) + 3 * n * (3 * q + 2 * r)
+    """Algorithmic bytes of one Heun step: two demag evaluations by the passes
+    that the mixed film runs (y transform and z convolution per ky class, one
+    write and one read of the padded spectrum), and the corrector and
+    stats/predictor passes."""
+    b = alg_bytes(nx, ny, nz, q, r)
+    return 2 * (b["demag_x_r2c"] + b["demag_yz_class"] + b["demag_y_inv"] + b["demag_x_c2r"]) \
+        + b["llg_stage"] + b["llg_stats"]
 
 
 def smooth_m0(nx, ny, nz):
