@@ -218,8 +218,10 @@ __global__ void __launch_bounds__((HIGH ? 24 : 12) * fx_lanes(N)) slab_multi(con
 // together, and the inverse y lines read it from there.  Against the y lines
 // and zreg_kernel the padded spectrum is written once less and read once less
 // (512x512x8 FP32: 207 MB read and written instead of 409), while the x
-// spectrum is read by four workgroups, next to each other on one XCD.  Bound
-// by VALU work at two workgroups per CU: three wavefronts per SIMD (168
+// spectrum is read by four workgroups, next to each other on one XCD.  Bound by
+// latency at two workgroups per CU: 74 us there with VALU instructions issued
+// in 46 % of the SIMDs' cycles, 1.7 wavefronts on a SIMD on average and 221 MB
+// at 3.0 TB/s.  Three wavefronts per SIMD (168
 // registers) take 76 us there, two 93 us, a component per lane (slab_rows)
 // 106 us, a workgroup of one wavefront per 64 columns that walks over its
 // lines 111 us; the two kernels it replaces 80 us.  Per step and the rule:

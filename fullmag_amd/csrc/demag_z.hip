@@ -313,8 +313,9 @@ __global__ void __launch_bounds__(kMaxBlock) zlds_kernel(ZLdsArgs<Real> a) {
 // columns.  CONV: each tensor entry oz is loaded (beside the columns, before
 // the transform) once per column and applied at kz = oz and pz - oz between
 // two barriers; the inverse transform's last pass stores straight to memory.
-// Bound by VALU work (about half of it butterflies) and by memory latency at
-// nine wavefronts per CU.  256x256x64 mixed (257x512 columns of 128, 507 MB):
+// Bound by VALU work (about half of it butterflies; issued in 62 % of the SIMDs'
+// cycles of the launch below) and by memory latency at nine wavefronts per CU
+// (1.9 per SIMD on average).  256x256x64 mixed (257x512 columns of 128, 507 MB):
 // 213 us with the staged lines of zlds_kernel, 131 us here, 147 us with one
 // column per lane (twice the wavefronts, but each pays its own twiddles and
 // 64-byte runs).  100^3 FP64: 214 -> 109 us.
