@@ -316,8 +316,8 @@ void fullmag_fdm_ext_batch_destroy(fullmag_fdm_batch *b) {
 // cell kernels, timing (demag + stats) at the current state; keeps the
 // fastest schedule and writes it as "key=value,..." into `chosen`.  The
 // plan-shaping knobs (radices, rows per x workgroup, y lines per workgroup,
-// long-z tile) are tried by re-planning the transforms in place; candidates
-// whose plan does not fit are skipped.
+// compile-time schedules or runtime plans, long-z tile) are tried by re-planning
+// the transforms in place; candidates whose plan does not fit are skipped.
 int fullmag_fdm_ext_autotune(fullmag_fdm_backend *handle, int reps, char *chosen, uint64_t chosen_len) {
     fm::Context *cp = handle ? fm::backend_context(handle) : nullptr;
     if (!cp || !cp->ready) return FULLMAG_FDM_ERR_INVALID;
