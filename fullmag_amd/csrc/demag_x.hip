@@ -69,7 +69,9 @@ __device__ __forceinline__ void xfwd_body_rt(const XArgs<Real> &a, const Src &sr
 // 66.2 us per step with the table, 67.7 with the roots ahead).  FP32 at the
 // frequencies k + 1/2 forms EXACT powers: a state's mean, which integer
 // frequencies keep at k = 0 away from every twiddle, spreads over all of them
-// there.  At integer frequencies they would cost more than they give (all lines
+// there (rms of H_demag, smooth state, 128x128x4: 3.4 and 3.2e-7; 500x250x8
+// random 2.4 and 2.2e-7 at 152.5 and 155.7 us per step, three 512x512 films 156.3
+// and 157.9).  At integer frequencies they would cost more than they give (all lines
 // so: 512x512x1 mixed 74.3 -> 76.2 us per step, 512x512x8 341 -> 349).
 template <typename Real, int N, bool SKEW>
 __device__ __forceinline__ auto x_roots(int t, const cplx<Real> *tw) {
@@ -100,25 +102,27 @@ __device__ __forceinline__ void xfwd_body(const XArgs<Real> &a, const Src &src, 
         // (n_in <= N / 2) and are not loaded
         const bool oka = ya < a.rows, okb = ya + 1 < a.rows;
         const int yA = oka ? ya : 0, yB = okb ? ya + 1 : 0;
-        double va[E / 2], vb[E / 2];
+        constexpr int H = SKEW ? E / 2 : 1;
+        double va[H], vb[H];
 #pragma unroll
         for (int e = 0; e < E / 2; ++e) {
             const int x = t + e * T;
             const bool okx = x < a.n_in;
             const int xs = okx ? x : 0;
             const double qa = src.load(c, z, yA, xs), qb = src.load(c, z, yB, xs);
-            va[e] = (okx && oka) ? qa : 0.0;
-            vb[e] = (okx && okb) ? qb : 0.0;
+            if constexpr (SKEW) {
+                va[e] = (okx && oka) ? qa : 0.0;
+                vb[e] = (okx && okb) ? qb : 0.0;
+            } else {
+                v[e] = {(okx && oka) ? Real(qa) : Real(0), (okx && okb) ? Real(qb) : Real(0)};
+            }
         }
         if constexpr (SKEW) {
-            cplx<double> w[E / 2];
+            cplx<double> w[H];
 #pragma unroll
-            for (int e = 0; e < E / 2; ++e) w[e] = a.sw64[t + e * T];
+            for (int e = 0; e < H; ++e) w[e] = a.sw64[t + e * T];
 #pragma unroll
-            for (int e = 0; e < E / 2; ++e) v[e] = skewed<Real>(va[e], vb[e], w[e]);
-        } else {
-#pragma unroll
-            for (int e = 0; e < E / 2; ++e) v[e] = {Real(va[e]), Real(vb[e])};
+            for (int e = 0; e < H; ++e) v[e] = skewed<Real>(va[e], vb[e], w[e]);
         }
 #pragma unroll
         for (int e = E / 2; e < E; ++e) v[e] = {Real(0), Real(0)};
