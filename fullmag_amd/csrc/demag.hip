@@ -1289,7 +1289,7 @@ bool stack_setup_t(Stack &s, std::string &err) {
     s.fused = !dp.three_d && dp.ly.fixed && !dp.tune.y_split &&
               ystack_fits<Real>(dp.py, L, s.kpw, std::min(dp.lds_limit, kLdsMax));
     // Frequencies k + 1/2 along x (skew_rule) where that saves a round: 3 films
-    // of 512x512, 513 workgroups, mixed 138.3 and 123.7 us per step, FP64 214.8
+    // of 512x512, 513 workgroups, mixed 138.3 and 125.4 us per step, FP64 214.8
     // and 203.1; without one saved, 100x300 four films FP64 79.5 and 83.0.
     dp.skew = tune.skew != 0 && s.fused &&
               saves_round(dp, (size_t)3 * L * s.kpw * line_slots(dp.ly) * ce, s.kpw);
